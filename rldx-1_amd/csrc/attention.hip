@@ -119,6 +119,7 @@ struct AttnArgs {
   int64_t kb_sb;
   int hq, hkv, group, sq, sk;
   int num_q_blocks;
+  int gsz, nh;  // attn_shared_kernel, causal: XCDs per group of nh heads
   float scale_log2;  // softmax scale * log2(e), > 0
   // fused Q RMSNorm + rotate-half RoPE (Qwen3-VL), used when kQNorm
   const uint16_t* q_norm_w;  // [D] bf16
@@ -134,6 +135,7 @@ struct AttnArgs {
   int num_seqs;
   int total_rows;
   int d_store;  // output columns written per head (<= D)
+  int o_vec16;  // row-major O: 16-byte aligned rows and heads (else 8-byte)
   // the first n_work workgroups compute attention; those after them read the
   // lines of `warm` (rldx_attention_packed_fwd_warm_bf16)
   int n_work;
@@ -150,39 +152,38 @@ struct AttnArgs {
 // scan of cu_seqlens is needed to place a sequence, and a slot finds its
 // sequence with one load per lane (up to 63 sequences) or a binary search.
 struct SeqSlot {
-  int start, len, base;
+  int start, len, base, seq;
 };
 
-__host__ __device__ constexpr int64_t seq_slot_count(int64_t rows, int64_t num_seqs) {
-  return (rows + 31 * num_seqs) / 32;
+__host__ __device__ constexpr int64_t seq_slot_count(int64_t rows, int64_t num_seqs, int64_t r = 32) {
+  return (rows + (r - 1) * num_seqs) / r;
 }
 
 __device__ __forceinline__ int clamp_row(int32_t c, int rows) { return c < 0 ? 0 : (c > rows ? rows : c); }
 
-// Called with the whole wave active.
+// Slots of R rows (the same placement with R in place of 32).  Called with the
+// whole wave active.
+template <int R = 32>
 __device__ __forceinline__ SeqSlot find_seq_slot(const int32_t* cu, int num_seqs, int rows, int slot) {
+  auto base_of = [](int c, int s) { return (static_cast<int64_t>(c) + (R - 1) * static_cast<int64_t>(s)) / R; };
   if (num_seqs <= 63) {
     // one load per lane: lane s holds c_s (lanes past num_seqs repeat c_num_seqs);
     // the sequence is the last s < num_seqs with base_s <= slot
     const int lane = static_cast<int>(threadIdx.x & 63);
     const int c = clamp_row(cu[min(lane, num_seqs)], rows);
-    const int64_t base = (static_cast<int64_t>(c) + 31 * static_cast<int64_t>(lane)) / 32;
-    const uint64_t cand = __ballot(lane < num_seqs && base <= slot);
+    const uint64_t cand = __ballot(lane < num_seqs && base_of(c, lane) <= slot);
     const int s = cand ? 63 - __builtin_clzll(cand) : 0;
     const int c0 = __builtin_amdgcn_readlane(c, s), c1 = __builtin_amdgcn_readlane(c, s + 1);
-    return SeqSlot{c0, c1 > c0 ? c1 - c0 : 0,
-                   static_cast<int>((static_cast<int64_t>(c0) + 31 * static_cast<int64_t>(s)) / 32)};
+    return SeqSlot{c0, c1 > c0 ? c1 - c0 : 0, static_cast<int>(base_of(c0, s)), s};
   }
   int lo = 0, hi = num_seqs - 1;  // last s with base_s <= slot (0 when there is none)
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    const int64_t base = (static_cast<int64_t>(clamp_row(cu[mid], rows)) + 31 * static_cast<int64_t>(mid)) / 32;
-    if (base <= slot) lo = mid;
+    if (base_of(clamp_row(cu[mid], rows), mid) <= slot) lo = mid;
     else hi = mid - 1;
   }
   const int c0 = clamp_row(cu[lo], rows), c1 = clamp_row(cu[lo + 1], rows);
-  return SeqSlot{c0, c1 > c0 ? c1 - c0 : 0,
-                 static_cast<int>((static_cast<int64_t>(c0) + 31 * static_cast<int64_t>(lo)) / 32)};
+  return SeqSlot{c0, c1 > c0 ? c1 - c0 : 0, static_cast<int>(base_of(c0, lo)), lo};
 }
 
 __device__ __forceinline__ float bf(uint16_t b) { return bf16_bits_to_f32(b); }
@@ -197,22 +198,13 @@ __device__ __forceinline__ float bf(uint16_t b) { return bf16_bits_to_f32(b); }
 // Roundings to bf16 use v_cvt_pk_bf16_f32 (round to nearest even).  The chunk
 // index is a template parameter: a run-time index into the register array
 // would compile to select chains over every chunk.
-template <int D, int K0>
-__device__ __forceinline__ void qnorm_rope_pair(const bf16x8 (&qreg)[D / 16], const AttnArgs& a, int pos, bool valid,
-                                                u32x4* qsh) {
+// 1 / rms of the lane pair's query row held in qreg.
+template <int D>
+__device__ __forceinline__ float qnorm_rinv(const bf16x8 (&qreg)[D / 16], float eps) {
 #pragma clang fp contract(off)
-  constexpr int KS = D / 16, K1 = K0 + KS / 2;
-  const int lane = threadIdx.x & 63;
-  const int g = lane >> 5;
-  const uint16_t* cr = a.cos + static_cast<int64_t>(valid ? pos : 0) * a.cs_ss + g * 8;
-  const uint16_t* sr = a.sin + static_cast<int64_t>(valid ? pos : 0) * a.cs_ss + g * 8;
-  const u32x4 w0 = *reinterpret_cast<const u32x4*>(a.q_norm_w + K0 * 16 + g * 8);
-  const u32x4 w1 = *reinterpret_cast<const u32x4*>(a.q_norm_w + K1 * 16 + g * 8);
-  const u32x4 c0 = *reinterpret_cast<const u32x4*>(cr + K0 * 16), c1 = *reinterpret_cast<const u32x4*>(cr + K1 * 16);
-  const u32x4 s0 = *reinterpret_cast<const u32x4*>(sr + K0 * 16), s1 = *reinterpret_cast<const u32x4*>(sr + K1 * 16);
   float ss = 0.f;
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
+  for (int ks = 0; ks < D / 16; ++ks) {
     const u32x4 raw = __builtin_bit_cast(u32x4, qreg[ks]);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -222,28 +214,78 @@ __device__ __forceinline__ void qnorm_rope_pair(const bf16x8 (&qreg)[D / 16], co
     }
   }
   ss = pair_sum(ss);
-  const float rinv = 1.0f / __builtin_sqrtf(ss * (1.0f / D) + a.eps);
-  const u32x4 x0 = __builtin_bit_cast(u32x4, qreg[K0]), x1 = __builtin_bit_cast(u32x4, qreg[K1]);
-  u32x4 o0, o1;
+  return 1.0f / __builtin_sqrtf(ss * (1.0f / D) + eps);
+}
+
+// The table and weight chunks of a rotate-half pair, then its arithmetic.
+struct QnormIn {
+  u32x4 w0, w1, c0, c1, s0, s1;
+};
+
+template <int D, int K0>
+__device__ __forceinline__ QnormIn qnorm_load(const AttnArgs& a, int pos, bool valid) {
+  constexpr int K1 = K0 + D / 32;
+  const int g = static_cast<int>(threadIdx.x & 63) >> 5;
+  const uint16_t* cr = a.cos + static_cast<int64_t>(valid ? pos : 0) * a.cs_ss + g * 8;
+  const uint16_t* sr = a.sin + static_cast<int64_t>(valid ? pos : 0) * a.cs_ss + g * 8;
+  QnormIn in;
+  in.w0 = *reinterpret_cast<const u32x4*>(a.q_norm_w + K0 * 16 + g * 8);
+  in.w1 = *reinterpret_cast<const u32x4*>(a.q_norm_w + K1 * 16 + g * 8);
+  in.c0 = *reinterpret_cast<const u32x4*>(cr + K0 * 16);
+  in.c1 = *reinterpret_cast<const u32x4*>(cr + K1 * 16);
+  in.s0 = *reinterpret_cast<const u32x4*>(sr + K0 * 16);
+  in.s1 = *reinterpret_cast<const u32x4*>(sr + K1 * 16);
+  return in;
+}
+
+__device__ __forceinline__ void qnorm_apply(const QnormIn& in, u32x4 x0, u32x4 x1, float rinv, bool sin_signed,
+                                            u32x4& o0, u32x4& o1) {
+#pragma clang fp contract(off)
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     // y = bf16(w * bf16(x * rinv)) for the two elements of word j of both chunks
     const uint32_t n0 = pack_bf16x2(bf16x2_lo(x0[j]) * rinv, bf16x2_hi(x0[j]) * rinv);
     const uint32_t n1 = pack_bf16x2(bf16x2_lo(x1[j]) * rinv, bf16x2_hi(x1[j]) * rinv);
-    const uint32_t y0 = pack_bf16x2(bf16x2_lo(w0[j]) * bf16x2_lo(n0), bf16x2_hi(w0[j]) * bf16x2_hi(n0));
-    const uint32_t y1 = pack_bf16x2(bf16x2_lo(w1[j]) * bf16x2_lo(n1), bf16x2_hi(w1[j]) * bf16x2_hi(n1));
+    const uint32_t y0 = pack_bf16x2(bf16x2_lo(in.w0[j]) * bf16x2_lo(n0), bf16x2_hi(in.w0[j]) * bf16x2_hi(n0));
+    const uint32_t y1 = pack_bf16x2(bf16x2_lo(in.w1[j]) * bf16x2_lo(n1), bf16x2_hi(in.w1[j]) * bf16x2_hi(n1));
     const float y0l = bf16x2_lo(y0), y0h = bf16x2_hi(y0), y1l = bf16x2_lo(y1), y1h = bf16x2_hi(y1);
     // chunk K0 (first half): partner -y1 (+y1 with a pre-signed sin); chunk K1: partner +y0
-    const float r0l = a.sin_signed ? y1l : -y1l, r0h = a.sin_signed ? y1h : -y1h;
-    const uint32_t t0 = pack_bf16x2(y0l * bf16x2_lo(c0[j]), y0h * bf16x2_hi(c0[j]));
-    const uint32_t u0 = pack_bf16x2(r0l * bf16x2_lo(s0[j]), r0h * bf16x2_hi(s0[j]));
-    const uint32_t t1 = pack_bf16x2(y1l * bf16x2_lo(c1[j]), y1h * bf16x2_hi(c1[j]));
-    const uint32_t u1 = pack_bf16x2(y0l * bf16x2_lo(s1[j]), y0h * bf16x2_hi(s1[j]));
+    const float r0l = sin_signed ? y1l : -y1l, r0h = sin_signed ? y1h : -y1h;
+    const uint32_t t0 = pack_bf16x2(y0l * bf16x2_lo(in.c0[j]), y0h * bf16x2_hi(in.c0[j]));
+    const uint32_t u0 = pack_bf16x2(r0l * bf16x2_lo(in.s0[j]), r0h * bf16x2_hi(in.s0[j]));
+    const uint32_t t1 = pack_bf16x2(y1l * bf16x2_lo(in.c1[j]), y1h * bf16x2_hi(in.c1[j]));
+    const uint32_t u1 = pack_bf16x2(y0l * bf16x2_lo(in.s1[j]), y0h * bf16x2_hi(in.s1[j]));
     o0[j] = pack_bf16x2(bf16x2_lo(t0) + bf16x2_lo(u0), bf16x2_hi(t0) + bf16x2_hi(u0));
     o1[j] = pack_bf16x2(bf16x2_lo(t1) + bf16x2_lo(u1), bf16x2_hi(t1) + bf16x2_hi(u1));
   }
+}
+
+template <int D, int K0>
+__device__ __forceinline__ void qnorm_rope_pair(const bf16x8 (&qreg)[D / 16], const AttnArgs& a, int pos, bool valid,
+                                                u32x4* qsh) {
+  constexpr int KS = D / 16, K1 = K0 + KS / 2;
+  const int lane = threadIdx.x & 63;
+  const QnormIn in = qnorm_load<D, K0>(a, pos, valid);
+  const float rinv = qnorm_rinv<D>(qreg, a.eps);
+  u32x4 o0, o1;
+  qnorm_apply(in, __builtin_bit_cast(u32x4, qreg[K0]), __builtin_bit_cast(u32x4, qreg[K1]), rinv, a.sin_signed != 0,
+              o0, o1);
   qsh[K0 * 64 + lane] = o0;
   qsh[K1 * 64 + lane] = o1;
+}
+
+// The same of a wave's own 32 query rows, all chunk pairs in its registers.
+template <int D, int K0 = 0>
+__device__ __forceinline__ void qnorm_rope_own(bf16x8 (&qreg)[D / 16], const AttnArgs& a, int pos, bool valid,
+                                               float rinv) {
+  constexpr int KS = D / 16, K1 = K0 + KS / 2;
+  const QnormIn in = qnorm_load<D, K0>(a, pos, valid);
+  u32x4 o0, o1;
+  qnorm_apply(in, __builtin_bit_cast(u32x4, qreg[K0]), __builtin_bit_cast(u32x4, qreg[K1]), rinv, a.sin_signed != 0,
+              o0, o1);
+  qreg[K0] = __builtin_bit_cast(bf16x8, o0);
+  qreg[K1] = __builtin_bit_cast(bf16x8, o1);
+  if constexpr (K0 + 1 < KS / 2) qnorm_rope_own<D, K0 + 1>(qreg, a, pos, valid, rinv);
 }
 
 template <int D>
@@ -283,10 +325,18 @@ __device__ __forceinline__ int div_small(int a, int b) {
 // LDS directly (buffer_load ... lds).
 template <int N>
 __device__ __forceinline__ void vm_wait_barrier() {
-  static_assert(N == 4 || N == 6 || N == 8, "vmcnt immediate: the V loads of the first tile");
+  static_assert((N >= 0 && N <= 9) || N == 12, "vmcnt immediate");
+  if constexpr (N == 12) asm volatile("s_waitcnt vmcnt(12) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (N == 9) asm volatile("s_waitcnt vmcnt(9) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   if constexpr (N == 8) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (N == 7) asm volatile("s_waitcnt vmcnt(7) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   if constexpr (N == 6) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (N == 5) asm volatile("s_waitcnt vmcnt(5) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   if constexpr (N == 4) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (N == 3) asm volatile("s_waitcnt vmcnt(3) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (N == 2) asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (N == 1) asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (N == 0) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
 template <int D, int NSUB, bool kCausal, bool kBias, bool kQNorm, bool kVarlen = false>
@@ -639,6 +689,381 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_kernel(AttnArgs a) {
           else
             *reinterpret_cast<uint2*>(orow + d) = wv;
         }
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The same attention for launches that fill the chip, with the K/V tiles shared
+// through LDS: 4 waves = NQ query blocks of 32 x NG key groups.  Per step every
+// key group takes one 32-key tile (tile i NG + group), read by its NQ waves from
+// LDS: a tile crosses from L2 once per 32 NQ queries (buffer_load ... lds, one
+// barrier per step) instead of once per 32.  attn_fwd_kernel reads 38 B/clk per
+// CU at 32/8 heads x 4096 causal, close to the ~48 B/clk a CU gets from L2.
+//   * NG = 1 (128 queries, no merge): a wave runs S, softmax and P V of one tile
+//     in sequence within 168 VGPRs, and three workgroups per CU overlap each
+//     other's matrix and vector phases.  The matrix cores are then busy 48 % and
+//     the vector ALU 46 % of the time: the two barely overlap, which bounds it.
+//   * NG = 2 (64 queries): half the chain of tiles per wave and twice the
+//     workgroups, for launches whose longest blocks bound NG = 1; S of the next
+//     tile is issued between the exponentials (two waves per SIMD), and the two
+//     partial states of a query block are merged at the end.
+// Operator times on MI355X, attn_fwd_kernel / NG = 1 / NG = 2 (us): causal GQA
+// 32/8 x 4096 215 / 153 / 182, 28/4 x 1280 40.5 / 39.7 / 34.2, 32/8 x 512 19.4 /
+// 23.0 / 19.5; ViT 16 x 72, images of 1024, 1600, 484, 2304, 196 tokens 110 / 91 /
+// 96, 2 x 196 10.8 / 13.0 / 12.2.
+// ---------------------------------------------------------------------------
+template <int D, int KS, int NG, bool kCausal, bool kBias, bool kQNorm, bool kVarlen>
+__global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_kernel(AttnArgs a) {
+  static_assert(!kVarlen || (!kCausal && !kBias && !kQNorm),
+                "variable-length mode: no mask, no fused Q normalisation");
+  constexpr int NW = 4, NQ = NW / NG, BN = kTileKeys, QB = 32 * NQ;
+  constexpr int KCH = D / 16;               // 1 KB chunks of a part of the packed tile
+  constexpr int DBLK = D / 32;              // 32-row blocks of O^T
+  constexpr int NK = NG * KS, NV = NG * KCH;  // chunks of a K / V slot (KS of K's KCH: the others are zero padding)
+  constexpr int NDK = (NK + NW - 1) / NW, NDV = (NV + NW - 1) / NW;  // chunks each wave loads
+  constexpr bool PIPE = NG > 1;             // S(i + 1) issued within step i
+  constexpr int NKS = 3, NVS = PIPE ? 2 : 3;  // ring slots
+  constexpr int TILE_BYTES = 128 * D;
+  constexpr int OP = D + 8;                 // pitch of the output rows staged in LDS
+  constexpr int kFlagTiles = 64 * 32;       // tiles with a bias flag; later ones always take the bias
+  constexpr int RING = (NKS * NK + NVS * NV) * 64;
+  constexpr int MERGE = NG > 1 ? NW * ((DBLK + 1) / 2 * 4 + 1) * 64 : 0;  // float4s of the state exchange
+  static_assert(NG == 1 || NG == 2, "key groups");
+  static_assert(MERGE + NQ * 32 * OP / 8 <= RING, "state exchange and output staging fit the rings");
+  __shared__ u32x4 ring[RING];
+  if (static_cast<int>(blockIdx.x) >= a.n_work) {  // warm-up workgroups (no barrier, no LDS)
+    warm_lines(a.warm, static_cast<int>(blockIdx.x) - a.n_work, 256);
+    return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int wq = wave % NQ, kg = wave / NQ;
+  const int l32 = lane & 31, g = lane >> 5;
+
+  // XCD-aware work mapping (workgroup i runs on XCD i % 8).  Causal: gsz XCDs
+  // share nh heads (gsz the smallest power of two for which the heads divide
+  // evenly) and take their query blocks longest first over all of those heads,
+  // so that the last blocks to start are the shortest.  Otherwise as attn_fwd_kernel.
+  int qb, h, b;
+  {
+    const int i = static_cast<int>(blockIdx.x), nqb = a.num_q_blocks;
+    int ph;
+    if constexpr (kCausal) {
+      const int xcd = i % kXcds, idx = i / kXcds * a.gsz + xcd % a.gsz;
+      const int qi = __builtin_amdgcn_readfirstlane(div_small(idx, a.nh));
+      if (qi >= nqb) return;
+      ph = xcd / a.gsz * a.nh + idx - qi * a.nh;
+      qb = nqb - 1 - qi;
+    } else {
+      const int total = a.n_work;
+      const int per = total / kXcds, rem = total % kXcds;
+      const int xcd = i % kXcds, k = i / kXcds;
+      const int p = xcd < rem ? xcd * (per + 1) + k : rem * (per + 1) + (xcd - rem) * per + k;
+      ph = __builtin_amdgcn_readfirstlane(div_small(p, nqb));  // batch * hq + head
+      qb = p - ph * nqb;
+    }
+    b = __builtin_amdgcn_readfirstlane(div_small(ph, a.hq));
+    h = ph - b * a.hq;
+  }
+  int sq = a.sq, sk = a.sk;
+  int64_t row0 = 0, tile0 = 0;
+  if constexpr (kVarlen) {
+    const SeqSlot ss = find_seq_slot<QB>(a.cu_seqlens, a.num_seqs, a.total_rows, qb);
+    const int lq = qb - ss.base;
+    if (lq < 0 || lq >= (ss.len + QB - 1) / QB) return;
+    qb = lq;
+    sq = sk = ss.len;
+    row0 = ss.start;
+    tile0 = (static_cast<int64_t>(ss.start) + 31 * static_cast<int64_t>(ss.seq)) / 32;
+  }
+  const int hk = __builtin_amdgcn_readfirstlane(div_small(h, a.group));
+  const int q_first = qb * QB + 32 * wq;  // the wave's first query
+  const int q_idx = q_first + l32;        // this lane's query
+  const int k_end = kCausal ? min(sk, min(sq, qb * QB + QB)) : sk;
+  const int ntiles = (k_end + BN - 1) / BN;  // >= 1
+  const int nsteps = (ntiles + NG - 1) / NG;
+  const int head_tiles = (sk + BN - 1) / BN;
+  // tiles below this are computed by the wave's query block (causal: up to its
+  // own last query; none past the last query row)
+  const int tile_end = q_first >= sq ? 0 : (kCausal ? min(ntiles, q_first / BN + 1) : ntiles);
+
+  // Q rows (older than every ring load, so waiting for them waits for nothing else)
+  bf16x8 qreg[KS];
+  const uint16_t* qrow = a.q + b * a.q_sb + h * a.q_sh + (row0 + min(q_idx, sq - 1)) * a.q_ss + g * 8;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+    qreg[ks] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(qrow + ks * 16));
+
+  const __amdgpu_buffer_rsrc_t kvr =
+      make_rsrc(a.kv + b * a.kv_sb + hk * a.kv_sh + tile0 * kv_tile_elems(D), head_tiles * TILE_BYTES);
+  u32x4* const kring = ring;
+  u32x4* const vring = ring + NKS * NK * 64;
+  // the K (V) part of step st's tiles (clamped) into a ring slot; a chunk that
+  // two waves load is written twice with the same bytes
+  auto dma_k = [&](int st, int slot) {
+#pragma unroll
+    for (int j = 0; j < NDK; ++j) {
+      const int c = min(wave + NW * j, NK - 1), t = min(st * NG + c / KS, ntiles - 1);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          kvr, (__attribute__((address_space(3))) void*)(kring + (slot * NK + c) * 64), 16, lane * 16,
+          t * TILE_BYTES + c % KS * 1024, 0, 0);
+    }
+  };
+  auto dma_v = [&](int st, int slot) {
+#pragma unroll
+    for (int j = 0; j < NDV; ++j) {
+      const int c = min(wave + NW * j, NV - 1), t = min(st * NG + c / KCH, ntiles - 1);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          kvr, (__attribute__((address_space(3))) void*)(vring + (slot * NV + c) * 64), 16, lane * 16,
+          t * TILE_BYTES + TILE_BYTES / 2 + c % KCH * 1024, 0, 0);
+    }
+  };
+  dma_k(0, 0);
+  if constexpr (PIPE) {
+    dma_k(1, 1);
+    dma_v(0, 0);
+    dma_k(2, 2);
+  } else {
+    dma_v(0, 0);
+    dma_k(1, 1);
+    dma_v(1, 1);
+  }
+
+  __amdgpu_buffer_rsrc_t bsr;
+  uint32_t bflag = 0;
+  if constexpr (kBias) {
+    // one flag bit per tile: any bias entry that is not +0 / -0 (NaN != 0 is
+    // true); lane j holds the bits of tiles 32 j .. 32 j + 31 (in a register: an
+    // LDS read in the loop would wait for every ring load in flight)
+    bsr = make_rsrc(a.key_bias + b * a.kb_sb, a.sk * 4);  // past sk: reads 0
+    for (int t0 = 0; t0 < min(ntiles, kFlagTiles); t0 += 16) {
+      float v[8];
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        v[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(bsr, ((t0 + 2 * r) * BN + lane) * 4, 0, 0));
+      uint32_t bits = 0;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const uint64_t bal = __ballot(v[r] != 0.f);
+        bits |= (static_cast<uint32_t>(bal) ? 1u : 0u) << (2 * r);
+        bits |= (static_cast<uint32_t>(bal >> 32) ? 2u : 0u) << (2 * r);
+      }
+      if (lane == (t0 >> 5)) bflag |= bits << (t0 & 31);
+    }
+  }
+  if constexpr (kQNorm) {
+    static_assert(!kQNorm || KS == KCH, "whole head rows");
+    qnorm_rope_own<D>(qreg, a, q_idx, q_idx < sq, qnorm_rinv<D>(qreg, a.eps));
+  }
+
+  floatx16 oacc[DBLK];
+#pragma unroll
+  for (int db = 0; db < DBLK; ++db) oacc[db] = floatx16{};
+  const bf16x2_t kOnes = {static_cast<__bf16>(1.0f), static_cast<__bf16>(1.0f)};
+  float m_ref = -__builtin_inff(), l_part = 0.f;
+  const float c = a.scale_log2;
+  const float kb = kLog2e / c;
+
+  u32x4 kop[KS], vop[KCH];
+  auto read_k = [&](int slot) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) kop[ks] = kring[(slot * NK + kg * KS + ks) * 64 + lane];
+  };
+  auto read_v = [&](int slot) {
+#pragma unroll
+    for (int cc = 0; cc < KCH; ++cc) vop[cc] = vring[(slot * NV + kg * KCH + cc) * 64 + lane];
+  };
+
+  auto score_mma = [&](int ks, floatx16& s) {
+    s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kop[ks]), qreg[ks], s, 0, 0, 0);
+  };
+  floatx16 sa = floatx16{}, sb;
+  if constexpr (PIPE) {
+    vm_wait_barrier<2 * NDK + NDV>();  // K of step 0 is in LDS
+    read_k(0);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) score_mma(ks, sa);
+  }
+
+  // Step i of the wave's tile t.  PIPE: scores S(i) in s; softmax of S(i) with the
+  // S(i + 1) MFMAs between the exponentials, then P(i) V(i).  Otherwise S(i), its
+  // softmax and P(i) V(i) in sequence.
+  int kslot = PIPE ? 1 : 0;  // ring slot of the K part that step i reads
+  auto body = [&](int i, int vslot, floatx16& s, floatx16& snew) {
+    const int kprev = kslot == 0 ? NKS - 1 : kslot - 1;
+    if constexpr (PIPE) {
+      vm_wait_barrier<NDK>();  // K(i + 1) and V(i) are in LDS; the slots of K(i) and V(i - 1) are free
+      dma_v(i + 1, vslot ^ 1);
+      dma_k(i + 3, kprev);
+    } else {
+      vm_wait_barrier<NDK + NDV>();  // K(i) and V(i) are in LDS; the slots of step i - 1 are free
+      dma_k(i + 2, kprev);
+      dma_v(i + 2, kprev);
+    }
+    const int t = i * NG + kg;
+    const int kcur = kslot;
+    kslot = kslot + 1 == NKS ? 0 : kslot + 1;
+    if (t >= tile_end) return;
+    read_k(kcur);
+    if constexpr (PIPE) {
+      read_v(vslot);
+    } else {
+      s = floatx16{};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) score_mma(ks, s);
+      read_v(kcur);
+    }
+    const int k0 = t * BN;
+    bool btile = false;
+    if constexpr (kBias)
+      btile = t >= kFlagTiles || ((__builtin_amdgcn_readlane(bflag, t >> 5) >> (t & 31)) & 1u);
+    if ((k0 + BN > sk) || (kCausal && k0 + BN - 1 > q_first) || btile) {
+      floatx4 bn[4] = {};
+      if constexpr (kBias) {
+        if (btile) load_bias(bn, bsr, k0 + 4 * g);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int key = k0 + 8 * (e >> 2) + 4 * g + (e & 3);
+        float sv = s[e];
+        if constexpr (kBias) {
+          if (btile) sv += bn[e >> 2][e & 3] * kb;
+        }
+        bool ok = key < sk;
+        if constexpr (kCausal) ok = ok && (key <= q_idx);
+        s[e] = ok ? sv : -__builtin_inff();
+      }
+    }
+    float mt = s[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mt = fmaxf(mt, s[e]);
+    mt *= c;
+    if (__any(mt > m_ref + kLazyThreshold)) {
+      const float mq = pair_max(mt);
+      const float new_ref = mq > m_ref + kLazyThreshold ? mq : m_ref;
+      const float alpha = (m_ref == -__builtin_inff()) ? 0.f : __builtin_amdgcn_exp2f(m_ref - new_ref);
+      m_ref = new_ref;
+      l_part *= alpha;
+#pragma unroll
+      for (int db = 0; db < DBLK; ++db) oacc[db] *= alpha;
+    }
+    const float nm = (m_ref == -__builtin_inff()) ? 0.f : -m_ref;
+    if constexpr (PIPE) snew = floatx16{};
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      s[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e], c, nm));
+      if constexpr (PIPE) {
+#pragma unroll
+        for (int ks = e * KS / 16; ks < (e + 1) * KS / 16; ++ks) score_mma(ks, snew);
+      }
+    }
+    bf16x8 pop[2];
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2) {
+      floatx8 pv;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) pv[e] = s[s2 * 8 + e];
+      pop[s2] = __builtin_convertvector(pv, bf16x8);
+      // the row sum takes the rounded P, so that P V / l is a mean of V with weights that sum to one
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        l_part = __builtin_amdgcn_fdot2_f32_bf16(bf16x2_t{pop[s2][2 * e], pop[s2][2 * e + 1]}, kOnes, l_part, false);
+    }
+#pragma unroll
+    for (int s2 = 0; s2 < 2; ++s2)
+#pragma unroll
+      for (int db = 0; db < DBLK; ++db)
+        oacc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, vop[db * 2 + s2]), pop[s2],
+                                                           oacc[db], 0, 0, 0);
+  };
+  if constexpr (PIPE) {
+    for (int i = 0; i < nsteps; i += 2) {
+      body(i, 0, sa, sb);
+      if (i + 1 >= nsteps) break;
+      body(i + 1, 1, sb, sa);
+    }
+  } else {
+    for (int i = 0; i < nsteps; ++i) body(i, 0, sa, sb);
+  }
+
+  vm_wait_barrier<0>();  // every wave has read its last tile, no ring load is in flight
+  constexpr int DB0 = NG == 1 ? DBLK : (DBLK + 1) / 2;  // d-blocks finished by key group 0 (the others by group 1)
+  float l = pair_sum(l_part), inv;
+  if constexpr (NG == 1) {
+    inv = l > 0.f ? 1.0f / l : 0.f;
+  } else {
+    // each key group hands the other the partial O of the d-blocks the other finishes
+    floatx4* const ex = reinterpret_cast<floatx4*>(ring);
+    floatx4* const mine = ex + wave * ((DB0 * 4 + 1) * 64);
+#pragma unroll
+    for (int db = 0; db < DBLK; ++db)
+      if ((db < DB0) == (kg == 1)) {
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4)
+          mine[((db < DB0 ? db : db - DB0) * 4 + q4) * 64 + lane] =
+              floatx4{oacc[db][q4 * 4], oacc[db][q4 * 4 + 1], oacc[db][q4 * 4 + 2], oacc[db][q4 * 4 + 3]};
+      }
+    mine[DB0 * 4 * 64 + lane] = floatx4{m_ref, l, 0.f, 0.f};
+    __syncthreads();
+    const floatx4* const part = ex + (wave ^ NQ) * ((DB0 * 4 + 1) * 64);
+    const floatx4 ml = part[DB0 * 4 * 64 + lane];
+    const float m = fmaxf(m_ref, ml[0]);
+    const float w0 = m_ref == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(m_ref - m);
+    const float w1 = ml[0] == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(ml[0] - m);
+    l = kg == 0 ? l * w0 + ml[1] * w1 : ml[1] * w1 + l * w0;  // the same bits in both groups
+    inv = l > 0.f ? 1.0f / l : 0.f;
+#pragma unroll
+    for (int db = 0; db < DBLK; ++db)
+      if ((db < DB0) == (kg == 0)) {
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const floatx4 o = part[((db < DB0 ? db : db - DB0) * 4 + q4) * 64 + lane];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) oacc[db][q4 * 4 + e] = oacc[db][q4 * 4 + e] * w0 + o[e] * w1;
+        }
+      }
+  }
+  // O rows through LDS to 16-byte pieces of whole rows (a wave writes and reads only the columns it finishes)
+  uint16_t* const ost = reinterpret_cast<uint16_t*>(ring + MERGE) + wq * (32 * OP);
+#pragma unroll
+  for (int db = 0; db < DBLK; ++db)
+    if (NG == 1 || (db < DB0) == (kg == 0)) {
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        uint2 wv;
+        wv.x = pack_bf16x2(oacc[db][4 * q4] * inv, oacc[db][4 * q4 + 1] * inv);
+        wv.y = pack_bf16x2(oacc[db][4 * q4 + 2] * inv, oacc[db][4 * q4 + 3] * inv);
+        *reinterpret_cast<uint2*>(ost + l32 * OP + db * 32 + q4 * 8 + g * 4) = wv;
+      }
+    }
+  const int d0 = kg == 0 ? 0 : DB0 * 32;                        // the wave's first column
+  const int cpr = (NG == 1 ? DBLK : kg == 0 ? DB0 : DBLK - DB0) * 4;  // its 16-byte pieces per row
+  for (int idx = lane; idx < 32 * cpr; idx += 64) {
+    const int r = idx / cpr, d = d0 + (idx - r * cpr) * 8;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(ost + r * OP + d);
+    const int qr = q_first + r;
+    bool stored = qr < sq && d < a.d_store;
+    if (a.o_packed_k > 0) {
+      int prow = qr;
+      if (a.o_nseg > 0) {
+        const bool s1 = a.o_nseg > 1 && qr >= a.o_seg_off[1], s2 = a.o_nseg > 2 && qr >= a.o_seg_off[2];
+        const int off = s2 ? a.o_seg_off[2] : s1 ? a.o_seg_off[1] : a.o_seg_off[0];
+        const int rows = s2 ? a.o_seg_rows[2] : s1 ? a.o_seg_rows[1] : a.o_seg_rows[0];
+        const int base = s2 ? a.o_seg_base[2] : s1 ? a.o_seg_base[1] : a.o_seg_base[0];
+        stored = stored && qr >= off && qr - off < rows;
+        prow = base + b * rows + (qr - off);
+      }
+      if (stored)
+        *reinterpret_cast<u32x4*>(a.o + packed_act_offset(prow, static_cast<int64_t>(h) * D + d, a.o_packed_k)) = v;
+    } else if (stored) {
+      uint16_t* dst = a.o + b * a.o_sb + h * a.o_sh + (row0 + qr) * a.o_ss + d;
+      if (a.o_vec16) {
+        *reinterpret_cast<u32x4*>(dst) = v;
+      } else {  // rows of 8-byte alignment only
+        *reinterpret_cast<uint2*>(dst) = uint2{v[0], v[1]};
+        *reinterpret_cast<uint2*>(dst + 4) = uint2{v[2], v[3]};
       }
     }
   }
@@ -1073,10 +1498,52 @@ constexpr int vit_padded_dim(int64_t hd) {
   return (hd < 8 || hd > 128 || hd % 8) ? 0 : (hd <= 64 ? 64 : (hd <= 96 ? 96 : 128));
 }
 
+// Key groups of attn_shared_kernel for a launch, or 0 for attn_fwd_kernel.
+// b64, b128: the launch's 64- and 128-query blocks per head; heads: batch x heads.
+// Measured on MI355X (operator us, attn_fwd_kernel / NG = 1 / NG = 2):
+//   causal: the longest block bounds a launch until the blocks of every length
+//   fill the chip, which heads x (blocks + 1) measures (twice the work over the
+//   longest chain).  NG = 2 wins from 440 (32/8 x 800: 29.5 / 28.3 / 25.2 at 448; 32/8 x
+//   512: 19.4 / 23.0 / 19.5 at 288), with chains past 20 steps from 528 (16/8 x 1536: 34.6 /
+//   43.5 / 36.0 at 400, x 2048: 44.7 / 53.9 / 44.5 at 528, x 2560: 63.7 / 67.8 / 53.8),
+//   NG = 1 over it from 540 (32/8 x 2048: 79.7 / 64.2 / 66.1 at 544; 16/8 x 4096:
+//   122 / 111 / 102 at 528, x 6144: 228 / 190 / 202 at 784).
+//   not causal: blocks of one length run in whole rounds over the chip.  NG = 1 wins
+//   from 380 workgroups (3 images of 1024: 51.9 / 43.5 / 44.4 at 384; 2304 + 0: 63.3 /
+//   64.1 / 64.1 at 288), below that NG = 2 where it makes one round of two
+//   workgroups per CU (1600: 42.3 / 40.8 / 35.9 at 400; joint 16 x 2144: 61.5 / 62.4 /
+//   71.7 at 544, 16 x 1120: 25.4 / 28.3 / 25.8 at 288).
+int shared_groups(bool causal, int64_t heads, int64_t b64, int64_t b128) {
+  if (causal) {
+    if (heads * (b128 + 1) >= 540) return 1;
+    return heads * (b64 + 1) >= (b64 <= 20 ? 440 : 528) ? 2 : 0;
+  }
+  if (heads * b128 >= 380) return 1;
+  return heads * b64 >= 400 && heads * b64 <= 512 ? 2 : 0;
+}
+
 template <int DP>
 hipError_t launch_vit(const VitArgs& v, AttnArgs a, int64_t slots, hipStream_t stream) {
   hipLaunchKernelGGL(vit_pack_kernel<DP>, dim3(static_cast<unsigned>(slots), static_cast<unsigned>(v.heads)),
                      dim3(256), 0, stream, v);
+  const int64_t b64 = seq_slot_count(v.rows, v.num_seqs, 64), b128 = seq_slot_count(v.rows, v.num_seqs, 128);
+  const int groups = shared_groups(false, v.heads, b64, b128);
+  if (groups > 0) {
+    a.num_q_blocks = static_cast<int>(groups == 1 ? b128 : b64);
+    a.n_work = a.num_q_blocks * v.heads;
+    const dim3 grid(static_cast<unsigned>(a.n_work));
+    constexpr int KS = DP / 16, KSN = DP == 96 ? 5 : KS;  // head_dim <= 80: the sixth 16-column step is all padding
+    const bool narrow = DP == 96 && v.hd <= 80;
+    if (groups == 1 && narrow)
+      hipLaunchKernelGGL((attn_shared_kernel<DP, KSN, 1, false, false, false, true>), grid, dim3(256), 0, stream, a);
+    else if (groups == 1)
+      hipLaunchKernelGGL((attn_shared_kernel<DP, KS, 1, false, false, false, true>), grid, dim3(256), 0, stream, a);
+    else if (narrow)
+      hipLaunchKernelGGL((attn_shared_kernel<DP, KSN, 2, false, false, false, true>), grid, dim3(256), 0, stream, a);
+    else
+      hipLaunchKernelGGL((attn_shared_kernel<DP, KS, 2, false, false, false, true>), grid, dim3(256), 0, stream, a);
+    return hipGetLastError();
+  }
   a.num_q_blocks = static_cast<int>(slots);
   a.n_work = static_cast<int>(slots * v.heads);
   hipLaunchKernelGGL((attn_fwd_kernel<DP, 1, false, false, false, true>),
@@ -1084,9 +1551,31 @@ hipError_t launch_vit(const VitArgs& v, AttnArgs a, int64_t slots, hipStream_t s
   return hipGetLastError();
 }
 
+template <int D, int NG, bool kCausal, bool kQNorm>
+void launch_shared(const AttnArgs& a, bool has_bias, dim3 grid, hipStream_t stream) {
+  if constexpr (!kQNorm) {
+    if (has_bias) {
+      hipLaunchKernelGGL((attn_shared_kernel<D, D / 16, NG, kCausal, true, false, false>), grid, dim3(256), 0, stream, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((attn_shared_kernel<D, D / 16, NG, kCausal, false, kQNorm, false>), grid, dim3(256), 0, stream, a);
+}
+
+// (the fused Q norm comes with a causal launch without a bias)
 template <int D, int NSUB, bool kQNorm>
 void launch_attn_d(AttnArgs a, int batch, bool causal, bool has_bias, hipStream_t stream) {
+  const int64_t heads = static_cast<int64_t>(a.hq) * batch, b64 = (a.sq + 63) / 64, b128 = (a.sq + 127) / 128;
+  const int groups = shared_groups(causal, heads, b64, b128);
+  if (groups > 0) a.num_q_blocks = static_cast<int>(groups == 1 ? b128 : b64);
   a.n_work = a.num_q_blocks * a.hq * batch;
+  if (groups > 0 && causal) {
+    int sets = kXcds;
+    while (heads % sets) sets /= 2;
+    a.gsz = kXcds / sets;
+    a.nh = static_cast<int>(heads / sets);
+    a.n_work = (a.num_q_blocks * a.nh + a.gsz - 1) / a.gsz * kXcds;
+  }
   // warm-up workgroups: about 1024 lines (128 KB) each, at most 256
   int n_pf = 0;
   if (a.warm.end[2] > 0) {
@@ -1095,6 +1584,15 @@ void launch_attn_d(AttnArgs a, int batch, bool causal, bool has_bias, hipStream_
   }
   dim3 grid(static_cast<unsigned>(a.n_work + n_pf));
   dim3 block(256);
+  if (groups > 0) {
+    if (causal && groups == 1) launch_shared<D, 1, true, kQNorm>(a, has_bias, grid, stream);
+    else if (causal) launch_shared<D, 2, true, kQNorm>(a, has_bias, grid, stream);
+    if constexpr (!kQNorm) {
+      if (!causal && groups == 1) launch_shared<D, 1, false, false>(a, has_bias, grid, stream);
+      else if (!causal) launch_shared<D, 2, false, false>(a, has_bias, grid, stream);
+    }
+    return;
+  }
   if (causal) {
     if (has_bias)
       hipLaunchKernelGGL((attn_fwd_kernel<D, NSUB, true, true, kQNorm>), grid, block, 0, stream, a);
@@ -1164,6 +1662,8 @@ void fill_qo(AttnArgs& a, const void* q, void* o, int64_t q_heads, int64_t kv_he
   a.sq = static_cast<int>(seq_q);
   a.sk = static_cast<int>(seq_k);
   a.scale_log2 = scale * kLog2e;
+  a.d_store = 1 << 30;
+  a.o_vec16 = reinterpret_cast<uintptr_t>(o) % 16 == 0 && os[0] % 8 == 0 && os[1] % 8 == 0 && os[2] % 8 == 0;
 }
 
 }  // namespace
@@ -1519,6 +2019,7 @@ extern "C" hipError_t rldx_vision_attention_bf16(const void* qkv, const float* r
   a.num_seqs = v.num_seqs;
   a.total_rows = v.rows;
   a.d_store = v.hd;
+  a.o_vec16 = a16(out);  // (whole rows and heads of num_heads * head_dim and head_dim % 8 columns)
   if (dp == 64) return launch_vit<64>(v, a, slots, stream);
   if (dp == 96) return launch_vit<96>(v, a, slots, stream);
   return launch_vit<128>(v, a, slots, stream);

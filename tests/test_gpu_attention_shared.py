@@ -1,0 +1,96 @@
+"""The attention kernel with K/V tiles shared through LDS (launches that fill the
+chip), at the edges of its query blocks, key tiles and key groups, against the
+CPU oracle; tolerances of the bf16 attention tests."""
+
+import pytest
+import torch
+
+from oracle import cpu_reference as ref
+from rldx_amd import functional as Fn
+from rldx_amd import workloads as W
+from tolerances import assert_bf16_close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return torch.device("cuda:0")
+
+
+def _inputs(B, Hq, Hkv, Sq, Sk, D, bias):
+    g = torch.Generator().manual_seed(Hq * 100 + Sq + Sk + D)
+    q, k, v = (torch.randn(B, h, s, D, generator=g).to(torch.bfloat16) for h, s in ((Hq, Sq), (Hkv, Sk), (Hkv, Sk)))
+    kb = None
+    if bias:
+        kb = torch.zeros(B, Sk)
+        kb[0, ::3] = 0.5 * torch.randn((Sk + 2) // 3, generator=g)  # every tile
+        if B > 1:  # whole tiles masked, one raised key, the rest zero
+            kb[1, 64:161] = float("-inf")
+            kb[1, 7] = 1.5
+    return q, k, v, kb
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,bias", [
+    # 128 queries per workgroup
+    (1, 128, 16, 417, 417, 128, True, False),
+    (1, 135, 135, 417, 417, 64, True, False),    # heads not divisible over the XCDs
+    (1, 128, 16, 513, 300, 128, True, True),     # queries past the last key
+    (2, 70, 10, 400, 500, 64, True, True),
+    (4, 32, 8, 290, 333, 128, False, True),
+    (4, 32, 32, 384, 32, 128, False, False),     # one key tile
+    (2, 64, 64, 257, 97, 64, False, True),
+    # 64 queries and two key groups per workgroup
+    (1, 64, 16, 449, 449, 128, True, False),
+    (1, 220, 4, 64, 64, 64, True, False),        # one query block: the second group's only tile is the diagonal
+    (2, 30, 10, 449, 449, 128, True, True),
+    (2, 32, 8, 400, 33, 128, False, True),       # a second key group with one partial tile
+    (1, 64, 64, 400, 31, 64, False, False),      # a second key group without a tile
+    (2, 32, 32, 400, 545, 64, False, True),
+])
+def test_attention_shared_tiles(dev, B, Hq, Hkv, Sq, Sk, D, causal, bias):
+    q, k, v, kb = _inputs(B, Hq, Hkv, Sq, Sk, D, bias)
+    o = Fn.attention(q.to(dev), k.to(dev), v.to(dev), key_bias=None if kb is None else kb.to(dev), causal=causal)
+    r = ref.sdpa(q, ref.repeat_kv(k, Hq // Hkv), ref.repeat_kv(v, Hq // Hkv), key_bias=kb, causal=causal)
+    assert_bf16_close(o, r, "attention, shared tiles")
+
+
+@pytest.mark.parametrize("B,H,S,D", [(4, 32, 290, 128), (2, 32, 400, 64)])
+def test_attention_shared_outputs(dev, B, H, S, D):
+    """Rows of 8-byte alignment, and the packed output by row segments: the same bits as contiguous rows."""
+    q, k, v, kb = (t.to(dev) for t in _inputs(B, H, H, S, S, D, True))
+    kvp = Fn.kv_pack(k, v)
+    o = Fn.attention_packed(q, kvp, S, key_bias=kb)
+    wide = torch.zeros(B, H, S, D + 4, dtype=torch.bfloat16, device=dev)
+    Fn.attention_packed(q, kvp, S, key_bias=kb, out=wide[..., :D])
+    assert torch.equal(wide[..., :D], o) and not wide[..., D:].any()
+    cut = 96  # rows [0, cut) of every batch entry, then rows [cut + 5, S); the 5 between are not stored
+    n1 = S - cut - 5
+    packed = Fn.PackedAct.empty(B * (cut + n1), H * D, dev)
+    Fn.attention_packed(q, kvp, S, key_bias=kb, out=packed, segments=[(0, cut, 0), (cut + 5, n1, B * cut)])
+    rows = o.permute(0, 2, 1, 3).reshape(B, S, H * D)
+    want = torch.cat([rows[:, :cut].reshape(-1, H * D), rows[:, cut + 5:].reshape(-1, H * D)])
+    assert torch.equal(packed.unpack(), want)
+
+
+@pytest.mark.parametrize("M,Hq,Hkv,D", [(449, 64, 16, 128), (417, 128, 16, 128), (385, 140, 4, 64), (70, 160, 8, 64)])
+def test_gqa_operator_shared_tiles(dev, M, Hq, Hkv, D):
+    """The fused Q norm + RoPE of a wave's own rows."""
+    inp = W.gqa_inputs(W.GqaCfg(q_heads=Hq, kv_heads=Hkv, head_dim=D, seq=M, seed=M))
+    o = Fn.llm_fused_attention(*(inp[n].to(dev) for n in ("qkv", "q_norm_w", "k_norm_w", "cos")),
+                               W.signed_sin(inp["sin"]).to(dev), Hq, Hkv, D)
+    r = ref.llm_fused_attention(inp["qkv"], inp["q_norm_w"], inp["k_norm_w"], inp["cos"], inp["sin"], Hq, Hkv, D)
+    assert_bf16_close(o, r, "GQA operator, shared tiles")
+
+
+@pytest.mark.parametrize("lengths,H,D", [
+    ((300, 1, 0, 450, 129), 48, 72), ((300, 1, 0, 450, 129), 48, 88), ((300, 1, 0, 450, 129), 48, 64),
+    ((300, 1, 0, 450, 129), 48, 120), ((300, 1, 0, 450, 129), 24, 72), ((300, 1, 0, 450, 129), 24, 96),
+    ((300, 1, 0, 450, 129), 24, 64), ((65, 448, 64), 48, 128),
+    (tuple((37 * i) % 50 for i in range(70)), 8, 80),  # binary-search lookup
+])
+def test_vision_attention_shared_tiles(dev, lengths, H, D):
+    inp = W.vit_attention_inputs(W.VitAttnCfg(lengths=lengths, heads=H, head_dim=D, seed=len(lengths) * 100 + D))
+    t = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in inp.items()}
+    o = Fn.vision_attention(t["qkv"], t["rope_cos"], t["rope_sin"], t["cu_seqlens"], t["scaling"], H, D)
+    assert_bf16_close(o, ref.vision_attention(**inp), f"vision attention {lengths} H={H} D={D}")
