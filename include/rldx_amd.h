@@ -248,6 +248,20 @@ hipError_t rldx_attention_packed_fwd_bf16(const void* q, const void* kv_packed, 
                                           hipStream_t stream);
 
 /*
+ * rldx_attention_packed_fwd_bf16 with a key mask in place of the additive bias:
+ * key_mask [batch or 1, seq_k] fp32 (row stride key_mask_batch_stride, 0 = one
+ * row for every batch entry), 0 = masked key, any other value visible
+ * (rldx/model/modules/action_model/blocks.py:843-864).  The same results as
+ * the bias 0 / -inf built from it, without a launch that builds it.
+ */
+hipError_t rldx_attention_packed_fwd_mask_bf16(const void* q, const void* kv_packed, const int64_t* packed_strides,
+                                               void* o, int32_t out_packed, int64_t batch, int64_t q_heads,
+                                               int64_t kv_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim,
+                                               const int64_t* q_strides, const int64_t* o_strides,
+                                               const float* key_mask, int64_t key_mask_batch_stride, float scale,
+                                               int32_t causal, hipStream_t stream);
+
+/*
  * rldx_attention_packed_fwd_bf16 with O written to a packed activation matrix
  * (out_packed as there, o_strides unused) by row segments, for a batch of
  * joint sequences whose streams the GEMMs hold stream by stream (every batch

@@ -93,12 +93,19 @@ __device__ __forceinline__ float pair_sum(float x) {
 
 // The 16 bias values of a lane's S^T accumulator rows: keys key0 + 8*qq + c,
 // qq, c in 0..3, with key0 = tile start + 4 * (lane half).
-__device__ __forceinline__ void load_bias(floatx4 (&out)[4], __amdgpu_buffer_rsrc_t r, int key0) {
+// is_mask: the entries are a key mask (0 = masked) and become -inf / 0.
+__device__ __forceinline__ void load_bias(floatx4 (&out)[4], __amdgpu_buffer_rsrc_t r, int key0, bool is_mask) {
 #pragma unroll
   for (int qq = 0; qq < 4; ++qq)
 #pragma unroll
     for (int cc = 0; cc < 4; ++cc)
       out[qq][cc] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, key0 * 4 + 32 * qq + 4 * cc, 0, 0));
+  if (is_mask) {
+#pragma unroll
+    for (int qq = 0; qq < 4; ++qq)
+#pragma unroll
+      for (int cc = 0; cc < 4; ++cc) out[qq][cc] = out[qq][cc] == 0.f ? -__builtin_inff() : 0.f;
+  }
 }
 
 struct AttnArgs {
@@ -117,6 +124,7 @@ struct AttnArgs {
   int o_seg_off[3], o_seg_rows[3], o_seg_base[3];
   const float* key_bias;  // [batch, sk] additive (natural-log units) or nullptr
   int64_t kb_sb;
+  int bias_is_mask;  // key_bias holds a key mask: 0 = masked (bias -inf), any other value visible (bias 0)
   int hq, hkv, group, sq, sk;
   int num_q_blocks;
   int gsz, nh;  // attn_shared_kernel, causal: XCDs per group of nh heads
@@ -471,11 +479,12 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_kernel(AttnArgs a) {
 
   // bias flags (NaN != 0 is true: a NaN bias is applied, not skipped)
   auto flagged = [&](int i) { return i >= 64 || ((wbias >> i) & 1ull); };
-  auto load_bias_of = [&](floatx4 (&dst)[4], int i) { load_bias(dst, bsr, (wave + NW * i) * BN + 4 * g); };
+  auto load_bias_of = [&](floatx4 (&dst)[4], int i) { load_bias(dst, bsr, (wave + NW * i) * BN + 4 * g, a.bias_is_mask); };
   if constexpr (kBias) {
+    const uint64_t flip = a.bias_is_mask ? ~0ull : 0ull;  // a mask: entries that are zero
 #pragma unroll
     for (int r = 0; r < kScanLoads; ++r) {
-      const uint64_t bal = __ballot(bscan[r] != 0.f);
+      const uint64_t bal = __ballot(bscan[r] != 0.f) ^ flip;
       if (bal & 0xffffffffull) wbias |= 1ull << (2 * r);
       if (bal >> 32) wbias |= 1ull << (2 * r + 1);
     }
@@ -838,6 +847,7 @@ __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_ke
     // true); lane j holds the bits of tiles 32 j .. 32 j + 31 (in a register: an
     // LDS read in the loop would wait for every ring load in flight)
     bsr = make_rsrc(a.key_bias + b * a.kb_sb, a.sk * 4);  // past sk: reads 0
+    const uint64_t flip = a.bias_is_mask ? ~0ull : 0ull;  // a mask: entries that are zero
     for (int t0 = 0; t0 < min(ntiles, kFlagTiles); t0 += 16) {
       float v[8];
 #pragma unroll
@@ -846,7 +856,7 @@ __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_ke
       uint32_t bits = 0;
 #pragma unroll
       for (int r = 0; r < 8; ++r) {
-        const uint64_t bal = __ballot(v[r] != 0.f);
+        const uint64_t bal = __ballot(v[r] != 0.f) ^ flip;
         bits |= (static_cast<uint32_t>(bal) ? 1u : 0u) << (2 * r);
         bits |= (static_cast<uint32_t>(bal >> 32) ? 2u : 0u) << (2 * r);
       }
@@ -922,7 +932,7 @@ __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_ke
     if ((k0 + BN > sk) || (kCausal && k0 + BN - 1 > q_first) || btile) {
       floatx4 bn[4] = {};
       if constexpr (kBias) {
-        if (btile) load_bias(bn, bsr, k0 + 4 * g);
+        if (btile) load_bias(bn, bsr, k0 + 4 * g, a.bias_is_mask);
       }
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
@@ -1734,7 +1744,8 @@ hipError_t attention_packed(const void* q, const void* kv_packed, const int64_t*
                             int64_t q_heads, int64_t kv_heads, int64_t seq_q, int64_t seq_k, int64_t head_dim,
                             const int64_t* q_strides, const int64_t* o_strides, const float* key_bias,
                             int64_t key_bias_batch_stride, float scale, int32_t causal, const void* const* warm_ptrs,
-                            const int64_t* warm_bytes, int32_t warm_count, hipStream_t stream) {
+                            const int64_t* warm_bytes, int32_t warm_count, hipStream_t stream,
+                            bool bias_is_mask = false) {
   const int64_t zero3[3] = {0, 0, 0};
   if (num_segments && (!out_packed || !segments_ok(segments, num_segments, batch, seq_q)))
     return hipErrorInvalidValue;
@@ -1757,6 +1768,7 @@ hipError_t attention_packed(const void* q, const void* kv_packed, const int64_t*
   if (key_bias && reinterpret_cast<uintptr_t>(key_bias) % 4) return hipErrorInvalidValue;
   AttnArgs a{};
   fill_qo(a, q, o, q_heads, kv_heads, seq_q, seq_k, q_strides, o_strides, key_bias, key_bias_batch_stride, scale);
+  a.bias_is_mask = bias_is_mask ? 1 : 0;
   a.o_packed_k = out_packed > 1 ? out_packed : (out_packed ? q_heads * head_dim : 0);
   a.o_nseg = num_segments;
   for (int s = 0; s < num_segments; ++s) {
@@ -1782,6 +1794,19 @@ extern "C" hipError_t rldx_attention_packed_fwd_bf16(const void* q, const void* 
   return attention_packed(q, kv_packed, packed_strides, o, out_packed, nullptr, 0, batch, q_heads, kv_heads, seq_q,
                           seq_k, head_dim, q_strides, o_strides, key_bias, key_bias_batch_stride, scale, causal,
                           nullptr, nullptr, 0, stream);
+}
+
+extern "C" hipError_t rldx_attention_packed_fwd_mask_bf16(const void* q, const void* kv_packed,
+                                                          const int64_t* packed_strides, void* o, int32_t out_packed,
+                                                          int64_t batch, int64_t q_heads, int64_t kv_heads,
+                                                          int64_t seq_q, int64_t seq_k, int64_t head_dim,
+                                                          const int64_t* q_strides, const int64_t* o_strides,
+                                                          const float* key_mask, int64_t key_mask_batch_stride,
+                                                          float scale, int32_t causal, hipStream_t stream) {
+  if (!key_mask) return hipErrorInvalidValue;
+  return attention_packed(q, kv_packed, packed_strides, o, out_packed, nullptr, 0, batch, q_heads, kv_heads, seq_q,
+                          seq_k, head_dim, q_strides, o_strides, key_mask, key_mask_batch_stride, scale, causal,
+                          nullptr, nullptr, 0, stream, true);
 }
 
 extern "C" hipError_t rldx_attention_packed_segments_fwd_bf16(

@@ -450,7 +450,7 @@ def kv_pack(k: torch.Tensor, v: torch.Tensor, layout: str = "bhsd") -> torch.Ten
 def attention_packed(q: torch.Tensor, kvp: torch.Tensor, seq_k: int, *, key_bias: Optional[torch.Tensor] = None,
                      causal: bool = False, scale: Optional[float] = None, layout: str = "bhsd",
                      out=None, warm: Optional[Sequence[torch.Tensor]] = None,
-                     segments: Optional[Sequence[tuple]] = None):
+                     segments: Optional[Sequence[tuple]] = None, key_mask: Optional[torch.Tensor] = None):
     """Attention with K/V given as packed tiles [B, Hkv, >= kv_packed_elems(seq_k, D)]
     (see kv_pack; the MSAT QKV kernel writes them directly).  `out` may be a
     PackedAct [Sq, Hq*D] (batch 1), or a column view of a wider one: O is then
@@ -461,8 +461,12 @@ def attention_packed(q: torch.Tensor, kvp: torch.Tensor, seq_k: int, *, key_bias
     not stored (rldx_attention_packed_segments_fwd_bf16).  warm: up to three
     tensors (e.g. the packed weights of a later GEMM) whose memory extra
     workgroups of the launch read into the memory-side cache while it runs
-    (rldx_attention_packed_fwd_warm_bf16; the attention result is unchanged)."""
-    _on_gpu(q, kvp, key_bias)
+    (rldx_attention_packed_fwd_warm_bf16; the attention result is unchanged).
+    key_mask: fp32 [Sk] or [B or 1, Sk], 0 = masked key, in place of key_bias
+    (rldx_attention_packed_fwd_mask_bf16; no warm ranges or segments)."""
+    _on_gpu(q, kvp, key_bias, key_mask)
+    _require(key_mask is None or (key_bias is None and segments is None and not warm),
+             "key_mask replaces key_bias and goes without warm ranges and segments")
     _require(q.dtype == BF16 and q.dim() == 4 and q.stride(-1) == 1, "q must be 4-D bf16, last dim contiguous")
     if layout == "bhsd":
         B, Hq, Sq, D = q.shape
@@ -498,7 +502,7 @@ def attention_packed(q: torch.Tensor, kvp: torch.Tensor, seq_k: int, *, key_bias
         _on_gpu(out)
         _require(out.shape == q.shape and out.dtype == BF16 and out.stride(-1) == 1, "out must match q")
         o_ptr, o_strides = out.data_ptr(), _bhs_strides(out, layout)
-    kb_ptr, kb_stride = _key_bias_args(key_bias, B, seq_k)
+    kb_ptr, kb_stride = _key_bias_args(key_bias if key_mask is None else key_mask, B, seq_k)
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     lib = _lib.load()
@@ -513,6 +517,8 @@ def attention_packed(q: torch.Tensor, kvp: torch.Tensor, seq_k: int, *, key_bias
             out.ld if out.ld != out.k else 1, seg, len(segments), B, Hq, Hkv, Sq, seq_k, D,
             _lib.i64_array(_bhs_strides(q, layout)), kb_ptr, kb_stride, float(scale), int(bool(causal)),
             _stream_ptr(q)), "rldx_attention_packed_segments_fwd_bf16")
+    elif key_mask is not None:
+        _lib.check(lib.rldx_attention_packed_fwd_mask_bf16(*args, _stream_ptr(q)), "rldx_attention_packed_fwd_mask_bf16")
     elif warm:
         ptrs, nbytes, count = _warm_args(warm, q.device)
         _lib.check(lib.rldx_attention_packed_fwd_warm_bf16(*args, ptrs, nbytes, count, _stream_ptr(q)),
@@ -1226,8 +1232,8 @@ def mask_to_key_bias(kv_mask: torch.Tensor) -> torch.Tensor:
     """1 = visible / 0 = masked (the eager encoder_attention_mask convention,
     blocks.py:843-864) -> fp32 additive bias 0 / -inf."""
     m = kv_mask if kv_mask.dim() == 2 else kv_mask.unsqueeze(0)
-    return torch.where(m == 0, torch.tensor(float("-inf"), device=m.device),
-                       torch.tensor(0.0, device=m.device)).to(F32).contiguous()
+    # (Python scalars: device fills; scalar tensors would be copied from the host, each copy waited for)
+    return torch.where(m == 0, float("-inf"), 0.0).to(F32).contiguous()
 
 
 def host_swiglu_bf16_bits(g_bits, u_bits):

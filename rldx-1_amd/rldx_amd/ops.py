@@ -39,11 +39,14 @@ from . import functional as Fn
 # ---------------------------------------------------------------------------
 
 
-def _attn_from_qkv(q, kvp, key_bias, M, H, D):
-    """(H, M, D) Q + packed K/V tiles (H, E) -> (1, M, H*D) bf16, written directly in token-major order."""
+def _attn_from_qkv(q, kvp, kv_mask, M, H, D):
+    """(H, M, D) Q + packed K/V tiles (H, E) -> (1, M, H*D) bf16, written directly in token-major order.
+    kv_mask: None, or [M] / [1, M] with 0 = masked key (read by the kernel itself when it is fp32)."""
     out = torch.empty((1, M, H, D), dtype=torch.bfloat16, device=q.device)
-    Fn.attention_packed(q.unsqueeze(0), kvp.unsqueeze(0), M, key_bias=key_bias, layout="bhsd",
-                        out=out.permute(0, 2, 1, 3))
+    direct = kv_mask is not None and kv_mask.dtype == torch.float32 and kv_mask.dim() in (1, 2) and kv_mask.stride(-1) == 1
+    bias = Fn.mask_to_key_bias(kv_mask) if kv_mask is not None and not direct else None
+    Fn.attention_packed(q.unsqueeze(0), kvp.unsqueeze(0), M, key_bias=bias, layout="bhsd",
+                        out=out.permute(0, 2, 1, 3), key_mask=kv_mask if direct else None)
     return out.view(1, M, H * D)
 
 
@@ -122,8 +125,7 @@ def ds_fused_attention_3way(
         Fn.StreamSpec(_qkv_cols(p_qkv)[:n_p], q_norm_p_weight, k_norm_p_weight, p_rope_cos, p_rope_sin),
     ]
     q, kvp = Fn.msat_qkv_norm_rope(streams, H, D, kv_packed=True)
-    bias = Fn.mask_to_key_bias(kv_mask) if kv_mask is not None else None
-    return _attn_from_qkv(q, kvp, bias, n_vl + n_sa + n_p, H, D)
+    return _attn_from_qkv(q, kvp, kv_mask, n_vl + n_sa + n_p, H, D)
 
 
 @ds_fused_attention_3way.register_fake
@@ -226,8 +228,7 @@ def ss_fused_attention_3way(
     if n_p > 0:
         streams.append(Fn.StreamSpec(p, p_q_norm_weight, p_k_norm_weight, p_rope_cos, p_rope_sin))
     q, kvp = Fn.msat_qkv_norm_rope(streams, H, D, kv_packed=True)
-    bias = Fn.mask_to_key_bias(kv_mask) if kv_mask is not None else None
-    return _attn_from_qkv(q, kvp, bias, n_x + n_p, H, D)
+    return _attn_from_qkv(q, kvp, kv_mask, n_x + n_p, H, D)
 
 
 @ss_fused_attention_3way.register_fake

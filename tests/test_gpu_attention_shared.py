@@ -94,3 +94,43 @@ def test_vision_attention_shared_tiles(dev, lengths, H, D):
     t = {k: (v.to(dev) if torch.is_tensor(v) else v) for k, v in inp.items()}
     o = Fn.vision_attention(t["qkv"], t["rope_cos"], t["rope_sin"], t["cu_seqlens"], t["scaling"], H, D)
     assert_bf16_close(o, ref.vision_attention(**inp), f"vision attention {lengths} H={H} D={D}")
+
+
+@pytest.mark.parametrize("B,H,S,D", [(1, 4, 77, 64), (2, 3, 1, 128), (4, 32, 290, 128), (2, 32, 400, 64), (1, 2, 2200, 128)])
+def test_attention_key_mask(dev, B, H, S, D):
+    """A key mask read by the kernel: the bits of the 0 / -inf bias built from it (2200 keys: past the flag scan)."""
+    q, k, v, _ = (t if t is None else t.to(dev) for t in _inputs(B, H, H, S, S, D, False))
+    kvp = Fn.kv_pack(k, v)
+    g = torch.Generator().manual_seed(S)
+    mask = (torch.rand(B, S, generator=g) > 0.3).float()
+    mask[:, 0] = float("nan")  # not zero: visible
+    mask[:, S // 2:S // 2 + 40] = -0.0
+    mask = mask.to(dev)
+    for m in (mask, mask[:1]):
+        bias = torch.where(m == 0, float("-inf"), 0.0).float()
+        o = Fn.attention_packed(q, kvp, S, key_mask=m)
+        assert torch.equal(o, Fn.attention_packed(q, kvp, S, key_bias=bias))
+
+
+def test_joint_operator_mask_types(dev):
+    """kv_mask of other types, shapes and strides gives the fp32 mask's result."""
+    import rldx_amd.ops  # noqa: F401
+
+    H, D, sizes = 4, 64, (40, 18, 9)
+    g = torch.Generator().manual_seed(5)
+    sa, vl, p = (torch.randn(n, 3 * H * D, generator=g).to(torch.bfloat16).to(dev) for n in (18, 40, 9))
+    w = [(1 + 0.1 * torch.randn(D, generator=g)).to(torch.bfloat16).to(dev) for _ in range(6)]
+    cs = [torch.randn(n, D // 2, generator=g).to(dev) for n in (18, 18, 9, 9)]
+    mask = torch.ones(1, sum(sizes))
+    mask[:, 30:34] = 0
+    mask[:, -3:] = 0
+    mask = mask.to(dev)
+    call = lambda m: torch.ops.ds.fused_attention_3way(sa, vl, p, *w, *cs, 18, 40, 9, H, D, m)  # noqa: E731
+    want = call(mask)
+    wide = torch.zeros(1, 2 * sum(sizes), device=dev)
+    wide[:, ::2] = mask
+    for m in (mask[0], mask.bool(), mask.long(), mask.bfloat16(), mask.double(), wide[:, ::2]):
+        assert torch.equal(call(m), want)
+    for bad in (mask[:, 1:], mask.expand(2, -1)):
+        with pytest.raises(RuntimeError):
+            call(bad)
