@@ -638,9 +638,10 @@ class PackedWeight:
         self.data, self.n, self.k, self.swiglu_pairs, self.row_sums = data, n, k, swiglu_pairs, row_sums
 
 
-def pack_weight(w: torch.Tensor, swiglu_pairs: bool = False) -> PackedWeight:
+def pack_weight(w: torch.Tensor, swiglu_pairs: bool = False, row_sums: bool = True) -> PackedWeight:
     """nn.Linear weight [out_features, in_features] bf16 -> PackedWeight.  With
-    swiglu_pairs, w = [gate; up] and the GEMM's SwiGLU epilogue can be used."""
+    swiglu_pairs, w = [gate; up] and the GEMM's SwiGLU epilogue can be used.
+    row_sums=False leaves out the sums that only the LayerNorm fold reads."""
     _on_gpu(w)
     _require(w.dtype == BF16 and w.dim() == 2 and w.stride(1) == 1, "weight must be 2-D bf16, rows contiguous")
     n, k = w.shape
@@ -649,7 +650,7 @@ def pack_weight(w: torch.Tensor, swiglu_pairs: bool = False) -> PackedWeight:
     lib = _lib.load()
     _lib.check(lib.rldx_gemm_pack_weight_bf16(w.data_ptr(), w.stride(0), n, k, int(swiglu_pairs), out.data_ptr(),
                                               _stream_ptr(w)), "rldx_gemm_pack_weight_bf16")
-    return PackedWeight(out, n, k, swiglu_pairs, w.float().sum(dim=1).contiguous())
+    return PackedWeight(out, n, k, swiglu_pairs, w.float().sum(dim=1).contiguous() if row_sums else None)
 
 
 class PackedAct:
