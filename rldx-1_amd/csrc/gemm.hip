@@ -1510,6 +1510,7 @@ hipError_t plan(const rldx_gemm_group_t* groups, int32_t num_groups, int64_t n, 
     m_begin += qkv ? (s.m + 31) / 32 * 32 : s.m;  // QKV: each stream starts a 32-key tile
   }
   args.num_groups = cnt;
+  *ws_bytes = 0;
   if (cnt == 0) return hipSuccess;
   // heaviest workgroups first (they take the first slot of every CU; the short
   // streams' workgroups fill the second)
