@@ -746,6 +746,22 @@ hipError_t rldx_grouped_gemm_qkv_norm_rope_ln_bf16(const rldx_gemm_group_t* grou
                                                    void* kv_packed, int64_t kv_packed_head_stride, float eps,
                                                    float ln_eps, hipStream_t stream);
 
+/*
+ * The fused input linear of a single-stream block (linear1 = [QKV | MLP] columns
+ * of one A operand, qkv->a_packed / mlp->a_packed [m, k]) in one launch:
+ *   qkv: rldx_grouped_gemm_qkv_norm_rope_bf16 with one stream `norm` (weight
+ *        [3 heads head_dim, k]; the stream's tables cover all m rows), head_dim 64;
+ *   mlp: rldx_grouped_gemm_bf16 with the packed SwiGLU epilogue (weight [n_mlp, k]
+ *        in swiglu_pairs order, packed out [m, n_mlp / 2]).
+ * The results of the two calls, bit for bit.
+ * Replaces: linear1 + its split in SingleStreamBlock.forward
+ *   (rldx/model/modules/action_model/blocks.py:166-254).
+ */
+hipError_t rldx_gemm_qkv_swiglu_bf16(const rldx_gemm_group_t* qkv, const rldx_msat_stream_t* norm, int64_t heads,
+                                     int64_t head_dim, void* q_out, int64_t q_head_stride, int64_t q_row_stride,
+                                     void* kv_packed, int64_t kv_packed_head_stride, float eps,
+                                     const rldx_gemm_group_t* mlp, int64_t n_mlp, int64_t k, hipStream_t stream);
+
 /* ------------------------------------------------------------------------ */
 /* Host-side diagnostics (no reference counterpart)                         */
 /* ------------------------------------------------------------------------ */

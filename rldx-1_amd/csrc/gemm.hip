@@ -58,6 +58,8 @@
 //     launched heaviest first; two workgroups fit on a CU (<= 72 KB LDS,
 //     <= 128 VGPRs), so the short streams' weight streaming runs beside the
 //     long stream's tiles.
+#include <type_traits>
+
 #include "rldx_amd.h"
 #include "rldx_common.h"
 
@@ -81,7 +83,8 @@ enum {
   kEpiBiasPacked = 4,
   kEpiResidualPacked = 5,
   kEpiQkv = 16,   // internal: rldx_grouped_gemm_qkv_norm_rope_bf16, head_dim 128
-  kEpiQkv64 = 17  // the same, head_dim 64 (two heads per 128-column tile)
+  kEpiQkv64 = 17,  // the same, head_dim 64 (two heads per 128-column tile)
+  kEpiLinear1 = 18  // internal: groups of kEpiQkv64 and of kEpiSwigluPacked in one launch (Group::epi)
 };
 constexpr bool qkv_epi(int epi) { return epi == kEpiQkv || epi == kEpiQkv64; }
 constexpr bool packed_out(int epi) {
@@ -211,6 +214,7 @@ struct Group {
   const float* lnstats;
   // residual epilogues: statistics of the output rows [m][n / 64][2], or null
   float* stats_out;
+  int epi;  // this group's epilogue (read by the kEpiLinear1 kernels)
 };
 
 // Outputs of the QKV epilogue: Q (H, M, 128) with strides (q_sh, q_sm), and the
@@ -261,8 +265,9 @@ __device__ __forceinline__ void wait_barrier() {
 // specialization whose body holds the 16-byte LDS-load builtin.  DP: the
 // kernel is a deep-ring instantiation (one workgroup per CU).  TR: the MFMAs
 // take (A chunk, W chunk), so each accumulator holds its block untransposed
-// (the V tiles of the QKV epilogue, whose lanes then hold packed V chunks).
-template <class C, int EPI, bool K, bool LN, bool DP, bool TR = false>
+// (the V tiles of the QKV epilogue, whose lanes then hold packed V chunks).  M:
+// the kernel mixes epilogues (kept apart for the same reason as K).
+template <class C, int EPI, bool K, bool LN, bool DP, bool TR = false, bool M = false>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& a, const Group& G, int item, u32x4* lds, float* wsl) {
   constexpr bool kSwiglu = EPI == kEpiSwiglu || EPI == kEpiSwigluPacked;
   constexpr int MB = C::MB, NB = C::NB, BNW = C::BNW, U = C::U, CH = C::CH, NSLOT = C::NSLOT;
@@ -1291,7 +1296,21 @@ __global__ __launch_bounds__(kThreads, DEEP ? 2 : 4) void gemm_kernel(GemmArgs a
   // splits of a tile) on consecutive workgroups, i.e. on different XCDs
   const int item = a.spread ? r : (r % kXcds) * G.per_xcd + r / kXcds;
   if (item >= G.items) return;
-  if constexpr (WIDE && DEEP) {  // 128-column tiles (whole heads for the QKV epilogue)
+  if constexpr (EPI == kEpiLinear1) {
+    static_assert(WIDE && !LN, "whole 128-column tiles of a group's own epilogue");
+    using T128 = std::conditional_t<DEEP, Cfg128D, Cfg128>;
+    using T64 = std::conditional_t<DEEP, Cfg64x128D, Cfg64x128>;
+    using T32 = std::conditional_t<DEEP, Cfg32x128D, Cfg32x128>;
+    if (G.epi == kEpiQkv64) {
+      if (G.cfg == kTile128) gemm_tile<T128, kEpiQkv64, WIDE, LN, DEEP, false, true>(a, G, item, lds, wsl);
+      else if (G.cfg == kTile64x128) gemm_tile<T64, kEpiQkv64, WIDE, LN, DEEP, false, true>(a, G, item, lds, wsl);
+      else gemm_tile<T32, kEpiQkv64, WIDE, LN, DEEP, false, true>(a, G, item, lds, wsl);
+    } else {
+      if (G.cfg == kTile128) gemm_tile<T128, kEpiSwigluPacked, WIDE, LN, DEEP, false, true>(a, G, item, lds, wsl);
+      else if (G.cfg == kTile64x128) gemm_tile<T64, kEpiSwigluPacked, WIDE, LN, DEEP, false, true>(a, G, item, lds, wsl);
+      else gemm_tile<T32, kEpiSwigluPacked, WIDE, LN, DEEP, false, true>(a, G, item, lds, wsl);
+    }
+  } else if constexpr (WIDE && DEEP) {  // 128-column tiles (whole heads for the QKV epilogue)
     if (G.cfg == kTile128) {
       if constexpr (EPI == kEpiQkv) {
         // V tiles (the last third of [Q | K | V]) with untransposed accumulators
@@ -1602,6 +1621,7 @@ hipError_t launch(const GemmArgs& args, int epilogue, hipStream_t stream, bool w
   switch (epilogue) {
     case kEpiQkv: launch_qkv<kEpiQkv, false>(args, grid, stream, deep); break;
     case kEpiQkv64: launch_qkv<kEpiQkv64, false>(args, grid, stream, deep); break;
+    case kEpiLinear1: launch_qkv<kEpiLinear1, false>(args, grid, stream, deep); break;
     case kEpiBias: launch_epi<kEpiBias, false>(args, grid, stream, deep, wide); break;
     case kEpiResidual: launch_epi<kEpiResidual, false>(args, grid, stream, deep, wide); break;
     case kEpiSwiglu: launch_epi<kEpiSwiglu, false>(args, grid, stream, deep, wide); break;
@@ -1920,11 +1940,13 @@ extern "C" int64_t rldx_grouped_gemm_mixed_workspace_bytes(const rldx_gemm_group
 }
 
 namespace {
-hipError_t gemm_qkv(const rldx_gemm_group_t* groups, const rldx_msat_stream_t* norms, int32_t num_groups,
+// Checks a QKV-epilogue call and fills its launch arguments (num_groups 0: nothing to do).
+hipError_t qkv_plan(const rldx_gemm_group_t* groups, const rldx_msat_stream_t* norms, int32_t num_groups,
                     int64_t heads, int64_t head_dim, int64_t k, void* q_out, int64_t q_head_stride,
                     int64_t q_row_stride, void* kv_packed, int64_t kv_packed_head_stride, float eps,
-                    const float* const* w_row_sums, const float* const* ln_stats, float ln_eps, hipStream_t stream,
-                    const int64_t* group_k = nullptr) {
+                    const float* const* w_row_sums, const float* const* ln_stats, float ln_eps,
+                    const int64_t* group_k, GemmArgs& args) {
+  args = GemmArgs{};
   if (!groups || !norms || num_groups < 1 || num_groups > 3) return hipErrorInvalidValue;
   // 128-column tiles of whole heads: head_dim 128, or 64 with an even head count
   if (!(head_dim == 128 || (head_dim == 64 && heads % 2 == 0)) || heads <= 0 || heads > 4096)
@@ -1951,7 +1973,6 @@ hipError_t gemm_qkv(const rldx_gemm_group_t* groups, const rldx_msat_stream_t* n
   if (m == 0) return hipSuccess;
   if (kv_packed_head_stride < (m + 31) / 32 * 64 * head_dim) return hipErrorInvalidValue;
   if (w_row_sums && !(ln_eps >= 0.f)) return hipErrorInvalidValue;
-  GemmArgs args;
   int64_t ws, co[3], po[3];
   const int epi = head_dim == 128 ? kEpiQkv : kEpiQkv64;
   const int64_t n = 3 * heads * head_dim;
@@ -1962,7 +1983,19 @@ hipError_t gemm_qkv(const rldx_gemm_group_t* groups, const rldx_msat_stream_t* n
   args.qkv = QkvOut{static_cast<uint16_t*>(q_out), static_cast<uint16_t*>(kv_packed), q_head_stride, q_row_stride,
                     kv_packed_head_stride, static_cast<int>(heads * head_dim), eps};
   args.ln_eps = ln_eps;
-  return launch(args, epi, stream, true, w_row_sums != nullptr);
+  return hipSuccess;
+}
+
+hipError_t gemm_qkv(const rldx_gemm_group_t* groups, const rldx_msat_stream_t* norms, int32_t num_groups,
+                    int64_t heads, int64_t head_dim, int64_t k, void* q_out, int64_t q_head_stride,
+                    int64_t q_row_stride, void* kv_packed, int64_t kv_packed_head_stride, float eps,
+                    const float* const* w_row_sums, const float* const* ln_stats, float ln_eps, hipStream_t stream,
+                    const int64_t* group_k = nullptr) {
+  GemmArgs args;
+  const hipError_t e = qkv_plan(groups, norms, num_groups, heads, head_dim, k, q_out, q_head_stride, q_row_stride,
+                                kv_packed, kv_packed_head_stride, eps, w_row_sums, ln_stats, ln_eps, group_k, args);
+  if (e != hipSuccess) return e;
+  return launch(args, head_dim == 128 ? kEpiQkv : kEpiQkv64, stream, true, w_row_sums != nullptr);
 }
 }  // namespace
 
@@ -1996,6 +2029,35 @@ extern "C" hipError_t rldx_grouped_gemm_qkv_norm_rope_ln_bf16(
   if (!w_row_sums || !ln_stats) return hipErrorInvalidValue;
   return gemm_qkv(groups, norms, num_groups, heads, head_dim, k, q_out, q_head_stride, q_row_stride, kv_packed,
                   kv_packed_head_stride, eps, w_row_sums, ln_stats, ln_eps, stream);
+}
+
+// QKV and SwiGLU columns of one A operand in one launch: the two plans, one
+// after the other in the grid.  A single-stream block of 82 rows (24 x 64 heads, K
+// 1536, 12288 MLP columns) ran its QKV GEMM in 9.5 us on 72-144 workgroups, the norm +
+// RoPE kernel after it in 4.9 us and the MLP GEMM in 15.9 us; the launch, its first
+// weight loads and its epilogue are ~4.5 us of each.  Together, the QKV tiles run
+// beside the MLP's: RLDX-1 action head 4.99 -> 4.74 ms per action.
+extern "C" hipError_t rldx_gemm_qkv_swiglu_bf16(const rldx_gemm_group_t* qkv, const rldx_msat_stream_t* norm,
+                                                int64_t heads, int64_t head_dim, void* q_out, int64_t q_head_stride,
+                                                int64_t q_row_stride, void* kv_packed, int64_t kv_packed_head_stride,
+                                                float eps, const rldx_gemm_group_t* mlp, int64_t n_mlp, int64_t k,
+                                                hipStream_t stream) {
+  if (!qkv || !norm || !mlp || qkv->m != mlp->m) return hipErrorInvalidValue;
+  GemmArgs args, tail;
+  const hipError_t e = qkv_plan(qkv, norm, 1, heads, head_dim, k, q_out, q_head_stride, q_row_stride, kv_packed,
+                                kv_packed_head_stride, eps, nullptr, nullptr, 0.f, nullptr, tail);
+  if (e != hipSuccess || head_dim != 64) return e != hipSuccess ? e : hipErrorInvalidValue;
+  int64_t ws, co[3], po[3];
+  const hipError_t em = plan(mlp, 1, n_mlp, k, kEpiSwigluPacked, 1, args, &ws, co, po, nullptr, true);
+  if (em != hipSuccess) return em;
+  if (args.num_groups == 0) return hipSuccess;
+  args.g[0].epi = kEpiSwigluPacked;
+  args.g[1] = tail.g[0];
+  args.g[1].epi = kEpiQkv64;
+  args.g[1].wg_begin = args.g[0].per_xcd * kXcds;
+  args.num_groups = 2;
+  args.qkv = tail.qkv;
+  return launch(args, kEpiLinear1, stream, true);
 }
 
 extern "C" hipError_t rldx_grouped_gemm_ln_bf16(const rldx_gemm_group_t* groups, const float* const* w_row_sums,

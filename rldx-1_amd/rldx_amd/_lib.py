@@ -141,6 +141,8 @@ SIGNATURES = {
     "rldx_grouped_gemm_qkv_norm_rope_ln_bf16": (c_i32, [ctypes.POINTER(GemmGroup), ctypes.POINTER(MsatStream),
                                                         ctypes.POINTER(c_vp), ctypes.POINTER(c_vp), c_i32, c_i64, c_i64,
                                                         c_i64, c_vp, c_i64, c_i64, c_vp, c_i64, c_f32, c_f32, c_vp]),
+    "rldx_gemm_qkv_swiglu_bf16": (c_i32, [ctypes.POINTER(GemmGroup), ctypes.POINTER(MsatStream), c_i64, c_i64, c_vp, c_i64,
+                                          c_i64, c_vp, c_i64, c_f32, ctypes.POINTER(GemmGroup), c_i64, c_i64, c_vp]),
     "rldx_grouped_gemm_stats_bf16": (c_i32, [ctypes.POINTER(GemmGroup), ctypes.POINTER(c_vp), c_i32, c_i64, c_i64,
                                              c_i32, c_i32, c_i32, c_vp, c_i64, c_vp]),
     "rldx_act_pack_stats_bf16": (c_i32, [c_vp, c_i64, c_i64, c_i64, c_vp, c_vp, c_vp]),

@@ -1080,6 +1080,38 @@ def grouped_gemm_qkv_norm_rope(items: Sequence[tuple], norms: Sequence[StreamSpe
     return q, kvp
 
 
+def gemm_qkv_swiglu(a: PackedAct, qkv: tuple, norm: StreamSpec, mlp: tuple, num_heads: int, head_dim: int,
+                    out: tuple, mlp_out: PackedAct, eps: float = 1e-6) -> None:
+    """The two column ranges of a single-stream block's linear1 in one launch
+    (rldx_gemm_qkv_swiglu_bf16, head_dim 64): grouped_gemm_qkv_norm_rope of
+    qkv = (PackedWeight [3 H D, k], bias or None) with the one stream `norm`
+    (its tables cover every row) into out = (q, kvp), and grouped_gemm
+    "swiglu_packed" of mlp = (PackedWeight, bias or None) into mlp_out."""
+    (qw, qb), (mw, mb) = qkv, mlp
+    q, kvp = out
+    m, k = a.m, a.k
+    _on_gpu(a.data, qw.data, mw.data, qb, mb, norm.q_w, norm.k_w, norm.cos, norm.sin, q, kvp, mlp_out.data)
+    _require(a.ld == k and qw.k == k and mw.k == k, "a must be a whole PackedAct [m, k] of the weights' k")
+    _require(head_dim == 64 and num_heads % 2 == 0 and qw.n == 3 * num_heads * head_dim and not qw.swiglu_pairs,
+             "the QKV weight must be [3 H 64, k] with an even head count")
+    _require(mw.swiglu_pairs and mlp_out.m == m and mlp_out.k == mw.n // 2, "mlp: a swiglu_pairs weight, out [m, n / 2]")
+    for b, w in ((qb, qw), (mb, mw)):
+        _require(b is None or (b.dtype == BF16 and b.is_contiguous() and b.numel() == w.n), "bias must be [n] bf16")
+    for t in (norm.q_w, norm.k_w):
+        _require(t.dtype == BF16 and t.numel() == head_dim and t.is_contiguous(), "norm weights must be contiguous bf16 [head_dim]")
+    _require(q.dtype == BF16 and q.shape == (num_heads, m, head_dim) and q.stride(2) == 1, "q out must be (H, M, D)")
+    _check_kvp_out(kvp, num_heads, m, head_dim)
+    keep = []
+    cos_p, sin_p, rope_ld = _rope_tables(norm, m, head_dim, keep)
+    gq = _lib.GemmGroup(a.data.data_ptr(), m, qw.data.data_ptr(), _ptr(qb), None, 0, None, 0)
+    gm = _lib.GemmGroup(a.data.data_ptr(), m, mw.data.data_ptr(), _ptr(mb), mlp_out.data.data_ptr(),
+                        0 if mlp_out.ld == mlp_out.k else mlp_out.ld, None, 0)
+    st = _lib.MsatStream(None, 0, m, norm.q_w.data_ptr(), norm.k_w.data_ptr(), cos_p, sin_p, rope_ld)
+    _lib.check(_lib.load().rldx_gemm_qkv_swiglu_bf16(
+        ctypes.byref(gq), ctypes.byref(st), num_heads, head_dim, q.data_ptr(), q.stride(0), q.stride(1), kvp.data_ptr(),
+        kvp.stride(0), float(eps), ctypes.byref(gm), mw.n, k, _stream_ptr(q)), "rldx_gemm_qkv_swiglu_bf16")
+
+
 # ---------------------------------------------------------------------------
 # Residual-add + norm epilogues (block boundaries)
 # ---------------------------------------------------------------------------

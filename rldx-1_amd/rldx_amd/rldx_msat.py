@@ -285,7 +285,7 @@ class RldxMsat:
 
     # packed weights and RoPE tables: shared by the chains of one model for every batch size
     _WEIGHTS = ("w", "sa_ffn_p", "vl_ffn_p", "ds", "ss", "vl_proj_to_sa", "proj_out_2", "proj_out_physics_2",
-                "ds_cos", "ds_sin", "ss_cos", "ss_sin", "p_cos", "p_sin")
+                "ds_cos", "ds_sin", "ss_cos", "ss_sin", "x_cos", "x_sin", "p_cos", "p_sin")
 
     def __init__(self, sd: Optional[dict], cfg: RldxMsatCfg, device, bf16_quirk: bool = True, vl_mask: bool = False,
                  batch: int = 1, weights_of: Optional["RldxMsat"] = None):
@@ -397,6 +397,9 @@ class RldxMsat:
 
         self.ds_cos, self.ds_sin = tables(ds_pos, rows=self.ns)
         self.ss_cos, self.ss_sin = tables(ss_pos, rows=self.ns)
+        # the single-stream tables over [VL | time | SA]: VL rows are not rotated
+        one, zero = torch.ones(self.nv, D // 2, device=self.dev), torch.zeros(self.nv, D // 2, device=self.dev)
+        self.x_cos, self.x_sin = torch.cat([one, self.ss_cos]), torch.cat([zero, self.ss_sin])
         if self.phys:
             self.p_cos, self.p_sin = tables(torch.arange(self.np_), axis0=1)
         self.proj_out_physics_2 = Fn.pack_weight(w["proj_out_physics_2.weight"]) if self.phys else None
@@ -464,6 +467,8 @@ class RldxMsat:
         self._ninf = torch.full((), float("-inf"), dtype=torch.float32, device=self.dev)
         self._zero = torch.zeros((), dtype=torch.float32, device=self.dev)
         self.graph = None
+        # one robot without a P stream: the rows of x are the joint sequence, so linear1 is one launch
+        self.fused_linear1 = B == 1 and not self.phys and D == 64 and H % 2 == 0
         # the pre-norms of a block's streams, one launch each time
         self.ds_norms = [(self.x_sa, self.h_sa), (self.x_vl, self.h_vl)] + ([(self.x_p, self.h_p)] if self.phys else [])
         self.ss_norms = [(self.x, self.h)] + ([(self.x_p, self.h_p)] if self.phys else [])
@@ -634,8 +639,15 @@ class RldxMsat:
 
     def _ss_block(self, blk: dict, gm: dict) -> None:
         cfg = self.cfg
-        B, nv, ns, inner = self.batch, self.nv, cfg.n_sa, cfg.inner
+        B, nv, ns = self.batch, self.nv, cfg.n_sa
         Fn.layernorm_pack_many(self.ss_norms, cfg.eps)
+        if self.fused_linear1:
+            Fn.gemm_qkv_swiglu(self.h, (blk["qkv"], blk["qkv.bias"]),
+                               Fn.StreamSpec(None, blk["q_norm"], blk["k_norm"], self.x_cos, self.x_sin),
+                               (blk["mlp"], blk["mlp.bias"]), cfg.heads, cfg.head_dim, (self.q[0], self.kvp[0]), self.gl,
+                               cfg.eps)
+            self._ss_tail(gm)
+            return
         self._gemm(gm["qkv"])
         self._gemm(gm["mlp"])
         streams = [(self.qkv_buf, nv, nv, blk["q_norm"], blk["k_norm"], None, None),
@@ -643,7 +655,11 @@ class RldxMsat:
         if self.phys:
             streams.append((self.qkv_p, self.np_, self.np_, blk["p_q_norm"], blk["p_k_norm"], self.p_cos, self.p_sin))
         self._qkv_norm_rope(streams)
-        Fn.attention_packed(self.q, self.kvp, self.N, key_bias=self._kb(), out=self.cat.cols(0, inner),
+        self._ss_tail(gm)
+
+    def _ss_tail(self, gm: dict) -> None:
+        """Attention -> columns [0, inner) of the linear2 operand, mlp_proj -> the others, linear2 + residual."""
+        Fn.attention_packed(self.q, self.kvp, self.N, key_bias=self._kb(), out=self.cat.cols(0, self.cfg.inner),
                             segments=self.segments)
         self._gemm(gm["mlp_proj"])
         self._gemm(gm["linear2"])

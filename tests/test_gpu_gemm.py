@@ -867,3 +867,48 @@ def test_grouped_gemm_qkv_norm_rope_layernorm_fold(dev, ms, H, k):
     assert torch.equal(q.view(torch.int16), q2.view(torch.int16))
     assert torch.equal(kvp.view(torch.int16), kvp2.view(torch.int16))
     assert_bf16_close(q, q3, "QKV epilogue with the LayerNorm fold vs LayerNorm-pack + QKV epilogue")
+
+
+@pytest.mark.parametrize("m,heads,k,n_mlp", [(82, 24, 1536, 12288), (18, 2, 256, 192), (33, 4, 384, 64), (64, 2, 128, 128),
+                                             (300, 16, 256, 8320), (130, 6, 256, 320)])
+def test_gemm_qkv_swiglu_matches_two_launches(dev, m, heads, k, n_mlp):
+    """linear1 of a single-stream block in one launch: the bits of the QKV GEMM with
+    its norm epilogue and of the SwiGLU GEMM (every tile shape, ragged rows, a
+    partial last column tile)."""
+    g = torch.Generator().manual_seed(m + n_mlp)
+    rnd = lambda *s, std=1.0: (std * torch.randn(*s, generator=g)).to(torch.bfloat16).to(dev)  # noqa: E731
+    D = 64
+    a = Fn.pack_act(rnd(m, k))
+    qw, mw = Fn.pack_weight(rnd(3 * heads * D, k, std=k ** -0.5)), Fn.pack_weight(rnd(n_mlp, k, std=k ** -0.5), True)
+    qb, mb = rnd(3 * heads * D), rnd(n_mlp)
+    cos, sin = (torch.randn(m, D // 2, generator=g).to(dev) for _ in range(2))
+    norm = Fn.StreamSpec(None, 1 + 0.1 * rnd(D), 1 + 0.1 * rnd(D), cos, sin)
+    for biases in ((qb, mb), (None, None)):
+        q, kvp = (torch.empty(heads, m, D, dtype=torch.bfloat16, device=dev),
+                  torch.full((heads, Fn.kv_packed_elems(m, D)), 9.0, dtype=torch.bfloat16, device=dev))
+        wide = Fn.PackedAct.empty(m, n_mlp // 2 + 32, dev)
+        wide.data.fill_(7.0)
+        Fn.gemm_qkv_swiglu(a, (qw, biases[0]), norm, (mw, biases[1]), heads, D, (q, kvp), wide.cols(32, n_mlp // 2 + 32))
+        rq, rkvp = Fn.grouped_gemm_qkv_norm_rope([(a, qw, biases[0])], [norm], heads, D)
+        ref_out = Fn.PackedAct.empty(m, n_mlp // 2, dev)
+        Fn.grouped_gemm([(a, mw, biases[1], ref_out, None)], "swiglu_packed")
+        assert torch.equal(q, rq) and torch.equal(kvp, rkvp)
+        got = wide.unpack()
+        assert torch.equal(got[:, 32:], ref_out.unpack()) and (got[:, :32] == 7.0).all()
+
+
+def test_gemm_qkv_swiglu_rejections(dev):
+    a = Fn.PackedAct.empty(64, 128, dev)
+    w = Fn.pack_weight(torch.zeros(384, 128, dtype=torch.bfloat16, device=dev))
+    mw = Fn.pack_weight(torch.zeros(128, 128, dtype=torch.bfloat16, device=dev), True)
+    nw = torch.ones(64, dtype=torch.bfloat16, device=dev)
+    q = torch.empty(2, 64, 64, dtype=torch.bfloat16, device=dev)
+    kvp = torch.empty(2, Fn.kv_packed_elems(64, 64), dtype=torch.bfloat16, device=dev)
+    out = Fn.PackedAct.empty(64, 64, dev)
+    norm = Fn.StreamSpec(None, nw, nw)
+    for args in ((a, (mw, None), norm, (mw, None), 2, 64, (q, kvp), out), (a, (w, None), norm, (w, None), 2, 64, (q, kvp), out),
+                 (a, (w, None), norm, (mw, None), 1, 128, (q, kvp), out), (a, (w, None), norm, (mw, None), 2, 64, (q, kvp[:, 1:]), out),
+                 (a, (w, None), norm, (mw, None), 2, 64, (q[:, 1:], kvp), out),
+                 (a, (w, None), norm, (mw, None), 2, 64, (q, kvp), Fn.PackedAct.empty(64, 128, dev))):
+        with pytest.raises(RuntimeError):
+            Fn.gemm_qkv_swiglu(*args)
