@@ -1350,6 +1350,162 @@ __global__ __launch_bounds__(kThreads, DEEP ? 2 : 4) void gemm_kernel(GemmArgs a
   }
 }
 
+// ---------------------------------------------------------------------------
+// One long stream with tiles enough for whole rounds over the chip: 256 x 256
+// tiles, 8 waves of 64 x 128 (4 x 2), one workgroup per CU.  A 128 x 128 tile loads
+// 8 KB per k-step for 16 MFMAs (64 B per MFMA clock of the CU, more than the ~48 B/clk
+// it gets from L2, which bounds it); this one 16 KB for 64 (32 B/clk), and its
+// waves read 6 KB of LDS for 8 MFMAs instead of 3 for 2.  The sums run over K in
+// the same order: the same bits.  Measured on MI355X (SwiGLU, us, 128 x 128 / 256
+// x 256): 2048 x 22016 x 4096 403 / 315 (1172 TFLOP/s), 1024 x 22016 x 4096 227 / 192,
+// 2048 x 8192 x 1536 59.2 / 50.0; bias 4096^3 160 / 108 (1271 TFLOP/s).
+// ---------------------------------------------------------------------------
+constexpr int kBigMB = 8, kBigNB = 8, kBigSlots = 4;
+constexpr int kBigChunks = 2 * (kBigMB + kBigNB);  // 1 KB chunks of a stage (two k-steps)
+
+template <int EPI>
+__global__ __launch_bounds__(kThreads, 2) void gemm_big_kernel(GemmArgs a) {
+  constexpr bool kSwiglu = EPI == kEpiSwiglu || EPI == kEpiSwigluPacked;
+  constexpr int MW = 2, NW = 4;  // m- and n-blocks per wave
+  constexpr int ND = kBigChunks / 8;
+  __shared__ __attribute__((aligned(16))) u32x4 ring[kBigSlots * kBigChunks * 64];
+  const Group& G = a.g[0];
+  const int b = static_cast<int>(blockIdx.x);
+  const int item = (b % kXcds) * G.per_xcd + b / kXcds;
+  if (item >= G.items) return;
+  const int lane = threadIdx.x & 63, l32 = lane & 31, g = lane >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int wm = wv >> 1, wn = wv & 1;
+  const int mt = item % G.m_tiles, nt = item / G.m_tiles;
+  const int ksteps = G.k / 16, stages = ksteps / 2;
+  const int mblocks = (G.m + 31) / 32, nblocks = G.n / 32;
+
+  // the chunks this wave loads per stage: q = wv + 8 j, k-step q / 16, chunk q % 16
+  // (m-blocks, then n-blocks; blocks past the edge re-read the last one)
+  __amdgpu_buffer_rsrc_t rs[ND];
+  int qoff[ND];
+#pragma unroll
+  for (int j = 0; j < ND; ++j) {
+    const int q = wv + 8 * j, u = q / 16, c = q % 16;
+    const bool act = c < kBigMB;
+    rs[j] = act ? rsrc(G.a, mblocks * ksteps * 1024) : rsrc(G.w, nblocks * ksteps * 1024);
+    const int blk = act ? min(mt * kBigMB + c, mblocks - 1) : min(nt * kBigNB + c - kBigMB, nblocks - 1);
+    qoff[j] = (blk * ksteps + u) * 1024;
+  }
+  auto dma = [&](int st, int slot) {
+    const int ks = min(st, stages - 1) * 2048;
+#pragma unroll
+    for (int j = 0; j < ND; ++j)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rs[j], (__attribute__((address_space(3))) void*)(ring + (slot * kBigChunks + wv + 8 * j) * 64), 16, lane * 16,
+          qoff[j] + ks, 0, 0);
+  };
+  u32x4 xa[2][MW], xw[2][NW];  // operands of the two k-steps of a stage
+  auto lread = [&](int u, int slot) {
+    const u32x4* s = ring + (slot * kBigChunks + u * 16) * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < MW; ++i) xa[u][i] = s[(wm * MW + i) * 64];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) xw[u][i] = s[(kBigMB + wn * NW + i) * 64];
+  };
+  floatx16 acc[MW][NW];
+#pragma unroll
+  for (int i = 0; i < MW; ++i)
+#pragma unroll
+    for (int j = 0; j < NW; ++j) acc[i][j] = floatx16{};
+  auto mma = [&](int u) {
+#pragma unroll
+    for (int j = 0; j < NW; ++j)
+#pragma unroll
+      for (int i = 0; i < MW; ++i)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xw[u][j]),
+                                                            __builtin_bit_cast(bf16x8, xa[u][i]), acc[i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int s = 0; s < kBigSlots - 1; ++s) dma(s, s);
+  wait_barrier<(kBigSlots - 2) * ND>();
+  lread(0, 0);
+  for (int st = 0; st < stages; ++st) {
+    const int slot = st & (kBigSlots - 1);
+    dma(st + kBigSlots - 1, (st + kBigSlots - 1) & (kBigSlots - 1));  // past the last stage: re-loads it into a free slot
+    __builtin_amdgcn_sched_barrier(0);
+    lread(1, slot);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(0);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_barrier<(kBigSlots - 2) * ND>();  // stage st + 1 is in LDS
+    __builtin_amdgcn_sched_barrier(0);
+    lread(0, (slot + 1) & (kBigSlots - 1));  // past the last stage: read, never used
+    __builtin_amdgcn_sched_barrier(0);
+    mma(1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  // Epilogue in registers: lane (l32, g) holds rows 32 (2 wm + i) + l32 of the tile
+  // and columns 8 q4 + 4 g + c of its n-blocks.  Lanes l and l + 32 swap halves of
+  // their 8-column chunks, so that lane half g stores chunk 2 pp + g whole.
+  const int n_out = kSwiglu ? G.n / 2 : G.n;
+  auto bias4 = [&](int col, float (&v)[4]) {  // (the launcher checks an 8-byte aligned bias)
+    const uint2 raw = G.bias ? *reinterpret_cast<const uint2*>(G.bias + col) : uint2{0, 0};
+    v[0] = bf16x2_lo(raw.x);
+    v[1] = bf16x2_hi(raw.x);
+    v[2] = bf16x2_lo(raw.y);
+    v[3] = bf16x2_hi(raw.y);
+  };
+  constexpr int NB_OUT = kSwiglu ? NW / 2 : NW;
+#pragma unroll
+  for (int j = 0; j < NB_OUT; ++j) {
+    const int c0 = (kSwiglu ? nt * (16 * kBigNB) + 64 * wn : nt * (32 * kBigNB) + 128 * wn) + 32 * j;  // the block's first output column
+    if (c0 >= n_out) break;
+    float b0[4][4], b1[4][4];
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      bias4(c0 + 8 * q4 + 4 * g, b0[q4]);
+      if constexpr (kSwiglu) bias4(n_out + c0 + 8 * q4 + 4 * g, b1[q4]);
+    }
+#pragma unroll
+    for (int i = 0; i < MW; ++i) {
+      uint32_t od[4][2];
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4)
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const int e = 4 * q4 + 2 * p;
+          if constexpr (kSwiglu) {
+            const uint32_t gp = pack_bf16x2(acc[i][2 * j][e] + b0[q4][2 * p], acc[i][2 * j][e + 1] + b0[q4][2 * p + 1]);
+            const uint32_t up =
+                pack_bf16x2(acc[i][2 * j + 1][e] + b1[q4][2 * p], acc[i][2 * j + 1][e + 1] + b1[q4][2 * p + 1]);
+            od[q4][p] = swiglu_bf16x2(bf16x2_lo(gp), bf16x2_hi(gp), bf16x2_lo(up), bf16x2_hi(up));
+          } else {
+            od[q4][p] = pack_bf16x2(acc[i][j][e] + b0[q4][2 * p], acc[i][j][e + 1] + b0[q4][2 * p + 1]);
+          }
+        }
+      const int row = (mt * kBigMB + wm * MW + i) * 32 + l32;
+#pragma unroll
+      for (int pp = 0; pp < 2; ++pp) {
+        const uint32_t w0 = g == 0 ? od[2 * pp + 1][0] : od[2 * pp][0];
+        const uint32_t w1 = g == 0 ? od[2 * pp + 1][1] : od[2 * pp][1];
+        const uint32_t x0 = static_cast<uint32_t>(__shfl_xor(static_cast<int>(w0), 32, 64));
+        const uint32_t x1 = static_cast<uint32_t>(__shfl_xor(static_cast<int>(w1), 32, 64));
+        u32x4 o = g == 0 ? u32x4{od[2 * pp][0], od[2 * pp][1], x0, x1} : u32x4{x0, x1, od[2 * pp + 1][0], od[2 * pp + 1][1]};
+        const int col = c0 + 8 * (2 * pp + g);
+        if (row < G.m) {
+          if constexpr (residual_epi(EPI)) {
+            const u32x4 r = *reinterpret_cast<const u32x4*>(
+                G.res + (EPI == kEpiResidualPacked ? packed_act_offset(row, col, G.ldr) : static_cast<int64_t>(row) * G.ldr + col));
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              o[e] = pack_bf16x2(bf16x2_lo(r[e]) + bf16x2_lo(o[e]), bf16x2_hi(r[e]) + bf16x2_hi(o[e]));
+          }
+          *reinterpret_cast<u32x4*>(G.out + (packed_out(EPI) ? packed_act_offset(row, col, G.ldo)
+                                                             : static_cast<int64_t>(row) * G.ldo + col)) = o;
+        }
+      }
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the ring's re-loads write LDS)
+}
+
 bool a16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 template <class C>
@@ -1596,6 +1752,38 @@ void launch_qkv(const GemmArgs& args, dim3 grid, hipStream_t stream, bool deep) 
     hipLaunchKernelGGL((gemm_kernel<EPI, false, true, LN>), grid, dim3(kThreads), 0, stream, args);
 }
 
+// Whether a launch takes the 256 x 256 tiles.  They run in whole rounds of 256
+// workgroups, each round as long as 1.4 rounds of 512 of the 128 x 128 tiles, whose
+// last round is shared by two workgroups per CU: a round of theirs counts 0.70, and
+// 0.15 for its end.  Measured at the line (us, 128 x 128 / 256 x 256): 1500 x 22016 x
+// 4096 294 / 281 (3 against 2.97), 2048 x 12288 x 1536 86.5 / 83.8 (2 against 2.25), 2048
+// x 4096 x 8192 133 / 149 (1 against 0.85).
+bool big_tiles(const GemmArgs& args, int epilogue, bool ln) {
+  const Group& G = args.g[0];
+  if (args.num_groups != 1 || ln || G.splits > 1 || G.stats_out || epilogue < kEpiBias || epilogue > kEpiResidualPacked)
+    return false;
+  if (G.cfg != kTile128 || reinterpret_cast<uintptr_t>(G.bias) % 8) return false;
+  const int64_t big = static_cast<int64_t>((G.m + 255) / 256) * ((G.n + 255) / 256);
+  return (big + 255) / 256 * 100 <= static_cast<int64_t>(G.items) * 70 / 512 + 15;  // (items: the 128 x 128 tiles)
+}
+
+hipError_t launch_big(GemmArgs args, int epilogue, hipStream_t stream) {
+  Group& G = args.g[0];
+  G.m_tiles = (G.m + 32 * kBigMB - 1) / (32 * kBigMB);
+  G.items = G.m_tiles * ((G.n + 32 * kBigNB - 1) / (32 * kBigNB));
+  G.per_xcd = (G.items + kXcds - 1) / kXcds;
+  const dim3 grid(static_cast<unsigned>(G.per_xcd * kXcds)), block(kThreads);
+  switch (epilogue) {
+    case kEpiBias: hipLaunchKernelGGL(gemm_big_kernel<kEpiBias>, grid, block, 0, stream, args); break;
+    case kEpiResidual: hipLaunchKernelGGL(gemm_big_kernel<kEpiResidual>, grid, block, 0, stream, args); break;
+    case kEpiSwiglu: hipLaunchKernelGGL(gemm_big_kernel<kEpiSwiglu>, grid, block, 0, stream, args); break;
+    case kEpiSwigluPacked: hipLaunchKernelGGL(gemm_big_kernel<kEpiSwigluPacked>, grid, block, 0, stream, args); break;
+    case kEpiBiasPacked: hipLaunchKernelGGL(gemm_big_kernel<kEpiBiasPacked>, grid, block, 0, stream, args); break;
+    default: hipLaunchKernelGGL(gemm_big_kernel<kEpiResidualPacked>, grid, block, 0, stream, args); break;
+  }
+  return hipGetLastError();
+}
+
 // ln: the groups carry W row sums (LayerNorm fold; plan() admits it for the
 // bias, packed-SwiGLU and QKV epilogues only)
 hipError_t launch(const GemmArgs& args, int epilogue, hipStream_t stream, bool wide = false, bool ln = false) {
@@ -1605,6 +1793,7 @@ hipError_t launch(const GemmArgs& args, int epilogue, hipStream_t stream, bool w
   const dim3 grid(static_cast<unsigned>(wgs));
   // at most one workgroup per CU (256 CUs): the deep-ring kernel
   const bool deep = wgs <= 256;
+  if (big_tiles(args, epilogue, ln)) return launch_big(args, epilogue, stream);
   if (ln) {
     if (epilogue == kEpiQkv)
       launch_qkv<kEpiQkv, true>(args, grid, stream, deep);

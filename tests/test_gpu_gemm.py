@@ -912,3 +912,38 @@ def test_gemm_qkv_swiglu_rejections(dev):
                  (a, (w, None), norm, (mw, None), 2, 64, (q, kvp), Fn.PackedAct.empty(64, 128, dev))):
         with pytest.raises(RuntimeError):
             Fn.gemm_qkv_swiglu(*args)
+
+
+@pytest.mark.parametrize("m,n,k", [(700, 21696, 128), (2039, 8128, 384), (2048, 8192, 256)])
+@pytest.mark.parametrize("epilogue", ["bias", "residual", "swiglu", "swiglu_packed", "bias_packed", "residual_packed"])
+def test_gemm_256_tiles_bit_identical(dev, m, n, k, epilogue):
+    """One long stream (256 x 256 tiles; ragged rows, a partial last column tile, one
+    ring's worth of K and more) gives the bits of its 256-row parts (128 x 128 tiles)."""
+    g = torch.Generator(device=dev).manual_seed(m + n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)  # noqa: E731
+    swiglu, packed = "swiglu" in epilogue, "packed" in epilogue
+    n_out = n // 2 if swiglu else n
+    a, w = Fn.pack_act(rnd(m, k)), Fn.pack_weight((rnd(n, k).float() * k ** -0.5).to(torch.bfloat16), swiglu)
+    res = rnd(m, n_out) if "residual" in epilogue else None
+    res_packed = rnd((m + 31) // 32 * 32 * n_out)
+    for bias in (rnd(n), None):
+        def run(step):
+            if packed:  # columns 16 .. of a wider packed matrix
+                out = Fn.PackedAct.empty(m, n_out + 16, dev)
+                out.data.fill_(3.0)
+                rp = None if res is None else Fn.PackedAct(res_packed, m, n_out)
+            else:
+                out = torch.full((m, n_out + 8), 3.0, dtype=torch.bfloat16, device=dev)
+                rp = res
+            for r0 in range(0, m, step):
+                r0, r1 = min(r0, max(0, (m - step) // 32 * 32)), min(m, r0 + step)  # (at least `step` rows each)
+                if packed:
+                    o = Fn.PackedAct(out.rows(r0, r1).data[512:], r1 - r0, n_out, n_out + 16)
+                    r = None if rp is None else rp.rows(r0, r1)
+                else:
+                    o, r = out[r0:r1, :n_out], None if rp is None else rp[r0:r1]
+                Fn.grouped_gemm([(a.rows(r0, r1), w, bias, o, r)], epilogue)
+            return out.unpack() if packed else out
+
+        whole, parts = run(m), run(256)
+        assert torch.equal(whole, parts), epilogue
