@@ -232,6 +232,7 @@ struct GemmArgs {
   int num_groups;
   int n, k;  // the first group's n, k (every group's with a uniform call); n = rows of W (2 N_half with SwiGLU)
   QkvOut qkv;
+  int wide;      // != 0: the plan took 128-column tiles by itself (see plan)
   int spread;    // != 0: the splits of a tile on different XCDs (RLDX_GEMM_SPLITS_ACROSS_XCDS)
   float ln_eps;  // LayerNorm fold (kernels instantiated with LN)
 };
@@ -1637,14 +1638,24 @@ hipError_t plan(const rldx_gemm_group_t* groups, int32_t num_groups, int64_t n, 
     // same sums, bit for bit).
     int mt, nt, cfg, kg;
     tiles_of<Cfg128>(s.m, n, mt, nt);
-    if (s.m >= 256 && static_cast<int64_t>(mt) * nt >= 128) {
+    // One SwiGLU group on its own (no other stream to run beside it), measured on
+    // MI355X (us, 64 x 64 / 64 x 128 / 128 x 128): 128 x 128 from 160 tiles also below
+    // 256 rows (82 x 22016 x 4096 59.1 / 59.4 / 46.6 at 172 tiles, 200 x 12288 x 1536
+    // 20.7 / 19.9 / 17.8 at 192; 200 x 8192 x 1536 15.1 / 13.8 / 17.2 at 128); else 64 x
+    // 128 (32 x 128) where 64 x 64 (32 x 64) needs more than one workgroup per CU and
+    // it does not (82 x 12288 x 1536 14.6 / 12.7 / 15.9; 18 x 22016 x 4096 44.1 / 40.9; but 82 x
+    // 8192 x 1536, 256 workgroups, 10.4 / 12.4 / 15.8).
+    const bool alone = swiglu && num_groups == 1 && split_k <= 1 && !group_splits && !w_row_sums;
+    const int64_t m64 = (s.m + 63) / 64;
+    const bool wide1 = alone && m64 * (n / 64) > 256 && m64 * ((n + 127) / 128) <= 256;
+    if (static_cast<int64_t>(mt) * nt >= (s.m >= 256 ? 128 : 160) && (s.m >= 256 || (alone && s.m > 64))) {
       cfg = kTile128;
       kg = Cfg128::KG;
-    } else if (wide && s.m > 32) {
+    } else if ((wide || wide1) && s.m > 32) {
       cfg = kTile64x128;
       kg = Cfg64x128::KG;
       tiles_of<Cfg64x128>(s.m, n, mt, nt);
-    } else if (wide) {
+    } else if (wide || wide1) {
       cfg = kTile32x128;
       kg = Cfg32x128::KG;
       tiles_of<Cfg32x128>(s.m, n, mt, nt);
@@ -1657,6 +1668,7 @@ hipError_t plan(const rldx_gemm_group_t* groups, int32_t num_groups, int64_t n, 
       kg = Cfg32::KG;
       tiles_of<Cfg32>(s.m, n, mt, nt);
     }
+    if (cfg == kTile64x128 || cfg == kTile32x128) args.wide = 1;
     const int64_t tiles = static_cast<int64_t>(mt) * nt;
     if (tiles > (int64_t{1} << 24)) return hipErrorInvalidValue;
     const int lstages = ksteps / (2 * kg);
@@ -1793,6 +1805,7 @@ hipError_t launch(const GemmArgs& args, int epilogue, hipStream_t stream, bool w
   const dim3 grid(static_cast<unsigned>(wgs));
   // at most one workgroup per CU (256 CUs): the deep-ring kernel
   const bool deep = wgs <= 256;
+  wide = wide || args.wide;
   if (big_tiles(args, epilogue, ln)) return launch_big(args, epilogue, stream);
   if (ln) {
     if (epilogue == kEpiQkv)

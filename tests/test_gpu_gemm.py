@@ -947,3 +947,30 @@ def test_gemm_256_tiles_bit_identical(dev, m, n, k, epilogue):
 
         whole, parts = run(m), run(256)
         assert torch.equal(whole, parts), epilogue
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 20480, 128), (82, 20416, 256), (255, 10240, 128),   # 128 x 128 tiles below 256 rows
+                                   (64, 16448, 128), (82, 12288, 256), (129, 8128, 128), (200, 8192, 128),  # 64 x 128
+                                   (18, 16448, 128), (32, 20544, 256)])                      # 32 x 128
+@pytest.mark.parametrize("packed", [False, True])
+def test_gemm_swiglu_alone_tiles(dev, m, n, k, packed):
+    """The tile shapes of a SwiGLU group on its own, ragged in rows and columns, against fp32 products and the
+    oracle's rounding chain; the 64- and 32-row tiles keep the sums of the other plan (the same call as one of
+    two groups), bit for bit."""
+    g = torch.Generator(device=dev).manual_seed(m + n)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)  # noqa: E731
+    # gate and up have std 0.5 (5 sigma over the 2 M values: 2.5): outputs stay below 4, where one bf16 ulp is
+    # 0.0156, inside the max-abs bound for a sum that rounds the other way
+    x, w, b = rnd(m, k), (0.4 * rnd(n, k).float() * k ** -0.5).to(torch.bfloat16), 0.3 * rnd(n)
+    a, pw = Fn.pack_act(x), Fn.pack_weight(w, True)
+    new = lambda: (Fn.PackedAct.empty(m, n // 2, dev) if packed  # noqa: E731
+                   else torch.empty(m, n // 2, dtype=torch.bfloat16, device=dev))
+    rows = lambda t: t.unpack() if packed else t  # noqa: E731
+    epi = "swiglu_packed" if packed else "swiglu"
+    out, two, other = new(), new(), new()
+    Fn.grouped_gemm([(a, pw, b, out, None)], epi)
+    y = (x.float() @ w.float().t() + b.float()).to(torch.bfloat16)
+    assert_bf16_close(rows(out), ref.swiglu(y.cpu()), f"SwiGLU GEMM {m} x {n} x {k}")
+    Fn.grouped_gemm([(a, pw, b, two, None), (a, pw, b, other, None)], epi)
+    if -(-m // 128) * -(-n // 128) < 160 or m <= 64:
+        assert torch.equal(rows(out), rows(two))
