@@ -1523,13 +1523,21 @@ constexpr int vit_padded_dim(int64_t hd) {
 //   64.1 / 64.1 at 288), below that NG = 2 where it makes one round of two
 //   workgroups per CU (1600: 42.3 / 40.8 / 35.9 at 400; joint 16 x 2144: 61.5 / 62.4 /
 //   71.7 at 544, 16 x 1120: 25.4 / 28.3 / 25.8 at 288).
-int shared_groups(bool causal, int64_t heads, int64_t b64, int64_t b128) {
+// head_dim 64 (half the matrix work per exponential: the old kernel and NG = 2 are
+// closer, NG = 1 is last until launches are very large), attention only / ViT:
+//   causal 32/8 x 800 10.2 / 15.2 / 10.6 at 448, x 1024 14.8 / 18.7 / 12.5 at 544; 16/8 x
+//   2048 18.6 / 31.2 / 19.6 at 528, x 2560 24.7 / 37.9 / 24.7 at 656; 32/8 x 4096 104 / 88 /
+//   86, x 6144 213 / 168 / 179 (NG = 1: 1056, 1568);
+//   not causal 1204 + 424 + 897 + 79 36.4 / 39.6 / 32.2 at 704 workgroups, 2304 + 196 + 79
+//   47.6 / 57.8 / 47.4 at 688, joint 24 x 1632 30.2 / 36.9 / 31.0 at 624.
+int shared_groups(bool causal, int64_t head_dim, int64_t heads, int64_t b64, int64_t b128) {
+  const bool narrow = head_dim <= 64;
   if (causal) {
-    if (heads * (b128 + 1) >= 540) return 1;
-    return heads * (b64 + 1) >= (b64 <= 20 ? 440 : 528) ? 2 : 0;
+    if (heads * (b128 + 1) >= (narrow ? 1200 : 540)) return 1;
+    return heads * (b64 + 1) >= (b64 <= 20 ? (narrow ? 530 : 440) : (narrow ? 650 : 528)) ? 2 : 0;
   }
-  if (heads * b128 >= 380) return 1;
-  return heads * b64 >= 400 && heads * b64 <= 512 ? 2 : 0;
+  if (!narrow && heads * b128 >= 380) return 1;
+  return (heads * b64 >= 400 && heads * b64 <= 512) || (narrow && heads * b64 >= 680) ? 2 : 0;
 }
 
 template <int DP>
@@ -1537,18 +1545,23 @@ hipError_t launch_vit(const VitArgs& v, AttnArgs a, int64_t slots, hipStream_t s
   hipLaunchKernelGGL(vit_pack_kernel<DP>, dim3(static_cast<unsigned>(slots), static_cast<unsigned>(v.heads)),
                      dim3(256), 0, stream, v);
   const int64_t b64 = seq_slot_count(v.rows, v.num_seqs, 64), b128 = seq_slot_count(v.rows, v.num_seqs, 128);
-  const int groups = shared_groups(false, v.heads, b64, b128);
+  const int groups = shared_groups(false, DP, v.heads, b64, b128);
   if (groups > 0) {
     a.num_q_blocks = static_cast<int>(groups == 1 ? b128 : b64);
     a.n_work = a.num_q_blocks * v.heads;
     const dim3 grid(static_cast<unsigned>(a.n_work));
     constexpr int KS = DP / 16, KSN = DP == 96 ? 5 : KS;  // head_dim <= 80: the sixth 16-column step is all padding
     const bool narrow = DP == 96 && v.hd <= 80;
-    if (groups == 1 && narrow)
-      hipLaunchKernelGGL((attn_shared_kernel<DP, KSN, 1, false, false, false, true>), grid, dim3(256), 0, stream, a);
-    else if (groups == 1)
-      hipLaunchKernelGGL((attn_shared_kernel<DP, KS, 1, false, false, false, true>), grid, dim3(256), 0, stream, a);
-    else if (narrow)
+    if constexpr (DP > 64) {
+      if (groups == 1) {
+        if (narrow)
+          hipLaunchKernelGGL((attn_shared_kernel<DP, KSN, 1, false, false, false, true>), grid, dim3(256), 0, stream, a);
+        else
+          hipLaunchKernelGGL((attn_shared_kernel<DP, KS, 1, false, false, false, true>), grid, dim3(256), 0, stream, a);
+        return hipGetLastError();
+      }
+    }
+    if (narrow)
       hipLaunchKernelGGL((attn_shared_kernel<DP, KSN, 2, false, false, false, true>), grid, dim3(256), 0, stream, a);
     else
       hipLaunchKernelGGL((attn_shared_kernel<DP, KS, 2, false, false, false, true>), grid, dim3(256), 0, stream, a);
@@ -1576,7 +1589,7 @@ void launch_shared(const AttnArgs& a, bool has_bias, dim3 grid, hipStream_t stre
 template <int D, int NSUB, bool kQNorm>
 void launch_attn_d(AttnArgs a, int batch, bool causal, bool has_bias, hipStream_t stream) {
   const int64_t heads = static_cast<int64_t>(a.hq) * batch, b64 = (a.sq + 63) / 64, b128 = (a.sq + 127) / 128;
-  const int groups = shared_groups(causal, heads, b64, b128);
+  const int groups = shared_groups(causal, D, heads, b64, b128);
   if (groups > 0) a.num_q_blocks = static_cast<int>(groups == 1 ? b128 : b64);
   a.n_work = a.num_q_blocks * a.hq * batch;
   if (groups > 0 && causal) {
@@ -1598,8 +1611,10 @@ void launch_attn_d(AttnArgs a, int batch, bool causal, bool has_bias, hipStream_
     if (causal && groups == 1) launch_shared<D, 1, true, kQNorm>(a, has_bias, grid, stream);
     else if (causal) launch_shared<D, 2, true, kQNorm>(a, has_bias, grid, stream);
     if constexpr (!kQNorm) {
-      if (!causal && groups == 1) launch_shared<D, 1, false, false>(a, has_bias, grid, stream);
-      else if (!causal) launch_shared<D, 2, false, false>(a, has_bias, grid, stream);
+      if constexpr (D > 64) {
+        if (!causal && groups == 1) launch_shared<D, 1, false, false>(a, has_bias, grid, stream);
+      }
+      if (!causal && groups == 2) launch_shared<D, 2, false, false>(a, has_bias, grid, stream);
     }
     return;
   }

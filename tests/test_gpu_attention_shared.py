@@ -34,12 +34,13 @@ def _inputs(B, Hq, Hkv, Sq, Sk, D, bias):
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal,bias", [
     # 128 queries per workgroup
     (1, 128, 16, 417, 417, 128, True, False),
-    (1, 135, 135, 417, 417, 64, True, False),    # heads not divisible over the XCDs
+    (1, 135, 135, 417, 417, 128, True, False),   # heads not divisible over the XCDs
+    (1, 251, 251, 513, 513, 64, True, False),
     (1, 128, 16, 513, 300, 128, True, True),     # queries past the last key
-    (2, 70, 10, 400, 500, 64, True, True),
+    (2, 130, 10, 400, 500, 64, True, True),
     (4, 32, 8, 290, 333, 128, False, True),
     (4, 32, 32, 384, 32, 128, False, False),     # one key tile
-    (2, 64, 64, 257, 97, 64, False, True),
+    (2, 64, 64, 257, 97, 128, False, True),
     # 64 queries and two key groups per workgroup
     (1, 64, 16, 449, 449, 128, True, False),
     (1, 220, 4, 64, 64, 64, True, False),        # one query block: the second group's only tile is the diagonal
@@ -47,6 +48,8 @@ def _inputs(B, Hq, Hkv, Sq, Sk, D, bias):
     (2, 32, 8, 400, 33, 128, False, True),       # a second key group with one partial tile
     (1, 64, 64, 400, 31, 64, False, False),      # a second key group without a tile
     (2, 32, 32, 400, 545, 64, False, True),
+    (4, 32, 16, 333, 290, 64, False, True),      # head_dim 64: also beyond one round of workgroups
+    (1, 280, 4, 64, 64, 64, True, False),
 ])
 def test_attention_shared_tiles(dev, B, Hq, Hkv, Sq, Sk, D, causal, bias):
     q, k, v, kb = _inputs(B, Hq, Hkv, Sq, Sk, D, bias)
@@ -73,7 +76,7 @@ def test_attention_shared_outputs(dev, B, H, S, D):
     assert torch.equal(packed.unpack(), want)
 
 
-@pytest.mark.parametrize("M,Hq,Hkv,D", [(449, 64, 16, 128), (417, 128, 16, 128), (385, 140, 4, 64), (70, 160, 8, 64)])
+@pytest.mark.parametrize("M,Hq,Hkv,D", [(449, 64, 16, 128), (417, 128, 16, 128), (385, 140, 4, 64), (449, 300, 4, 64), (70, 200, 8, 64)])
 def test_gqa_operator_shared_tiles(dev, M, Hq, Hkv, D):
     """The fused Q norm + RoPE of a wave's own rows."""
     inp = W.gqa_inputs(W.GqaCfg(q_heads=Hq, kv_heads=Hkv, head_dim=D, seq=M, seed=M))
