@@ -8,8 +8,11 @@ with `torch.empty` (caching allocator, hipGraph-safe) unless `out=` is given.
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import gc
 import math
+import threading
 from typing import Optional, Sequence
 
 import torch
@@ -808,6 +811,42 @@ def action_decode_euler(x: PackedAct, w_out: torch.Tensor, b_out: torch.Tensor, 
     _lib.check(_lib.load().rldx_action_decode_euler_bf16(x.data.data_ptr(), n, hidden, float(eps), w_out.data_ptr(),
                                                          b_out.data_ptr(), adim, float(dt), act.data_ptr(),
                                                          _stream_ptr(act)), "rldx_action_decode_euler_bf16")
+
+
+_gc_lock = threading.Lock()
+_gc_holds = 0
+_gc_resume = False
+
+
+@contextlib.contextmanager
+def hold_gc():
+    """Automatic cyclic garbage collection off inside (nested and from several
+    threads: on again when the last one leaves, if it was on)."""
+    global _gc_holds, _gc_resume
+    with _gc_lock:
+        if _gc_holds == 0:
+            _gc_resume = gc.isenabled()
+            gc.disable()
+        _gc_holds += 1
+    try:
+        yield
+    finally:
+        with _gc_lock:
+            _gc_holds -= 1
+            if _gc_holds == 0 and _gc_resume:
+                gc.enable()
+
+
+@contextlib.contextmanager
+def record_graph(graph: "torch.cuda.CUDAGraph"):
+    """torch.cuda.graph(graph) that no garbage collection can break.  A dropped
+    chain that was installed on a module is a reference cycle (module.forward is
+    the dispatcher, which holds the module), so its recorded graphs die in whatever
+    collection comes next; a graph's destructor synchronises the device, which is
+    an error while a stream is capturing, and an error in a destructor ends the
+    process."""
+    with hold_gc(), torch.cuda.graph(graph):
+        yield
 
 
 class GemmWorkspace:

@@ -314,7 +314,7 @@ class MsatActionStep:
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
+        with Fn.record_graph(self.graph):
             self.run()
         torch.cuda.synchronize()
 

@@ -776,7 +776,7 @@ class RldxMsat:
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
+        with Fn.record_graph(self.graph):
             self._forward_static()
         torch.cuda.synchronize()
 
@@ -1278,7 +1278,7 @@ class RldxActionHead:
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
+        with Fn.record_graph(self.graph):
             self.run()
         torch.cuda.synchronize()
 

@@ -1,5 +1,6 @@
 """pytest configuration: import paths and the `gpu` marker."""
 
+import gc
 import sys
 from pathlib import Path
 
@@ -13,6 +14,14 @@ for p in (ROOT, ROOT / "rldx-1_amd"):
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a ROCm GPU (MI355X / gfx950)")
+
+
+@pytest.fixture(autouse=True)
+def collect_before_gpu_tests(request):
+    """Graphs of earlier tests that sit in reference cycles are freed here, not by
+    a collection inside a test's own stream capture (where freeing one aborts)."""
+    if request.node.get_closest_marker("gpu"):
+        gc.collect()
 
 
 @pytest.fixture(scope="session")

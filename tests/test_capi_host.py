@@ -578,3 +578,32 @@ def test_residual_packed_epilogue_and_layernorm_fold_rejections():
     assert pack(4096, 1536, 10, 1536, 8192, None, None) == inval
     assert pack(4096, 1536, 10, 1552, 8192, 16384, None) == inval  # k % 64
     assert pack(4096, 1536, 10, 1536, 8192, 16388, None) == inval  # stats alignment
+
+
+def test_no_garbage_collection_while_a_graph_is_recorded():
+    """hold_gc (around every stream capture of the package) keeps cyclic garbage
+    alive whatever is allocated inside, also nested, and resumes collection after."""
+    import gc
+    import inspect
+    import weakref
+
+    from rldx_amd import msat_step, rldx_msat
+
+    class Node:
+        pass
+
+    assert gc.isenabled()
+    node = Node()
+    node.me, seen = node, weakref.ref(node)
+    with Fn.hold_gc():
+        del node
+        with Fn.hold_gc():
+            pass
+        keep = [[] for _ in range(200000)]
+        assert seen() is not None and not gc.isenabled()
+    assert gc.isenabled()
+    del keep
+    gc.collect()
+    assert seen() is None
+    for mod in (msat_step, rldx_msat):
+        assert "torch.cuda.graph(" not in inspect.getsource(mod)
