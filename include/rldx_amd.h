@@ -516,6 +516,44 @@ hipError_t rldx_action_decode_euler_bf16(const void* packed, int64_t n, int64_t 
                                          const void* b_out, int64_t action_dim, float dt, void* act,
                                          hipStream_t stream);
 
+/* One strided block of rows, per batch entry (strides in bytes). */
+typedef struct rldx_copy_rows {
+  const void* src;
+  void* dst;
+  int64_t rows, row_bytes;
+  int64_t src_row_stride, src_batch_stride, dst_row_stride, dst_batch_stride;
+} rldx_copy_rows_t;
+
+/*
+ * Copies up to 4 row blocks of `batch` entries in one launch (the time token, SA
+ * and VL inputs of a denoising step: three copies of the eager chain,
+ * rldx/inference/action_model/engine/custom_msat_chain.py:109-126).  Row lengths,
+ * pointers and strides are multiples of 16 bytes; the blocks do not overlap.
+ */
+hipError_t rldx_copy_rows_many(const rldx_copy_rows_t* copies, int32_t count, int64_t batch, hipStream_t stream);
+
+/*
+ * dst[i][b] = src[i][idx[b]] for up to 16 stacked parameters of num_slabs slabs of
+ * slab_bytes[i] bytes each (multiples of 16) and batch ids idx (device memory), one
+ * launch: the per-embodiment weights W[e], b[e] of CategorySpecificLinear
+ * (rldx/model/modules/action_model/embodiment_conditioned_mlp.py:72-82).  An id
+ * outside [0, num_slabs) copies nothing.
+ */
+hipError_t rldx_gather_slabs(const void* const* src, void* const* dst, const int64_t* slab_bytes, int32_t count,
+                             const int64_t* idx, int64_t batch, int64_t num_slabs, hipStream_t stream);
+
+/*
+ * packed [batch rows, d] (packed activation order) = LN(x) (1 + scale) + shift:
+ * LayerNorm without affine parameters, then bf16(1 + scale), the product and the sum
+ * each rounded to bf16 (MSAT._output_projection,
+ * rldx/model/modules/action_model/msat.py:777-781).  x: rows of `batch` entries
+ * (strides in elements, % 8), shift / scale [batch, d] with one batch stride (% 8);
+ * d % 16 == 0, d <= 8192.
+ */
+hipError_t rldx_adaln_pack_bf16(const void* x, int64_t x_row_stride, int64_t x_batch_stride, int64_t rows,
+                                int64_t batch, const void* shift, const void* scale, int64_t mod_batch_stride,
+                                int64_t d, float eps, void* packed, hipStream_t stream);
+
 /* One stream of a grouped GEMM. */
 typedef struct rldx_gemm_group {
   const void* a_packed;  /* [m, k] bf16 activations in the packed activation order */

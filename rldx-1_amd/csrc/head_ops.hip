@@ -1,0 +1,255 @@
+// The small data movements of the action head around the MSAT blocks, one launch
+// where the eager chain has several.  Each torch launch there runs 4-5 us of a
+// captured graph on a few hundred KB: latency, not bandwidth, so the win is the
+// number of launches:
+// an action of 4 steps at the release shape took 4.740 ms with the 14 index_selects,
+// 12 copies and 16 modulation launches they replace, 4.617 ms now (bits unchanged).
+// Row and slab pieces are 16 KB per workgroup (4 loads of 16 bytes in flight per
+// thread): below the size of every operand there, so each launch covers the chip.
+//   * copy_rows_many: up to 4 strided row blocks (time token, SA and VL inputs of a
+//     denoising step into the chain's buffers);
+//   * gather_slabs: slab idx[b] of up to 16 stacked parameters (the embodiment's
+//     encoder / decoder weights) into per-robot buffers;
+//   * adaln_pack: the output modulation LN(x) (1 + scale) + shift and the packing of
+//     its rows for the output projection.
+#include "rldx_amd.h"
+#include "rldx_common.h"
+
+namespace rldx {
+namespace {
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kMaxCopies = 4, kMaxSlabs = 16;
+constexpr int kPiece = 1024;  // 16-byte units per workgroup (256 threads x 4)
+
+bool a16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+struct CopyArgs {
+  const char* src[kMaxCopies];
+  char* dst[kMaxCopies];
+  int64_t src_row[kMaxCopies], src_batch[kMaxCopies], dst_row[kMaxCopies], dst_batch[kMaxCopies];
+  int units[kMaxCopies];          // 16-byte units per row
+  int total[kMaxCopies];          // rows x units
+  int begin[kMaxCopies + 1];      // first workgroup
+  int count;
+};
+
+__global__ __launch_bounds__(256) void copy_rows_kernel(CopyArgs a) {
+  int i = 0;
+#pragma unroll
+  for (int c = 1; c < kMaxCopies; ++c)
+    if (c < a.count && static_cast<int>(blockIdx.x) >= a.begin[c]) i = c;
+  const int64_t b = blockIdx.y;
+  const int base = (static_cast<int>(blockIdx.x) - a.begin[i]) * kPiece + static_cast<int>(threadIdx.x);
+  const int units = a.units[i], total = a.total[i];
+  u32x4 v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int u = min(base + 256 * j, total - 1), r = u / units;
+    v[j] = *reinterpret_cast<const u32x4*>(a.src[i] + b * a.src_batch[i] + r * a.src_row[i] + (u - r * units) * 16LL);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int u = base + 256 * j, r = u / units;
+    if (u < total)
+      *reinterpret_cast<u32x4*>(a.dst[i] + b * a.dst_batch[i] + r * a.dst_row[i] + (u - r * units) * 16LL) = v[j];
+  }
+}
+
+struct SlabArgs {
+  const char* src[kMaxSlabs];
+  char* dst[kMaxSlabs];
+  int64_t units[kMaxSlabs];  // 16-byte units per slab
+  int begin[kMaxSlabs + 1];
+  const int64_t* idx;
+  int64_t num;
+  int count;
+};
+
+__global__ __launch_bounds__(256) void gather_slabs_kernel(SlabArgs a) {
+  int i = 0;
+  for (int c = 1; c < a.count; ++c)
+    if (static_cast<int>(blockIdx.x) >= a.begin[c]) i = c;
+  const int64_t b = blockIdx.y, e = a.idx[b];
+  if (e < 0 || e >= a.num) return;  // (the host checks the ids; never read outside the stack)
+  const int64_t units = a.units[i];
+  const u32x4* src = reinterpret_cast<const u32x4*>(a.src[i]) + e * units;
+  u32x4* dst = reinterpret_cast<u32x4*>(a.dst[i]) + b * units;
+  const int64_t base = static_cast<int64_t>(static_cast<int>(blockIdx.x) - a.begin[i]) * kPiece + threadIdx.x;
+  u32x4 v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int64_t u = base + 256 * j;
+    v[j] = src[u < units ? u : units - 1];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (base + 256 * j < units) dst[base + 256 * j] = v[j];
+}
+
+// One wave per row; lane j holds columns 8 (j + 64 c) .. +7.  LayerNorm without
+// affine parameters as rows_pack_kernel (two passes in registers, one rounding),
+// then bf16(1 + scale), the product and the sum, each rounded, as the eager chain.
+struct AdalnArgs {
+  const uint16_t* x;
+  const uint16_t *shift, *scale;
+  uint16_t* out;
+  int64_t x_row, x_batch, mod_batch;
+  int rows, batch, d;
+  float eps;
+};
+
+template <int CPL>
+__global__ __launch_bounds__(256) void adaln_pack_kernel(AdalnArgs a) {
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x & 63;
+  const int t = static_cast<int>(blockIdx.x) * 4 + (threadIdx.x >> 6);  // row of the packed output
+  if (t >= a.rows * a.batch) return;
+  const int b = t / a.rows, r = t - b * a.rows, d = a.d;
+  const uint16_t* xr = a.x + b * a.x_batch + r * a.x_row;
+  const uint16_t* sh = a.shift + b * a.mod_batch;
+  const uint16_t* sc = a.scale + b * a.mod_batch;
+  const u32x4 z = {0, 0, 0, 0};
+  u32x4 raw[CPL], shv[CPL], scv[CPL];
+  float sum = 0.f;
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) {
+    const int col = 8 * (lane + 64 * c);
+    raw[c] = col < d ? *reinterpret_cast<const u32x4*>(xr + col) : z;
+    shv[c] = col < d ? *reinterpret_cast<const u32x4*>(sh + col) : z;
+    scv[c] = col < d ? *reinterpret_cast<const u32x4*>(sc + col) : z;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      sum += bf16x2_lo(raw[c][i]);
+      sum += bf16x2_hi(raw[c][i]);
+    }
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  const float mean = sum / static_cast<float>(d);
+  float sq = 0.f;
+#pragma unroll
+  for (int c = 0; c < CPL; ++c)
+    if (8 * (lane + 64 * c) < d) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float lo = bf16x2_lo(raw[c][i]) - mean, hi = bf16x2_hi(raw[c][i]) - mean;
+        sq += lo * lo;
+        sq += hi * hi;
+      }
+    }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) sq += __shfl_xor(sq, o, 64);
+  const float rstd = 1.0f / __builtin_sqrtf(sq / static_cast<float>(d) + a.eps);
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) {
+    const int col = 8 * (lane + 64 * c);
+    if (col >= d) continue;
+    u32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t y = pack_bf16x2((bf16x2_lo(raw[c][i]) - mean) * rstd, (bf16x2_hi(raw[c][i]) - mean) * rstd);
+      const uint32_t s1 = pack_bf16x2(1.0f + bf16x2_lo(scv[c][i]), 1.0f + bf16x2_hi(scv[c][i]));
+      const uint32_t p = pack_bf16x2(bf16x2_lo(y) * bf16x2_lo(s1), bf16x2_hi(y) * bf16x2_hi(s1));
+      o[i] = pack_bf16x2(bf16x2_lo(p) + bf16x2_lo(shv[c][i]), bf16x2_hi(p) + bf16x2_hi(shv[c][i]));
+    }
+    *reinterpret_cast<u32x4*>(a.out + packed_act_offset(t, col, d)) = o;
+  }
+}
+
+}  // namespace
+}  // namespace rldx
+
+using namespace rldx;
+
+extern "C" hipError_t rldx_copy_rows_many(const rldx_copy_rows_t* copies, int32_t count, int64_t batch,
+                                          hipStream_t stream) {
+  if (!copies || count < 1 || count > kMaxCopies || batch < 0 || batch > 65535) return hipErrorInvalidValue;
+  CopyArgs a{};
+  int n = 0;
+  int64_t blocks = 0;
+  for (int i = 0; i < count; ++i) {
+    const rldx_copy_rows_t& c = copies[i];
+    if (c.rows < 0 || c.row_bytes < 0 || c.row_bytes % 16) return hipErrorInvalidValue;
+    if (c.rows == 0 || c.row_bytes == 0) continue;
+    if (!c.src || !c.dst || !a16(c.src) || !a16(c.dst) || c.src_row_stride % 16 || c.src_batch_stride % 16 ||
+        c.dst_row_stride % 16 || c.dst_batch_stride % 16)
+      return hipErrorInvalidValue;
+    const int64_t units = c.row_bytes / 16;
+    if (c.rows > (1 << 24) || units > (1 << 24) || c.rows * units > (1 << 30)) return hipErrorInvalidValue;
+    a.src[n] = static_cast<const char*>(c.src);
+    a.dst[n] = static_cast<char*>(c.dst);
+    a.src_row[n] = c.src_row_stride;
+    a.src_batch[n] = c.src_batch_stride;
+    a.dst_row[n] = c.dst_row_stride;
+    a.dst_batch[n] = c.dst_batch_stride;
+    a.units[n] = static_cast<int>(units);
+    a.total[n] = static_cast<int>(c.rows * units);
+    a.begin[n] = static_cast<int>(blocks);
+    blocks += (c.rows * units + kPiece - 1) / kPiece;
+    ++n;
+  }
+  if (n == 0 || batch == 0) return hipSuccess;
+  a.count = n;
+  hipLaunchKernelGGL(copy_rows_kernel, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(batch)), dim3(256), 0,
+                     stream, a);
+  return hipGetLastError();
+}
+
+extern "C" hipError_t rldx_gather_slabs(const void* const* src, void* const* dst, const int64_t* slab_bytes,
+                                        int32_t count, const int64_t* idx, int64_t batch, int64_t num_slabs,
+                                        hipStream_t stream) {
+  if (!src || !dst || !slab_bytes || count < 1 || count > kMaxSlabs || batch < 0 || batch > 65535 || num_slabs < 0)
+    return hipErrorInvalidValue;
+  SlabArgs a{};
+  int n = 0;
+  int64_t blocks = 0;
+  for (int i = 0; i < count; ++i) {
+    if (slab_bytes[i] < 0 || slab_bytes[i] % 16) return hipErrorInvalidValue;
+    if (slab_bytes[i] == 0) continue;
+    if (!src[i] || !dst[i] || !a16(src[i]) || !a16(dst[i])) return hipErrorInvalidValue;
+    a.src[n] = static_cast<const char*>(src[i]);
+    a.dst[n] = static_cast<char*>(dst[i]);
+    a.units[n] = slab_bytes[i] / 16;
+    a.begin[n] = static_cast<int>(blocks);
+    blocks += (a.units[n] + kPiece - 1) / kPiece;
+    if (blocks > (1 << 30)) return hipErrorInvalidValue;
+    ++n;
+  }
+  if (n == 0 || batch == 0) return hipSuccess;
+  if (!idx || reinterpret_cast<uintptr_t>(idx) % 8) return hipErrorInvalidValue;
+  a.idx = idx;
+  a.num = num_slabs;
+  a.count = n;
+  hipLaunchKernelGGL(gather_slabs_kernel, dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(batch)), dim3(256),
+                     0, stream, a);
+  return hipGetLastError();
+}
+
+extern "C" hipError_t rldx_adaln_pack_bf16(const void* x, int64_t x_row_stride, int64_t x_batch_stride, int64_t rows,
+                                           int64_t batch, const void* shift, const void* scale,
+                                           int64_t mod_batch_stride, int64_t d, float eps, void* packed,
+                                           hipStream_t stream) {
+  if (rows < 0 || batch < 0 || d < 0 || !(eps >= 0.f)) return hipErrorInvalidValue;
+  if (rows == 0 || batch == 0 || d == 0) return hipSuccess;
+  if (!x || !shift || !scale || !packed || !a16(x) || !a16(shift) || !a16(scale) || !a16(packed) || x_row_stride % 8 ||
+      x_batch_stride % 8 || mod_batch_stride % 8 || d % 16 || d > 8192 || rows * batch > (1 << 28))
+    return hipErrorInvalidValue;
+  const AdalnArgs a{static_cast<const uint16_t*>(x),     static_cast<const uint16_t*>(shift),
+                    static_cast<const uint16_t*>(scale), static_cast<uint16_t*>(packed),
+                    x_row_stride,                        x_batch_stride,
+                    mod_batch_stride,                    static_cast<int>(rows),
+                    static_cast<int>(batch),             static_cast<int>(d),
+                    eps};
+  const dim3 grid(static_cast<unsigned>((rows * batch + 3) / 4)), block(256);
+  if (d <= 1024)
+    hipLaunchKernelGGL(adaln_pack_kernel<2>, grid, block, 0, stream, a);
+  else if (d <= 2048)
+    hipLaunchKernelGGL(adaln_pack_kernel<4>, grid, block, 0, stream, a);
+  else if (d <= 4096)
+    hipLaunchKernelGGL(adaln_pack_kernel<8>, grid, block, 0, stream, a);
+  else
+    hipLaunchKernelGGL(adaln_pack_kernel<16>, grid, block, 0, stream, a);
+  return hipGetLastError();
+}

@@ -26,6 +26,14 @@ class Rows(ctypes.Structure):
                 ("packed", ctypes.c_void_p)]
 
 
+class CopyRows(ctypes.Structure):
+    """rldx_copy_rows_t"""
+
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p)] + [
+        (n, ctypes.c_int64) for n in ("rows", "row_bytes", "src_row_stride", "src_batch_stride", "dst_row_stride",
+                                      "dst_batch_stride")]
+
+
 class GemmGroup(ctypes.Structure):
     """rldx_gemm_group_t"""
 
@@ -150,6 +158,9 @@ SIGNATURES = {
     "rldx_action_encode_pack_bf16": (c_i32, [c_vp, c_i64, c_i64, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp, c_vp,
                                              ctypes.POINTER(Rows), ctypes.POINTER(c_vp), c_i32, c_vp]),
     "rldx_action_decode_euler_bf16": (c_i32, [c_vp, c_i64, c_i64, c_f32, c_vp, c_vp, c_i64, c_f32, c_vp, c_vp]),
+    "rldx_copy_rows_many": (c_i32, [ctypes.POINTER(CopyRows), c_i32, c_i64, c_vp]),
+    "rldx_gather_slabs": (c_i32, [ctypes.POINTER(c_vp), ctypes.POINTER(c_vp), c_i64p, c_i32, c_vp, c_i64, c_i64, c_vp]),
+    "rldx_adaln_pack_bf16": (c_i32, [c_vp, c_i64, c_i64, c_i64, c_i64, c_vp, c_vp, c_i64, c_i64, c_f32, c_vp, c_vp]),
     "rldx_grouped_gemm_mixed_bf16": (c_i32, [ctypes.POINTER(GemmGroup), c_i64p, c_i64p, ctypes.POINTER(c_i32),
                                              ctypes.POINTER(c_vp), c_i32, c_i32, c_i32, c_vp, c_i64, c_vp]),
     "rldx_grouped_gemm_mixed_workspace_bytes": (c_i64, [ctypes.POINTER(GemmGroup), c_i64p, c_i64p,

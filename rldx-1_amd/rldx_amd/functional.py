@@ -849,6 +849,73 @@ def record_graph(graph: "torch.cuda.CUDAGraph"):
         yield
 
 
+def copy_rows_many(pairs: Sequence[tuple]) -> None:
+    """dst.copy_(src) of up to 4 pairs of [B, rows, d] tensors in one launch
+    (rldx_copy_rows_many); pairs whose types or alignment the kernel does not
+    take are copied by torch."""
+    _require(1 <= len(pairs) <= 4, "between 1 and 4 copies")
+    batch = pairs[0][0].shape[0]
+    descs, n, dev = (_lib.CopyRows * len(pairs))(), 0, pairs[0][1].device
+    for src, dst in pairs:
+        _on_gpu(dst)
+        _require(src.dim() == 3 and src.shape == dst.shape and src.shape[0] == batch, "pairs of [B, rows, d] tensors")
+        es = dst.element_size()
+        strides = [src.stride(1), src.stride(0), dst.stride(1), dst.stride(0)]
+        if (src.device != dev or dst.device != dev or src.dtype != dst.dtype or src.stride(2) != 1 or dst.stride(2) != 1 or
+                src.shape[2] * es % 16 or any(v * es % 16 for v in strides) or src.data_ptr() % 16 or dst.data_ptr() % 16):
+            dst.copy_(src)
+            continue
+        descs[n] = _lib.CopyRows(src.data_ptr(), dst.data_ptr(), src.shape[1], src.shape[2] * es, *[v * es for v in strides])
+        n += 1
+    if n:
+        _lib.check(_lib.load().rldx_copy_rows_many(descs, n, batch, _stream_ptr(pairs[0][1])), "rldx_copy_rows_many")
+
+
+def gather_slabs(pairs: Sequence[tuple], idx: torch.Tensor) -> None:
+    """out[b] = stack[idx[b]] of up to 16 (stack [E, ...], out [B, ...]) pairs in one
+    launch (rldx_gather_slabs); a pair the kernel does not take goes to torch.index_select."""
+    _require(1 <= len(pairs) <= 16, "between 1 and 16 stacks")
+    _require(idx.dtype == torch.int64 and idx.dim() == 1 and idx.is_contiguous(), "idx must be contiguous int64 [B]")
+    _on_gpu(idx)
+    E, take = pairs[0][0].shape[0], []
+    for stack, out in pairs:
+        _require(stack.dtype == out.dtype and out.shape[0] == idx.numel() and out[0].numel() == stack[0].numel(),
+                 "stacks [E, ...] and outs [B, ...] of one slab shape")
+        if (stack.shape[0] == E and stack.device == out.device == idx.device and stack.is_contiguous() and
+                out.is_contiguous() and stack[0].numel() * stack.element_size() % 16 == 0 and
+                stack.data_ptr() % 16 == 0 and out.data_ptr() % 16 == 0):
+            take.append((stack, out))
+        else:  # (a bias of 7 actions: 14-byte slabs)
+            torch.index_select(stack, 0, idx, out=out.view(idx.numel(), *stack.shape[1:]))
+    if not take:
+        return
+    ptrs = lambda i: (ctypes.c_void_p * len(take))(*[p[i].data_ptr() for p in take])  # noqa: E731
+    nbytes = _lib.i64_array([s[0].numel() * s.element_size() for s, _ in take])
+    _lib.check(_lib.load().rldx_gather_slabs(ptrs(0), ptrs(1), nbytes, len(take), idx.data_ptr(), idx.numel(), E,
+                                             _stream_ptr(idx)), "rldx_gather_slabs")
+
+
+def adaln_pack(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor, out: PackedAct, eps: float = 1e-6) -> None:
+    """out (PackedAct [B rows, d]) = LN(x) (1 + scale[:, None]) + shift[:, None] for x [B, rows, d] and shift, scale
+    [B, d], bf16, each step rounded (rldx_adaln_pack_bf16)."""
+    B, rows, d = x.shape
+    ok = all(t.dtype == BF16 and t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and t.device == x.device
+             for t in (x, shift, scale)) and tuple(shift.shape) == tuple(scale.shape) == (B, d)
+    if not (ok and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0 and
+            (B == 1 or (shift.stride(0) == scale.stride(0) and shift.stride(0) % 8 == 0))):
+        # a modulation of the caller's own in another type, shape or layout
+        y = torch.nn.functional.layer_norm(x, (d,), eps=eps)
+        mod = torch.empty_like(y, memory_format=torch.contiguous_format)
+        torch.add(y * (1 + scale[:, None]), shift[:, None], out=mod)
+        pack_act(mod.view(B * rows, d), out=out)
+        return
+    _on_gpu(x, shift, scale)
+    _check_pack_target(out, B * rows, d)
+    _lib.check(_lib.load().rldx_adaln_pack_bf16(x.data_ptr(), x.stride(1), x.stride(0), rows, B, shift.data_ptr(),
+                                                scale.data_ptr(), shift.stride(0) if B > 1 else 0, d, float(eps),
+                                                out.data.data_ptr(), _stream_ptr(x)), "rldx_adaln_pack_bf16")
+
+
 class GemmWorkspace:
     """Device scratch of the split-K grouped GEMM: per-tile arrival counters and
     fp32 partial tiles.  Zero-filled once here; every launch leaves its counters

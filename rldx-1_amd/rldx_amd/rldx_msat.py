@@ -27,10 +27,12 @@ widths, so each linear is one launch of groups with their own n and k):
     LayerNorm -> packed h_s, both      rldx_layernorm_pack_many_bf16
     w12 + SwiGLU -> packed             rldx_grouped_gemm_mixed_bf16 (swiglu)
     w3 + residual (in place)           rldx_grouped_gemm_mixed_bf16 (residual)
-Per SingleStreamBlock (7 launches):
-    LayerNorm -> packed h; linear1's QKV columns (+ bias); linear1's MLP columns
-    + SwiGLU -> packed; QK-RMSNorm + RoPE; attention -> columns [0, inner) of
-    the packed linear2 operand; mlp_proj (+ bias) -> its columns [inner, ...);
+Per SingleStreamBlock (5 launches for one robot without a P stream, heads of
+64; 7 otherwise):
+    LayerNorm -> packed h; linear1: QKV columns (+ bias, QK-RMSNorm, RoPE, K/V)
+    and MLP columns (SwiGLU -> packed) in one launch (else three: the two GEMMs
+    and rldx_msat_qkv_norm_rope_bf16); attention -> columns [0, inner) of the
+    packed linear2 operand; mlp_proj (+ bias) -> its columns [inner, ...);
     linear2 + residual (in place).
 VL rows are padded to a multiple of 32 (whole 32-row blocks of the packed
 activations, so the SA rows of a packed matrix start at a block boundary); the
@@ -43,8 +45,9 @@ tiles: each is split over K (split_for) towards 256 workgroups, partials summed
 in a fixed order in one shared workspace.
 The SwiGLU widths of the double-stream FFNs (SA 4096, VL 10922) are padded
 with zero weight rows / columns to a multiple of 128 (silu(0) * 0 = 0, so the
-padding contributes nothing).  The output projection's tiny modulation
-(F.silu(temb) -> proj_out_1, LayerNorm * (1 + scale) + shift) runs as torch ops.
+padding contributes nothing).  The output modulation LayerNorm * (1 + scale) +
+shift is one launch into the packed operand of proj_out_2; its shift and scale
+(F.silu(temb) -> proj_out_1) run as torch ops.
 """
 
 from __future__ import annotations
@@ -441,7 +444,6 @@ class RldxMsat:
         self.qkv = self.qkv_buf[:B * nx]
         self.gl = Fn.PackedAct.empty(B * nx, cfg.ss_expanded, self.dev)
         self.cat = Fn.PackedAct.empty(self.pa + B * npp, inner + cfg.ss_hidden, self.dev)
-        self.mod = ebuf(B * cfg.n_sa_pure, cfg.sa_dim)
         self.mod_packed = Fn.PackedAct.empty(B * cfg.n_sa_pure, cfg.sa_dim, self.dev)
         self.out = ebuf(B, cfg.n_sa_pure, cfg.output_dim)
         self.inputs = dict(sa=ebuf(B, cfg.n_sa_pure, cfg.sa_dim), vl=ebuf(B, cfg.n_vl, cfg.vl_dim),
@@ -452,7 +454,6 @@ class RldxMsat:
             self.qkv_p = ebuf(B * npp, 3 * inner)
             self.gl_p = Fn.PackedAct.empty(B * npp, self.sa_ffn_p, self.dev)
             self.gl_p_ss = Fn.PackedAct.empty(B * npp, cfg.ss_expanded, self.dev)
-            self.mod_p = ebuf(B * npp, cfg.sa_dim)
             self.mod_p_packed = Fn.PackedAct.empty(B * npp, cfg.sa_dim, self.dev)
             self.out_p = ebuf(B, npp, cfg.output_dim)
             self.inputs["p"] = ebuf(B, npp, cfg.sa_dim)
@@ -715,14 +716,13 @@ class RldxMsat:
             Fn._require(encoder_attention_mask is None and physics_attention_mask is None,
                         "attention masks need a chain built with vl_mask=True")
         x_sa = self.x_sa.view(B, cfg.n_sa, d)
-        x_sa[:, :nt].copy_(time_token)
-        x_sa[:, nt:].copy_(hidden_states)
         x_vl = self.x_vl.view(B, self.nv, cfg.vl_dim)
-        x_vl[:, :nv].copy_(encoder_hidden_states)
+        copies = [(time_token, x_sa[:, :nt]), (hidden_states, x_sa[:, nt:]), (encoder_hidden_states, x_vl[:, :nv])]
         if self.nv > nv:
             x_vl[:, nv:].zero_()
         if self.phys:
-            self.x_p.view(B, self.np_, d).copy_(physics_embs)
+            copies.append((physics_embs, self.x_p.view(B, self.np_, d)))
+        Fn.copy_rows_many(copies)
         for blk, gm in zip(self.ds, self.ds_gemms):
             self._ds_block(blk, gm)
         # x = [vl_proj_to_sa(vl) | time token | SA]
@@ -732,14 +732,10 @@ class RldxMsat:
             self._ss_block(blk, gm)
         # AdaLN output projections (msat.py:771-781)
         shift, scale, *pmod = self.adaln_of(temb) if adaln is None else adaln
-        sa = F.layer_norm(x_sa[:, nt:], (d,), eps=1e-6)
-        torch.add(sa * (1 + scale[:, None]), shift[:, None], out=self.mod.view(B, cfg.n_sa_pure, d))
-        Fn.pack_act(self.mod, out=self.mod_packed)
+        Fn.adaln_pack(x_sa[:, nt:], shift, scale, self.mod_packed)
         if self.phys:
             pshift, pscale = pmod
-            ph = F.layer_norm(self.x_p.view(B, self.np_, d), (d,), eps=1e-6)
-            torch.add(ph * (1 + pscale[:, None]), pshift[:, None], out=self.mod_p.view(B, self.np_, d))
-            Fn.pack_act(self.mod_p, out=self.mod_p_packed)
+            Fn.adaln_pack(self.x_p.view(B, self.np_, d), pshift, pscale, self.mod_p_packed)
         self._gemm(self.out_gemm)
         if self.phys:
             return {"action": self.out, "physics": self.out_p}
@@ -1229,9 +1225,8 @@ class RldxActionHead:
     def run(self) -> torch.Tensor:
         sd, mc, cfg = self.sd, self.msat.cfg, self.cfg
         d, H = self.d, cfg.action_horizon
-        for n in _CAT_LINEARS:
-            torch.index_select(sd[f"{n}.W"], 0, self.e_idx, out=self.w_e[n])
-            torch.index_select(sd[f"{n}.b"], 0, self.e_idx, out=self.b_e[n][:, 0])
+        Fn.gather_slabs([(sd[f"{n}.W"], self.w_e[n]) for n in _CAT_LINEARS] +
+                        [(sd[f"{n}.b"], self.b_e[n]) for n in _CAT_LINEARS], self.e_idx)
         if cfg.use_vlln:
             self.vl_n.copy_(F.layer_norm(self.vl, (mc.vl_dim,), sd["vlln.weight"], sd["vlln.bias"], cfg.vlln_eps))
         h = F.relu(self._cat(self.state, "state_encoder.layer1"))

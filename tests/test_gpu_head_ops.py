@@ -1,0 +1,74 @@
+"""GPU tests of the action head's small launches: the strided row copies, the
+gather of stacked parameters (both bit for bit) and the output modulation with
+its packing (against the eager chain on the CPU)."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from rldx_amd import functional as Fn
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def rnd(*shape, seed=0, dtype=BF16):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype).cuda()
+
+
+@pytest.mark.parametrize("batch", [1, 3])
+def test_copy_rows_many(batch):
+    """1 unit, one workgroup exactly (1024 units), one past it, strided and broadcast
+    sources; nothing outside the destination rows changes.  A row of 12 bytes and a
+    source of another type take torch's copy."""
+    srcs = [rnd(batch, 1, 8, seed=1), rnd(batch, 16, 1024, seed=2)[:, ::2, :512], rnd(1, 41, 200, seed=3).expand(batch, 41, 200),
+            rnd(batch, 18, 1536, seed=4)]
+    buf = [torch.full((batch, s.shape[1] + 2, s.shape[2] + 8), 7.0, dtype=BF16, device="cuda") for s in srcs]
+    Fn.copy_rows_many([(s, b[:, 1:-1, :-8]) for s, b in zip(srcs, buf)])
+    for s, b in zip(srcs, buf):
+        assert torch.equal(b[:, 1:-1, :-8], s)
+        assert bool((b[:, 0] == 7).all() and (b[:, -1] == 7).all() and (b[:, :, -8:] == 7).all())
+    odd = [(rnd(batch, 5, 6), torch.zeros(batch, 5, 6, dtype=BF16, device="cuda")),
+           (rnd(batch, 5, 16, dtype=torch.float32), torch.zeros(batch, 5, 16, dtype=BF16, device="cuda"))]
+    Fn.copy_rows_many(odd)
+    assert all(torch.equal(d, s.to(BF16)) for s, d in odd)
+    with pytest.raises(Exception):
+        Fn.copy_rows_many([(srcs[0], buf[1])])
+
+
+@pytest.mark.parametrize("ids", [[2], [0, 4, 4]])
+def test_gather_slabs(ids):
+    """Slabs of one unit, of 1024 units and of one more, and one of 14 bytes (torch's
+    index_select); an id outside the stacks copies nothing."""
+    idx = torch.tensor(ids, device="cuda")
+    stacks = [rnd(5, 8, seed=1), rnd(5, 64, 128, seed=2), rnd(5, 8200, seed=3), rnd(5, 7, seed=4)]
+    outs = [torch.zeros(len(ids), 1, *s.shape[1:], dtype=BF16, device="cuda") for s in stacks]
+    Fn.gather_slabs(list(zip(stacks, outs)), idx)
+    for s, o in zip(stacks, outs):
+        assert torch.equal(o[:, 0], s[idx])
+    kept = outs[1].clone()
+    Fn.gather_slabs([(stacks[1], outs[1])], idx * 0 + 5)
+    Fn.gather_slabs([(stacks[1], outs[1])], idx * 0 - 1)
+    assert torch.equal(outs[1], kept)
+
+
+@pytest.mark.parametrize("batch,rows,d", [(1, 1, 16), (1, 17, 1536), (3, 31, 1040), (2, 33, 2064), (1, 3, 8192)])
+def test_adaln_pack(batch, rows, d):
+    """Each CPL of the kernel at its first width and rows across 32-row blocks.  The
+    CPU chain rounds at the same three places; only the LayerNorm's summation order
+    differs, so a value near a rounding edge may take the neighbouring bf16 in each of
+    them: 3 steps of at most 2^-7 relative, and seldom (fp32 sums differ by ~2^-20,
+    edges are hit once in ~2^11 values)."""
+    x = rnd(batch, rows + 2, d, seed=d)[:, 1:-1] * 3 + 1
+    shift, scale = rnd(batch, 2 * d, seed=d + 1).chunk(2, dim=1)
+    m = batch * rows
+    for s in (scale, scale.float()):  # (a scale of another type takes the eager chain)
+        y = F.layer_norm(x.cpu(), (d,), eps=1e-6) * (1 + s.cpu()[:, None])
+        want = (y + shift.cpu()[:, None]).to(BF16).float().view(m, d)
+        out = Fn.PackedAct.empty(m, d, "cuda")
+        Fn.adaln_pack(x, shift, s, out)
+        got = out.data.cpu().view(-1, d // 16, 2, 32, 8)  # [32-row block, 16-column chunk, half, row, 8]
+        got = got.permute(0, 3, 1, 2, 4).reshape(-1, d)[:m].float()
+        bound = 3 * 2**-7 * torch.maximum(y.float().abs().view(m, d), want.abs())
+        assert bool(((got - want).abs() <= bound).all())
+        assert int((got != want).sum()) <= 4 + m * d // 256
