@@ -10,7 +10,9 @@
 //     (rldx/model/modules/backbone/modeling_qwen3_vl.py:139-176, :356-490;
 //     rldx/inference/backbone/llm/engine/kernels/fused_llm_attention.py:379-770).
 //
-// Design (short sequences: 608 / 1280 tokens, batch 1)
+// Design (short sequences, launches of up to about two workgroups per CU; longer
+// ones take attn_shared_kernel below, whose waves read K/V tiles that the workgroup
+// loads into LDS once -- shared_groups() draws the line)
 //   * K and V are read in a packed tile layout (below) in which every MFMA
 //     operand of a 32-key tile is one contiguous 1 KB block: lane l reads the
 //     16 bytes at l*16.  Operands therefore go straight from global memory into
@@ -1633,10 +1635,10 @@ void launch_attn_d(AttnArgs a, int batch, bool causal, bool has_bias, hipStream_
 
 template <bool kQNorm>
 hipError_t launch_attn(AttnArgs a, int64_t head_dim, int batch, bool causal, bool has_bias, hipStream_t stream) {
-  // 32 queries per workgroup: at 608-2560 tokens the kernel is latency-bound, and
-  // twice the workgroups (two per CU, two waves per SIMD) beat the doubled K/V
-  // operand reuse of 64-query workgroups (measured on MI355X: 12 x 608 masked
-  // 9.6 vs 14.4 us, 28/4 x 1280 causal 29.5 vs 39.6 us).
+  // 32 queries per workgroup where the tiles are not shared through LDS: these
+  // launches are latency-bound, and twice the workgroups (two per CU, two waves per
+  // SIMD) beat the doubled K/V operand reuse of 64-query workgroups of the same
+  // kernel (measured on MI355X: 12 x 608 masked 9.6 vs 14.4 us).
   constexpr int NSUB = 1;
   a.num_q_blocks = (a.sq + 32 * NSUB - 1) / (32 * NSUB);
   if (head_dim == 128)

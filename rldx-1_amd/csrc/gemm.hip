@@ -42,7 +42,8 @@
 //     64 x 64 one.
 //   * Tile shapes: 128 x 128 (waves 4 x 2, 32 x 64 each) for long streams with
 //     enough tiles; 64 x 64 (waves 2 x 2 in two K-groups) and 32 x 64 (waves
-//     1 x 2 in four K-groups) for the short streams and the N = 1536 GEMMs.
+//     1 x 2 in four K-groups) for the short streams and the N = 1536 GEMMs;
+//     256 x 256 in a kernel of their own (gemm_big_kernel) for one long stream.
 //     K-groups take alternate stages; their partial tiles are summed in a
 //     fixed order, so results are deterministic.
 //   * Stage pipeline per wave: issue the loads of stage s + NSLOT - 1, MFMAs of
