@@ -978,7 +978,10 @@ __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_ke
 #pragma unroll
       for (int e = 0; e < 8; ++e) pv[e] = s[s2 * 8 + e];
       pop[s2] = __builtin_convertvector(pv, bf16x8);
-      // the row sum takes the rounded P, so that P V / l is a mean of V with weights that sum to one
+      // The row sum takes the rounded P, so that P V / l is a mean of V with weights
+      // that sum to one, two per instruction.  Against plain adds of the unrounded P:
+      // 28/4 x 1280 36.9 -> 33.9 us, 32/8 x 4096 158.6 -> 153.6, and the output's
+      // error against 64 bits is 0.1-0.3 % less (12 shapes, two seeds).
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         l_part = __builtin_amdgcn_fdot2_f32_bf16(bf16x2_t{pop[s2][2 * e], pop[s2][2 * e + 1]}, kOnes, l_part, false);
