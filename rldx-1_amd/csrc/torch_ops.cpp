@@ -19,6 +19,7 @@
 #include <cmath>
 #include <mutex>
 #include <unordered_map>
+#include <vector>
 
 #include "rldx_amd.h"
 
@@ -300,11 +301,13 @@ Tensor swiglu(const Tensor& x) {
 // Packed weights of ss::fused_mlp_swiglu.  Python packs a weight, keeps the packed
 // copy for as long as the weight lives and enters it here; forget() takes it out
 // when the weight dies.  The weak reference keeps the address from being another
-// tensor's meanwhile, and the version and the data pointer must be the packed ones.
+// tensor's meanwhile, and the version, the data pointer, the sizes and the strides
+// must be the packed ones (`w.data = w.data[:rows]` changes the sizes alone).
 struct Packed {
   c10::weak_intrusive_ptr<c10::TensorImpl> w;
   uint32_t version;
   const void* data;
+  std::vector<int64_t> sizes, strides;
   Tensor packed;
 };
 std::mutex g_packed_mutex;
@@ -319,7 +322,7 @@ void remember_packed(const Tensor& w, const Tensor& packed) {
   const std::lock_guard<std::mutex> lock(g_packed_mutex);
   packed_weights().insert_or_assign(
       key_of(w), Packed{c10::weak_intrusive_ptr<c10::TensorImpl>(w.getIntrusivePtr()),
-                        static_cast<uint32_t>(w._version()), w.data_ptr(), packed});
+                        static_cast<uint32_t>(w._version()), w.data_ptr(), w.sizes().vec(), w.strides().vec(), packed});
 }
 void forget_packed(int64_t key) {
   Tensor drop;  // freed outside the lock
@@ -329,14 +332,16 @@ void forget_packed(int64_t key) {
   drop = std::move(it->second.packed);
   packed_weights().erase(it);
 }
-Tensor packed_of(const Tensor& w) {
-  if (w.is_inference()) return Tensor();
+OptTensor packed_of(const Tensor& w) {
+  if (w.is_inference()) return std::nullopt;
   const std::lock_guard<std::mutex> lock(g_packed_mutex);
   auto it = packed_weights().find(key_of(w));
-  if (it == packed_weights().end() || it->second.w.expired() || it->second.data != w.data_ptr() ||
-      it->second.version != static_cast<uint32_t>(w._version()))
-    return Tensor();
-  return it->second.packed;
+  if (it == packed_weights().end()) return std::nullopt;
+  const Packed& p = it->second;
+  if (p.w.expired() || p.data != w.data_ptr() || p.version != static_cast<uint32_t>(w._version()) ||
+      w.sizes() != p.sizes || w.strides() != p.strides)
+    return std::nullopt;
+  return p.packed;
 }
 
 RLDX_OP(Mlp, "ss::fused_mlp_swiglu");
@@ -344,13 +349,13 @@ Tensor mlp(const Tensor& x, const Tensor& w, const Tensor& bias, SymInt split_) 
   const int64_t split = split_.guard_int(__FILE__, __LINE__);
   if (split <= 1 && rows2d(x) && x.size(0) > 0 && bf16(w) && w.dim() == 2 && w.size(0) % 2 == 0 &&
       one_device(x, w, bias) && vec(bias, w.size(0)) && w.size(1) == x.size(1)) {
-    const Tensor pw = packed_of(w);
-    if (pw.defined()) {
+    const OptTensor pw = packed_of(w);
+    if (pw.has_value()) {
       const c10::OptionalDeviceGuard guard(x.device());
       const int64_t M = x.size(0), K = x.size(1), n = w.size(0);
       Tensor a = at::empty({(M + 31) / 32 * 32 * K}, x.options()), out = at::empty({M, n / 2}, x.options());
       hipStream_t st = stream_of(x);
-      const rldx_gemm_group_t g{a.data_ptr(), M, pw.data_ptr(), bias.data_ptr(), out.data_ptr(), n / 2, nullptr, 0};
+      const rldx_gemm_group_t g{a.data_ptr(), M, pw->data_ptr(), bias.data_ptr(), out.data_ptr(), n / 2, nullptr, 0};
       if (rldx_act_pack_bf16(x.data_ptr(), x.stride(0), M, K, a.data_ptr(), st) == hipSuccess &&
           rldx_grouped_gemm_bf16(&g, 1, n, K, RLDX_GEMM_EPI_SWIGLU, st) == hipSuccess)
         return out;
@@ -428,4 +433,5 @@ TORCH_LIBRARY_IMPL(rldx_amd, AutogradCUDA, m) { RLDX_AUTOGRAD(m, "swiglu", Swigl
 TORCH_LIBRARY(rldx_native, m) {
   m.def("remember_packed(Tensor w, Tensor packed) -> ()", &remember_packed);
   m.def("forget_packed(int key) -> ()", &forget_packed);
+  m.def("packed_of(Tensor w) -> Tensor?", &packed_of);
 }

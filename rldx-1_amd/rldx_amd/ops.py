@@ -345,21 +345,23 @@ def _(x):
 # ---------------------------------------------------------------------------
 # The grouped GEMM reads weights in its packed operand order.  Weights are
 # static, so each one is packed once and the packed copy is kept for as long as
-# the weight tensor lives; an in-place update of the weight (version change)
-# packs it again.
-_packed_weights: dict = {}  # id(weight) -> (weakref to weight, version, data pointer, swiglu_pairs, PackedWeight)
+# the weight tensor lives; an in-place update of the weight (version change) and
+# storage of another address, shape or strides under the same tensor (w.data = ...,
+# which changes no version) pack it again.
+_packed_weights: dict = {}  # id(weight) -> (weakref to weight, what was packed, PackedWeight)
 
 
 def _packed_weight(w: torch.Tensor, swiglu_pairs: bool) -> Fn.PackedWeight:
+    state = (w._version, w.data_ptr(), tuple(w.shape), w.stride(), swiglu_pairs)
     hit = _packed_weights.get(id(w))
-    if hit is not None and hit[0]() is w and hit[1:4] == (w._version, w.data_ptr(), swiglu_pairs):
-        return hit[4]
+    if hit is not None and hit[0]() is w and hit[1] == state:
+        return hit[2]
     pw = Fn.pack_weight(w if w.stride(1) == 1 else w.contiguous(), swiglu_pairs=swiglu_pairs, row_sums=False)
     if hit is None or hit[0]() is not w:
         weakref.finalize(w, _packed_weights.pop, id(w), None)
         if _native:
             weakref.finalize(w, torch.ops.rldx_native.forget_packed, int(w._cdata)).atexit = False
-    _packed_weights[id(w)] = (weakref.ref(w), w._version, w.data_ptr(), swiglu_pairs, pw)
+    _packed_weights[id(w)] = (weakref.ref(w), state, pw)
     if _native and swiglu_pairs:
         torch.ops.rldx_native.remember_packed(w, pw.data)
     return pw

@@ -125,6 +125,12 @@ def test_mlp_weight_updates_and_lifetime(dev):
     _same(op(x, w, b), impl._init_fn(x, w.clone(), b))
     w.data = _rnd(dev, 128, 128, seed=9)  # new storage
     _same(op(x, w, b), impl._init_fn(x, w.clone(), b))
+    whole = w.data  # the same storage under other shapes: fewer rows, all of them again, transposed
+    for data in (whole[:64], whole, whole.t(), whole[64:]):
+        w.data = data
+        for _ in range(2):
+            _same(op(x, w, b[:len(data)].clone()), impl._init_fn(x, data.contiguous().clone(), b[:len(data)].clone()))
+    w.data = whole
     # weights that come and go, at addresses used before; nothing packed is kept
     n = len(ops._packed_weights)
     for i in range(5):

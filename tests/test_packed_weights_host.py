@@ -1,0 +1,72 @@
+"""Host tests of the packed-weight cache of ss::fused_mlp_swiglu (rldx_amd/ops.py and its
+copy in csrc/torch_ops.cpp): a packed copy serves a weight only as it was when packed."""
+
+import pytest
+import torch
+
+from rldx_amd import functional as Fn
+
+ops = pytest.importorskip("rldx_amd.ops")
+BF16 = torch.bfloat16
+
+
+@pytest.fixture
+def packs(monkeypatch):
+    """pack_weight without a GPU: the packed copy is a copy; the list holds the weights' shapes as packed."""
+    seen = []
+
+    def pack(w, swiglu_pairs=False, row_sums=True):
+        seen.append(tuple(w.shape))
+        return Fn.PackedWeight(w.clone().reshape(-1), *w.shape, swiglu_pairs)
+
+    monkeypatch.setattr(Fn, "pack_weight", pack)
+    return seen
+
+
+def _w(*shape):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(sum(shape))).to(BF16)
+
+
+@pytest.mark.parametrize("change", [lambda t: t[:64], lambda t: t.t(), lambda t: t[:, :64], lambda t: t.view(256, 64),
+                                    lambda t: t.view(64, 2, 128)[:, 0]], ids=["rows", "transposed", "columns", "view", "strided"])
+def test_storage_of_another_shape_is_packed_again(packs, change):
+    """`w.data = view of the same storage` keeps the tensor, its version and its data
+    pointer; only the shape and the strides tell it from the packed one."""
+    w = _w(128, 128)
+    before = ops._packed_weight(w, True)
+    assert ops._packed_weight(w, True) is before and len(packs) == 1
+    state = (w._version, w.data_ptr())
+    w.data = change(w.data)
+    assert (w._version, w.data_ptr()) == state
+    after = ops._packed_weight(w, True)
+    assert after is not before and (after.n, after.k) == tuple(w.shape)
+    assert torch.equal(after.data.view(w.shape), w) and len(packs) == 2
+
+
+def test_storage_grown_in_place_is_packed_again(packs):
+    base = _w(256, 128)
+    w = base[:128].detach()
+    small = ops._packed_weight(w, True)
+    w.data = base
+    grown = ops._packed_weight(w, True)
+    assert (small.n, grown.n) == (128, 256) and packs == [(128, 128), (256, 128)]
+
+
+@pytest.mark.skipif(not ops._native, reason="librldx_torch.so was not built")
+def test_native_copy_serves_the_packed_shape_only():
+    native = torch.ops.rldx_native
+    w, packed = _w(128, 128), torch.zeros(128 * 128, dtype=BF16)
+    whole = w.data
+    assert native.packed_of(w) is None
+    native.remember_packed(w, packed)
+    try:
+        for other in (whole[:64], whole.t(), whole[:, :64], whole.view(256, 64)):
+            assert native.packed_of(w).data_ptr() == packed.data_ptr()
+            w.data = other
+            assert native.packed_of(w) is None
+            w.data = whole
+        w.add_(1)  # a new version
+        assert native.packed_of(w) is None
+    finally:
+        native.forget_packed(int(w._cdata))
+    assert native.packed_of(w) is None
