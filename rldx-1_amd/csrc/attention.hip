@@ -873,7 +873,6 @@ __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_ke
   floatx16 oacc[DBLK];
 #pragma unroll
   for (int db = 0; db < DBLK; ++db) oacc[db] = floatx16{};
-  const bf16x2_t kOnes = {static_cast<__bf16>(1.0f), static_cast<__bf16>(1.0f)};
   float m_ref = -__builtin_inff(), l_part = 0.f;
   const float c = a.scale_log2;
   const float kb = kLog2e / c;
@@ -952,9 +951,18 @@ __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_ke
 #pragma unroll
     for (int e = 1; e < 16; ++e) mt = fmaxf(mt, s[e]);
     mt *= c;
-    if (__any(mt > m_ref + kLazyThreshold)) {
+    // The softmax reference: of the first 4 tiles each tile's own maximum (also below
+    // the last one, by less than 2^8), later the maximum so far, moved when a tile
+    // exceeds it by 2^3.  A key that sets a reference weighs exactly 1, which the
+    // rounding of P to bf16 keeps: attn_fwd_kernel has four such keys per row (its
+    // waves' first tiles), and a row that moved its one reference by 2^8 only had an
+    // error against 64 bits up to 27 % larger (128 keys; 0.5-4 % at 256-4096).  With
+    // these it is the same up to 128 keys and 0-16 % smaller beyond (14 shapes, scores
+    // of std 1 to 2.5).  32/8 x 4096 causal 135 -> 136.5 us, 28/4 x 1280 as before.
+    const bool own = i < 4 / NG;
+    if (own || __any(mt > m_ref + 3.f)) {
       const float mq = pair_max(mt);
-      const float new_ref = mq > m_ref + kLazyThreshold ? mq : m_ref;
+      const float new_ref = own ? (mq > m_ref - 8.f ? mq : m_ref) : fmaxf(mq, m_ref);
       const float alpha = (m_ref == -__builtin_inff()) ? 0.f : __builtin_amdgcn_exp2f(m_ref - new_ref);
       m_ref = new_ref;
       l_part *= alpha;
@@ -963,14 +971,17 @@ __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_ke
     }
     const float nm = (m_ref == -__builtin_inff()) ? 0.f : -m_ref;
     if constexpr (PIPE) snew = floatx16{};
+    float psum = 0.f;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       s[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e], c, nm));
+      psum += s[e];
       if constexpr (PIPE) {
 #pragma unroll
         for (int ks = e * KS / 16; ks < (e + 1) * KS / 16; ++ks) score_mma(ks, snew);
       }
     }
+    l_part += psum;
     bf16x8 pop[2];
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
@@ -978,13 +989,6 @@ __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_ke
 #pragma unroll
       for (int e = 0; e < 8; ++e) pv[e] = s[s2 * 8 + e];
       pop[s2] = __builtin_convertvector(pv, bf16x8);
-      // The row sum takes the rounded P, so that P V / l is a mean of V with weights
-      // that sum to one, two per instruction.  Against plain adds of the unrounded P:
-      // 28/4 x 1280 36.9 -> 33.9 us, 32/8 x 4096 158.6 -> 153.6, and the output's
-      // error against 64 bits is 0.1-0.3 % less (12 shapes, two seeds).
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        l_part = __builtin_amdgcn_fdot2_f32_bf16(bf16x2_t{pop[s2][2 * e], pop[s2][2 * e + 1]}, kOnes, l_part, false);
     }
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2)

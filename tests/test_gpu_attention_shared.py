@@ -58,6 +58,53 @@ def test_attention_shared_tiles(dev, B, Hq, Hkv, Sq, Sk, D, causal, bias):
     assert_bf16_close(o, r, "attention, shared tiles")
 
 
+@pytest.mark.parametrize("Hq,Hkv,S,D,causal,part", [
+    (400, 400, 128, 128, False, 80), (416, 416, 64, 64, False, 104), (64, 16, 600, 128, False, 4),  # part: heads per unshared launch
+    (32, 8, 800, 128, True, 8), (300, 60, 128, 128, True, 40), (32, 8, 2100, 128, True, 4), (40, 8, 1100, 64, True, 10)])
+@pytest.mark.parametrize("sharp", [1.0, 2.0])
+def test_shared_tiles_lose_no_precision(dev, Hq, Hkv, S, D, causal, part, sharp):
+    """The error against float64 is not above that of the kernel without shared tiles
+    (the same heads in launches too small to share).  Both round P and O to bf16 and add
+    in fp32, so equal errors are equal up to a few values on a rounding edge: 0.1 %."""
+    g = torch.Generator(device=dev).manual_seed(S + Hq)
+    rnd = lambda h, x=1.0: (x * torch.randn(1, h, S, D, generator=g, device=dev)).to(torch.bfloat16)  # noqa: E731
+    q, k, v = rnd(Hq, sharp), rnd(Hkv), rnd(Hkv)
+    n = Hq // Hkv
+    whole = Fn.attention(q, k, v, causal=causal)
+    parts = torch.cat([Fn.attention(q[:, h:h + part], k[:, h // n:(h + part + n - 1) // n], v[:, h // n:(h + part + n - 1) // n],
+                                    causal=causal) for h in range(0, Hq, part)], dim=1)
+    err, norm = [0.0, 0.0], 0.0
+    for h in range(Hq):
+        p = q[0, h].double() @ k[0, h // n].double().t() * D ** -0.5
+        if causal:
+            p.masked_fill_(torch.ones(S, S, dtype=torch.bool, device=dev).triu(1), float("-inf"))
+        r = torch.softmax(p, -1) @ v[0, h // n].double()
+        norm += float(r.square().sum())
+        for i, o in enumerate((whole, parts)):
+            err[i] += float((o[0, h].double() - r).square().sum())
+    err = [(e / norm) ** 0.5 for e in err]
+    assert err[0] <= 1.001 * err[1], f"shared {err[0]:.4e}, unshared {err[1]:.4e}"
+
+
+@pytest.mark.parametrize("H,S,causal", [(400, 128, False), (64, 600, False), (32, 800, True), (300, 128, True)])
+def test_shared_tiles_infinite_scores(dev, H, S, causal):
+    """Keys that score -inf are ignored, a query with a score of +inf is NaN as in softmax,
+    and the other queries and heads are untouched by it."""
+    g = torch.Generator().manual_seed(S)
+    q, k, v = (torch.randn(1, H, S, 128, generator=g).to(torch.bfloat16) for _ in range(3))
+    clean = Fn.attention(q.to(dev), k.to(dev), v.to(dev), causal=causal)
+    q[0, 3] = q[0, 3].abs()
+    k[0, 3, 40] = -3e38       # -inf for every query of positive elements ...
+    q[0, 3, 90] = -q[0, 3, 90]  # ... and +inf for this one
+    o = Fn.attention(q.to(dev), k.to(dev), v.to(dev), causal=causal)
+    r = ref.sdpa(q[:, 3:4].float(), k[:, 3:4].float(), v[:, 3:4].float(), causal=causal)
+    nan = torch.isnan(r[0, 0]).all(dim=-1)
+    assert nan.nonzero().tolist() == [[90]] and bool(torch.isnan(o[0, 3, 90]).all())
+    assert_bf16_close(o[0, 3].cpu()[~nan], r[0, 0][~nan], "the other queries")
+    rest = [h for h in range(H) if h != 3]
+    assert torch.equal(o[:, rest], clean[:, rest])
+
+
 @pytest.mark.parametrize("B,H,S,D", [(4, 32, 290, 128), (2, 32, 400, 64)])
 def test_attention_shared_outputs(dev, B, H, S, D):
     """Rows of 8-byte alignment, and the packed output by row segments: the same bits as contiguous rows."""
