@@ -1518,11 +1518,10 @@ constexpr int vit_padded_dim(int64_t hd) {
 }
 
 // Key groups of attn_shared_kernel for a launch, or 0 for attn_fwd_kernel.
-// b64, b128: the launch's 64- and 128-query blocks per head; heads: batch x heads.
 // Measured on MI355X (operator us, attn_fwd_kernel / NG = 1 / NG = 2):
 //   causal: the longest block bounds a launch until the blocks of every length
 //   fill the chip, which heads x (blocks + 1) measures (twice the work over the
-//   longest chain).  NG = 2 wins from 440 (32/8 x 800: 29.5 / 28.3 / 25.2 at 448; 32/8 x
+//   longest chain).  NG = 2 wins from 430 (32/8 x 800: 29.5 / 28.3 / 25.2 at 432; 32/8 x
 //   512: 19.4 / 23.0 / 19.5 at 288), with chains past 20 steps from 528 (16/8 x 1536: 34.6 /
 //   43.5 / 36.0 at 400, x 2048: 44.7 / 53.9 / 44.5 at 528, x 2560: 63.7 / 67.8 / 53.8),
 //   NG = 1 over it from 540 (32/8 x 2048: 79.7 / 64.2 / 66.1 at 544; 16/8 x 4096:
@@ -1539,14 +1538,50 @@ constexpr int vit_padded_dim(int64_t hd) {
 //   86, x 6144 213 / 168 / 179 (NG = 1: 1056, 1568);
 //   not causal 1204 + 424 + 897 + 79 36.4 / 39.6 / 32.2 at 704 workgroups, 2304 + 196 + 79
 //   47.6 / 57.8 / 47.4 at 688, joint 24 x 1632 30.2 / 36.9 / 31.0 at 624.
-int shared_groups(bool causal, int64_t head_dim, int64_t heads, int64_t b64, int64_t b128) {
-  const bool narrow = head_dim <= 64;
-  if (causal) {
-    if (heads * (b128 + 1) >= (narrow ? 1200 : 540)) return 1;
-    return heads * (b64 + 1) >= (b64 <= 20 ? (narrow ? 530 : 440) : (narrow ? 650 : 528)) ? 2 : 0;
+// Few query rows per head: below 33 only one wave of a workgroup has queries, and walks
+// all the key tiles that attn_fwd_kernel splits over four (not causal 384 heads x 1 row x
+// 512 keys 9.4 / 13.7 / 11.4, x 4096 45.0 / 76.4 / 49.1; 512 x 1 x 4096 178 / 185 / 179); up to 64
+// NG = 2 fits them (384 x 64 x 512 17.3 / 19.5 / 15.9, x 4096 72.5 / 105 / 67.9, 2048 x 64 x
+// 2048 413 / 397 / 386).  Causal blocks of so few rows have as few keys: NG = 1, from the
+// line where its one workgroup per head saves a round of the chip (rows <= 16: 448 heads 6.08 /
+// 6.19 / 7.69, 576 9.12 / 7.09 / 10.6; x 32: 288 6.95 / 6.48 / 7.98, head_dim 64 5.01 / 4.80 /
+// 5.44; head_dim 64 x 64: 320 5.47 / 5.70, 384 6.31 / 6.01 / 6.23).
+// Past one round of two workgroups per CU NG = 2 falls behind: causal blocks of at most
+// 448 queries then take NG = 1 (112 heads x 280 15.1 / 12.4 / 16.1, 104 x 384 21.5 / 15.9 /
+// 17.8), 33-64 rows from 640 heads (560 x 64 x 700 40.0 / 44.0 / 41.3, 640 42.6 / 45.7 / 41.8).
+// Partly filled blocks count by their rows where the launch has few blocks (156 heads x 78
+// causal, 7.3 / - / 7.8; head_dim 64 224 heads x 79 x 542 10.0 / - / 11.5, 208 x 214 x 1247, 695
+// by rows, 26.3 / - / 27.9) and in a batch of
+// images: many small images leave most blocks nearly empty and a long one bounds the
+// launch (16 images of 2078 rows, the longest 661, 12 heads, 384 by blocks, 195 by rows:
+// 28.8 / 33.5; head_dim 64 3 images of 1574, the longest 1208, 16 heads: 23.5 / - / 26.0;
+// images of one size, 30 x 64 at 16 heads, 23.2 / 20.3, cannot be told from these).
+struct AttnShape {
+  bool causal;
+  int64_t images;     // of a batch of images (rows: of all of them), 0 otherwise
+  int64_t head_dim, heads;  // heads: batch x heads
+  int64_t rows;       // query rows per head
+  int64_t b64, b128;  // 64- and 128-query blocks per head (at most, for a batch of images)
+};
+int shared_groups(const AttnShape& s) {
+  const bool narrow = s.head_dim <= 64;
+  if (s.causal) {
+    if (s.rows <= (narrow ? 64 : 32)) return s.heads >= (s.rows <= 16 ? 513 : s.rows <= 32 ? 270 : 384) ? 1 : 0;
+    if (s.heads * (s.b128 + 1) >= (narrow ? 1200 : 540)) return 1;
+    if (s.b64 > 20) return s.heads * (s.b64 + 1) >= (narrow ? 650 : 528) ? 2 : 0;
+    if (s.heads * (s.rows + 64) < (narrow ? 530 : 430) * 64) return 0;
+    return !narrow && s.b64 <= 7 && s.heads * s.b64 > 512 ? 1 : 2;
   }
-  if (!narrow && heads * b128 >= 380) return 1;
-  return (heads * b64 >= 400 && heads * b64 <= 512) || (narrow && heads * b64 >= 680) ? 2 : 0;
+  if (!s.images && s.rows <= 64 && !narrow)
+    return s.rows > 32 && s.heads >= 380 && (s.heads <= 512 || s.heads >= 640) ? 2 : 0;
+  const int64_t blocks = s.heads * s.b64, filled = s.heads * s.rows / 64;
+  if (!narrow) {
+    if ((s.images ? filled / 2 : s.heads * s.b128) >= 380) return 1;
+    return blocks >= 400 && blocks <= 512 && (!s.images || filled >= 380) ? 2 : 0;
+  }
+  if (!s.images && s.rows <= 32) return 0;
+  if (blocks >= 400 && blocks <= 512 && filled >= (s.images > 1 ? 470 : 380)) return 2;
+  return blocks >= 680 && filled >= (s.images ? 450 : 700) ? 2 : 0;
 }
 
 template <int DP>
@@ -1554,7 +1589,7 @@ hipError_t launch_vit(const VitArgs& v, AttnArgs a, int64_t slots, hipStream_t s
   hipLaunchKernelGGL(vit_pack_kernel<DP>, dim3(static_cast<unsigned>(slots), static_cast<unsigned>(v.heads)),
                      dim3(256), 0, stream, v);
   const int64_t b64 = seq_slot_count(v.rows, v.num_seqs, 64), b128 = seq_slot_count(v.rows, v.num_seqs, 128);
-  const int groups = shared_groups(false, DP, v.heads, b64, b128);
+  const int groups = shared_groups({false, v.num_seqs, DP, v.heads, v.rows, b64, b128});
   if (groups > 0) {
     a.num_q_blocks = static_cast<int>(groups == 1 ? b128 : b64);
     a.n_work = a.num_q_blocks * v.heads;
@@ -1598,7 +1633,7 @@ void launch_shared(const AttnArgs& a, bool has_bias, dim3 grid, hipStream_t stre
 template <int D, int NSUB, bool kQNorm>
 void launch_attn_d(AttnArgs a, int batch, bool causal, bool has_bias, hipStream_t stream) {
   const int64_t heads = static_cast<int64_t>(a.hq) * batch, b64 = (a.sq + 63) / 64, b128 = (a.sq + 127) / 128;
-  const int groups = shared_groups(causal, D, heads, b64, b128);
+  const int groups = shared_groups({causal, 0, D, heads, a.sq, b64, b128});
   if (groups > 0) a.num_q_blocks = static_cast<int>(groups == 1 ? b128 : b64);
   a.n_work = a.num_q_blocks * a.hq * batch;
   if (groups > 0 && causal) {

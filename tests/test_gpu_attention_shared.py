@@ -50,6 +50,13 @@ def _inputs(B, Hq, Hkv, Sq, Sk, D, bias):
     (2, 32, 32, 400, 545, 64, False, True),
     (4, 32, 16, 333, 290, 64, False, True),      # head_dim 64: also beyond one round of workgroups
     (1, 280, 4, 64, 64, 64, True, False),
+    # either side of the lines for few query rows and partly filled blocks
+    (2, 64, 16, 128, 500, 128, False, True), (1, 400, 80, 33, 70, 128, False, True), (4, 110, 10, 64, 160, 128, False, False),
+    (13, 32, 8, 32, 600, 128, False, False), (20, 32, 8, 1, 290, 128, False, True), (20, 28, 28, 40, 97, 128, False, False),
+    (1, 260, 4, 33, 33, 128, True, False), (1, 220, 4, 64, 64, 128, True, True), (17, 16, 4, 32, 32, 128, True, False),
+    (33, 16, 16, 7, 7, 64, True, False), (24, 16, 8, 50, 50, 64, True, True), (20, 16, 16, 64, 64, 64, True, False),
+    (7, 16, 4, 280, 280, 128, True, True), (1, 260, 4, 70, 70, 64, True, False), (13, 12, 4, 78, 78, 128, True, False),
+    (4, 32, 16, 384, 290, 64, False, True), (8, 28, 28, 79, 97, 64, False, False), (8, 28, 28, 120, 97, 64, False, True),
 ])
 def test_attention_shared_tiles(dev, B, Hq, Hkv, Sq, Sk, D, causal, bias):
     q, k, v, kb = _inputs(B, Hq, Hkv, Sq, Sk, D, bias)
@@ -123,7 +130,8 @@ def test_attention_shared_outputs(dev, B, H, S, D):
     assert torch.equal(packed.unpack(), want)
 
 
-@pytest.mark.parametrize("M,Hq,Hkv,D", [(449, 64, 16, 128), (417, 128, 16, 128), (385, 140, 4, 64), (449, 300, 4, 64), (70, 200, 8, 64)])
+@pytest.mark.parametrize("M,Hq,Hkv,D", [(449, 64, 16, 128), (417, 128, 16, 128), (385, 140, 4, 64), (449, 300, 4, 64), (70, 200, 8, 64), (70, 260, 4, 64),
+                                        (280, 112, 28, 128), (20, 640, 32, 128), (64, 400, 40, 64)])
 def test_gqa_operator_shared_tiles(dev, M, Hq, Hkv, D):
     """The fused Q norm + RoPE of a wave's own rows."""
     inp = W.gqa_inputs(W.GqaCfg(q_heads=Hq, kv_heads=Hkv, head_dim=D, seq=M, seed=M))
@@ -138,6 +146,10 @@ def test_gqa_operator_shared_tiles(dev, M, Hq, Hkv, D):
     ((300, 1, 0, 450, 129), 48, 120), ((300, 1, 0, 450, 129), 24, 72), ((300, 1, 0, 450, 129), 24, 96),
     ((300, 1, 0, 450, 129), 24, 64), ((65, 448, 64), 48, 128),
     (tuple((37 * i) % 50 for i in range(70)), 8, 80),  # binary-search lookup
+    # enough rows, not only blocks, for 128 and 64 queries per workgroup
+    ((300, 1, 0, 450, 129), 64, 72), ((300, 1, 0, 450, 129), 64, 120), ((300, 1, 0, 450, 129), 28, 72),
+    ((300, 1, 0, 450, 129), 28, 96), ((300, 1, 0, 450, 129), 56, 64), ((65, 448, 64), 48, 96), ((65, 700, 64), 32, 64),
+    (tuple((37 * i) % 50 for i in range(70)), 32, 80), (tuple((37 * i) % 50 for i in range(70)), 32, 64),
 ])
 def test_vision_attention_shared_tiles(dev, lengths, H, D):
     inp = W.vit_attention_inputs(W.VitAttnCfg(lengths=lengths, heads=H, head_dim=D, seed=len(lengths) * 100 + D))
