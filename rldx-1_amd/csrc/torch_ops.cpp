@@ -12,11 +12,15 @@
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/Event.h>
 #include <c10/core/GradMode.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
+#include <atomic>
 #include <cmath>
+#include <memory>
 #include <mutex>
 #include <unordered_map>
 #include <vector>
@@ -303,26 +307,40 @@ Tensor swiglu(const Tensor& x) {
 // when the weight dies.  The weak reference keeps the address from being another
 // tensor's meanwhile, and the version, the data pointer, the sizes and the strides
 // must be the packed ones (`w.data = w.data[:rows]` changes the sizes alone).
+// Made: the launch that wrote the copy.  Work on another stream waits for its event; a
+// stream capture takes the copy only when it is complete, because a replay waits for
+// nothing outside its graph.
+struct Made {
+  c10::Event event{c10::DeviceType::CUDA};
+  c10::Stream stream;
+  std::atomic<bool> done{false};
+  explicit Made(c10::Stream s) : stream(s) { event.record(s); }
+};
 struct Packed {
   c10::weak_intrusive_ptr<c10::TensorImpl> w;
   uint32_t version;
   const void* data;
   std::vector<int64_t> sizes, strides;
   Tensor packed;
+  std::shared_ptr<Made> made;  // null: host memory
 };
 std::mutex g_packed_mutex;
 std::unordered_map<int64_t, Packed>& packed_weights() {
   static auto* m = new std::unordered_map<int64_t, Packed>();  // (never destroyed: entries may outlive the runtime's exit)
   return *m;
 }
+c10::Stream current_stream(const Tensor& t) {
+  return c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getStream(t.device());
+}
 int64_t key_of(const Tensor& w) { return reinterpret_cast<int64_t>(w.unsafeGetTensorImpl()); }
 
 void remember_packed(const Tensor& w, const Tensor& packed) {
   if (w.is_inference()) return;  // no version counter
+  Packed p{c10::weak_intrusive_ptr<c10::TensorImpl>(w.getIntrusivePtr()), static_cast<uint32_t>(w._version()),
+           w.data_ptr(), w.sizes().vec(), w.strides().vec(), packed,
+           packed.is_cuda() ? std::make_shared<Made>(current_stream(packed)) : nullptr};
   const std::lock_guard<std::mutex> lock(g_packed_mutex);
-  packed_weights().insert_or_assign(
-      key_of(w), Packed{c10::weak_intrusive_ptr<c10::TensorImpl>(w.getIntrusivePtr()),
-                        static_cast<uint32_t>(w._version()), w.data_ptr(), w.sizes().vec(), w.strides().vec(), packed});
+  packed_weights().insert_or_assign(key_of(w), std::move(p));
 }
 void forget_packed(int64_t key) {
   Tensor drop;  // freed outside the lock
@@ -332,16 +350,40 @@ void forget_packed(int64_t key) {
   drop = std::move(it->second.packed);
   packed_weights().erase(it);
 }
+// Whether work on the current stream can read a copy; makes the stream wait for it where it has to.
+bool readable(const Tensor& packed, Made& m) {
+  const c10::Stream cur = current_stream(packed);
+  if (!m.done) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream_of(packed), &capture) != hipSuccess) return false;
+    {
+      // (a query ends no capture, neither this stream's nor another thread's)
+      c10::hip::HIPStreamCaptureModeGuard relaxed(hipStreamCaptureModeRelaxed);
+      m.done = m.event.query();
+    }
+    if (!m.done && capture != hipStreamCaptureStatusNone) return false;
+    if (!m.done && cur != m.stream) m.event.block(cur);
+  }
+  if (cur != m.stream) packed.record_stream(cur);
+  return true;
+}
 OptTensor packed_of(const Tensor& w) {
   if (w.is_inference()) return std::nullopt;
-  const std::lock_guard<std::mutex> lock(g_packed_mutex);
-  auto it = packed_weights().find(key_of(w));
-  if (it == packed_weights().end()) return std::nullopt;
-  const Packed& p = it->second;
-  if (p.w.expired() || p.data != w.data_ptr() || p.version != static_cast<uint32_t>(w._version()) ||
-      w.sizes() != p.sizes || w.strides() != p.strides)
-    return std::nullopt;
-  return p.packed;
+  Tensor packed;
+  std::shared_ptr<Made> made;
+  {
+    const std::lock_guard<std::mutex> lock(g_packed_mutex);
+    auto it = packed_weights().find(key_of(w));
+    if (it == packed_weights().end()) return std::nullopt;
+    const Packed& p = it->second;
+    if (p.w.expired() || p.data != w.data_ptr() || p.version != static_cast<uint32_t>(w._version()) ||
+        w.sizes() != p.sizes || w.strides() != p.strides)
+      return std::nullopt;
+    packed = p.packed;
+    made = p.made;
+  }
+  if (made && !readable(packed, *made)) return std::nullopt;
+  return packed;
 }
 
 RLDX_OP(Mlp, "ss::fused_mlp_swiglu");

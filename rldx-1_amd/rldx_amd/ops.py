@@ -348,20 +348,50 @@ def _(x):
 # the weight tensor lives; an in-place update of the weight (version change) and
 # storage of another address, shape or strides under the same tensor (w.data = ...,
 # which changes no version) pack it again.
-_packed_weights: dict = {}  # id(weight) -> (weakref to weight, what was packed, PackedWeight)
+_packed_weights: dict = {}  # id(weight) -> _PackedEntry
+
+
+class _PackedEntry:
+    """A packed copy of `ref()` as it was in `state`, written by a launch on `stream` that `event` follows."""
+
+    __slots__ = ("ref", "state", "pw", "stream", "event")
+
+    def __init__(self, w: torch.Tensor, state: tuple, pw: Fn.PackedWeight):
+        self.ref, self.state, self.pw, self.stream = weakref.ref(w), state, pw, None
+        if w.is_cuda:
+            self.stream = torch.cuda.current_stream(w.device)
+            self.event = torch.cuda.Event()
+            self.event.record(self.stream)
+
+    def readable(self, w: torch.Tensor, cur, capturing: bool) -> bool:
+        """Whether work on stream `cur` can read the copy; makes `cur` wait for it where it has to.  A graph
+        takes it only when it is known to be complete: a recorded wait would not outlive the capture."""
+        if _native and self.pw.swiglu_pairs:
+            return torch.ops.rldx_native.packed_of(w) is not None
+        if capturing:
+            return False
+        if cur != self.stream:
+            cur.wait_event(self.event)
+            self.pw.data.record_stream(cur)
+        return True
 
 
 def _packed_weight(w: torch.Tensor, swiglu_pairs: bool) -> Fn.PackedWeight:
     state = (w._version, w.data_ptr(), tuple(w.shape), w.stride(), swiglu_pairs)
+    cur = torch.cuda.current_stream(w.device) if w.is_cuda else None
+    capturing = cur is not None and torch.cuda.is_current_stream_capturing()
     hit = _packed_weights.get(id(w))
-    if hit is not None and hit[0]() is w and hit[1] == state:
-        return hit[2]
+    hit = hit if hit is not None and hit.ref() is w else None
+    if hit is not None and hit.state == state and hit.readable(w, cur, capturing):
+        return hit.pw
     pw = Fn.pack_weight(w if w.stride(1) == 1 else w.contiguous(), swiglu_pairs=swiglu_pairs, row_sums=False)
-    if hit is None or hit[0]() is not w:
+    if capturing:  # only recorded: the graph packs at each replay, and nobody else may read this copy
+        return pw
+    if hit is None:
         weakref.finalize(w, _packed_weights.pop, id(w), None)
         if _native:
             weakref.finalize(w, torch.ops.rldx_native.forget_packed, int(w._cdata)).atexit = False
-    _packed_weights[id(w)] = (weakref.ref(w), state, pw)
+    _packed_weights[id(w)] = _PackedEntry(w, state, pw)
     if _native and swiglu_pairs:
         torch.ops.rldx_native.remember_packed(w, pw.data)
     return pw

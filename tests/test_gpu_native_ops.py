@@ -147,3 +147,80 @@ def test_mlp_weight_updates_and_lifetime(dev):
     gc.collect()
     assert torch.cuda.memory_allocated() < before  # the weight and its packed copy are both freed
     assert len(ops._packed_weights) <= n
+
+
+def _busy(dev, seconds=0.02):
+    """Work that keeps the current stream busy for a while (bf16 products of about 0.1 ms each)."""
+    a = torch.ones(4096, 4096, dtype=BF16, device=dev)
+    for _ in range(int(seconds / 1e-4)):
+        a @ a
+
+
+def test_mlp_weight_packed_on_another_stream(dev):
+    """A copy that one stream is still to pack is waited for by the stream that finds it."""
+    op, impl, (x, _, b) = _calls(dev)["mlp"]
+    one, two = torch.cuda.Stream(), torch.cuda.Stream()
+    for trial in range(3):
+        w = _rnd(dev, 128, 128, seed=40 + trial)
+        want, want2 = (impl._init_fn(x, w.clone(), b, n) for n in (1, 2))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(one):
+            _busy(dev)
+            first = op(x, w, b)
+        with torch.cuda.stream(two):
+            second = op(x, w, b)
+            split = op(x, w, b, 2)  # (the Python path)
+        torch.cuda.synchronize()
+        _same(first, want)
+        _same(second, want)
+        _same(split, want2)
+
+
+@pytest.mark.parametrize("split", [1, 2])
+def test_mlp_weight_packed_in_a_capture(dev, split):
+    """The first call with a weight inside a capture only records its packing: calls before
+    the first replay, other graphs and later updates of the weight are right all the same."""
+    op, impl, (x, _, b) = _calls(dev)["mlp"]
+    x = x.contiguous()
+    w = _rnd(dev, 128, 128, seed=50)
+    op(x, w.clone(), b, split)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = op(x, w, b, split)
+    _same(op(x, w, b, split), impl._init_fn(x, w.clone(), b, split))  # before any replay
+    for step in range(4):
+        x.copy_(_rnd(dev, 19, 128, seed=60 + step))
+        if step == 2:
+            w.mul_(0.5)
+        graph.replay()
+        want = impl._init_fn(x, w.clone(), b, split)
+        _same(out, want)
+        _same(op(x, w, b, split), want)
+
+
+def test_mlp_weight_packed_before_a_capture(dev):
+    """A capture takes a copy that is complete, and packs for itself beside one that is not."""
+    op, impl, (x, _, b) = _calls(dev)["mlp"]
+    x = x.contiguous()
+    for busy in (False, True):
+        w = _rnd(dev, 128, 128, seed=70 + busy)
+        side = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        graph, capture = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        op(x, _rnd(dev, 128, 128, seed=80), b)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            if busy:
+                _busy(dev)
+            op(x, w, b)
+        if not busy:
+            torch.cuda.synchronize()
+        with torch.cuda.stream(capture):
+            graph.capture_begin()
+            out = op(x, w, b)
+            graph.capture_end()
+            graph.replay()
+        capture.synchronize()
+        _same(out.clone(), impl._init_fn(x, w.clone(), b))
+        torch.cuda.synchronize()
