@@ -339,15 +339,19 @@ void remember_packed(const Tensor& w, const Tensor& packed) {
   Packed p{c10::weak_intrusive_ptr<c10::TensorImpl>(w.getIntrusivePtr()), static_cast<uint32_t>(w._version()),
            w.data_ptr(), w.sizes().vec(), w.strides().vec(), packed,
            packed.is_cuda() ? std::make_shared<Made>(current_stream(packed)) : nullptr};
+  std::optional<Packed> old;  // freed outside the lock: the last reference to a tensor of Python's takes the GIL
   const std::lock_guard<std::mutex> lock(g_packed_mutex);
-  packed_weights().insert_or_assign(key_of(w), std::move(p));
+  auto [it, inserted] = packed_weights().try_emplace(key_of(w), std::move(p));
+  if (inserted) return;
+  old.emplace(std::move(it->second));
+  it->second = std::move(p);
 }
 void forget_packed(int64_t key) {
-  Tensor drop;  // freed outside the lock
+  std::optional<Packed> old;  // freed outside the lock, as above
   const std::lock_guard<std::mutex> lock(g_packed_mutex);
   auto it = packed_weights().find(key);
   if (it == packed_weights().end()) return;
-  drop = std::move(it->second.packed);
+  old.emplace(std::move(it->second));
   packed_weights().erase(it);
 }
 // Whether work on the current stream can read a copy; makes the stream wait for it where it has to.

@@ -1,6 +1,11 @@
 """Host tests of the packed-weight cache of ss::fused_mlp_swiglu (rldx_amd/ops.py and its
 copy in csrc/torch_ops.cpp): a packed copy serves a weight only as it was when packed."""
 
+import os
+import subprocess
+import sys
+from pathlib import Path
+
 import pytest
 import torch
 
@@ -70,3 +75,30 @@ def test_native_copy_serves_the_packed_shape_only():
     finally:
         native.forget_packed(int(w._cdata))
     assert native.packed_of(w) is None
+
+
+_LOCK_ORDER = """
+import threading, torch
+import rldx_amd.ops
+native = torch.ops.rldx_native
+w = torch.zeros(64, 64, dtype=torch.bfloat16)
+
+class Noted(torch.Tensor):  # a Python object whose end runs Python code
+    def __del__(self):
+        for _ in range(1000):
+            native.packed_of(w)
+
+for _ in range(200):
+    native.remember_packed(w, torch.zeros(64 * 64, dtype=torch.bfloat16).as_subclass(Noted))
+native.forget_packed(int(w._cdata))
+print("done")
+"""
+
+
+@pytest.mark.skipif(not ops._native, reason="librldx_torch.so was not built")
+def test_replaced_copies_are_freed_outside_the_lock():
+    """A packed tensor may be Python's last one, and its end may run Python code that calls
+    the operator again: with the table's lock held that would never return."""
+    env = {**os.environ, "PYTHONPATH": str(Path(ops.__file__).resolve().parents[1])}
+    r = subprocess.run([sys.executable, "-c", _LOCK_ORDER], env=env, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.strip() == "done", r.stderr[-2000:]
