@@ -641,15 +641,20 @@ class PackedWeight:
         self.data, self.n, self.k, self.swiglu_pairs, self.row_sums = data, n, k, swiglu_pairs, row_sums
 
 
-def pack_weight(w: torch.Tensor, swiglu_pairs: bool = False, row_sums: bool = True) -> PackedWeight:
+def pack_weight(w: torch.Tensor, swiglu_pairs: bool = False, row_sums: bool = True,
+                out: Optional[torch.Tensor] = None) -> PackedWeight:
     """nn.Linear weight [out_features, in_features] bf16 -> PackedWeight.  With
     swiglu_pairs, w = [gate; up] and the GEMM's SwiGLU epilogue can be used.
-    row_sums=False leaves out the sums that only the LayerNorm fold reads."""
+    row_sums=False leaves out the sums that only the LayerNorm fold reads.  out:
+    the data of a PackedWeight of this shape, written in place."""
     _on_gpu(w)
     _require(w.dtype == BF16 and w.dim() == 2 and w.stride(1) == 1, "weight must be 2-D bf16, rows contiguous")
     n, k = w.shape
     _require(n % (64 if swiglu_pairs else 32) == 0 and k % 16 == 0, "weight shape not tileable")
-    out = torch.empty(n * k, dtype=BF16, device=w.device)
+    if out is None:
+        out = torch.empty(n * k, dtype=BF16, device=w.device)
+    _on_gpu(w, out)
+    _require(out.dtype == BF16 and out.numel() == n * k and out.is_contiguous(), "out must hold the packed weight")
     lib = _lib.load()
     _lib.check(lib.rldx_gemm_pack_weight_bf16(w.data_ptr(), w.stride(0), n, k, int(swiglu_pairs), out.data_ptr(),
                                               _stream_ptr(w)), "rldx_gemm_pack_weight_bf16")

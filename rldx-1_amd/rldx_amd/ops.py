@@ -345,9 +345,10 @@ def _(x):
 # ---------------------------------------------------------------------------
 # The grouped GEMM reads weights in its packed operand order.  Weights are
 # static, so each one is packed once and the packed copy is kept for as long as
-# the weight tensor lives; an in-place update of the weight (version change) and
-# storage of another address, shape or strides under the same tensor (w.data = ...,
-# which changes no version) pack it again.
+# the weight tensor lives; an in-place update of the weight (version change) packs
+# it again, over the same memory (a captured graph takes the update with the next
+# call outside it); so does storage of another address, shape or strides under the
+# same tensor (w.data = ..., which changes no version), into memory of its own.
 _packed_weights: dict = {}  # id(weight) -> _PackedEntry
 
 
@@ -384,7 +385,15 @@ def _packed_weight(w: torch.Tensor, swiglu_pairs: bool) -> Fn.PackedWeight:
     hit = hit if hit is not None and hit.ref() is w else None
     if hit is not None and hit.state == state and hit.readable(w, cur, capturing):
         return hit.pw
-    pw = Fn.pack_weight(w if w.stride(1) == 1 else w.contiguous(), swiglu_pairs=swiglu_pairs, row_sums=False)
+    old = None
+    if hit is not None and not capturing and hit.state[1:] == state[1:]:
+        # updated in place: written over the old copy, whose address captured graphs hold.  The update came after
+        # every earlier call in stream order, and this call after the update.
+        old = hit.pw.data
+        if cur is not None and cur != hit.stream:
+            cur.wait_event(hit.event)
+            old.record_stream(cur)
+    pw = Fn.pack_weight(w if w.stride(1) == 1 else w.contiguous(), swiglu_pairs=swiglu_pairs, row_sums=False, out=old)
     if capturing:  # only recorded: the graph packs at each replay, and nobody else may read this copy
         return pw
     if hit is None:

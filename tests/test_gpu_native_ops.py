@@ -199,6 +199,28 @@ def test_mlp_weight_packed_in_a_capture(dev, split):
         _same(op(x, w, b, split), want)
 
 
+def test_mlp_weight_updated_after_a_capture(dev):
+    """A graph that reads a weight's packed copy: after an in-place update and one call
+    outside the graph its replays see the new weight."""
+    op, impl, (x, _, b) = _calls(dev)["mlp"]
+    x = x.contiguous()
+    w = _rnd(dev, 128, 128, seed=90)
+    op(x, w, b)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = op(x, w, b)
+    for step in range(4):
+        x.copy_(_rnd(dev, 19, 128, seed=91 + step))
+        w.mul_(0.75)
+        want = impl._init_fn(x, w.clone(), b)
+        _same(op(x, w, b), want)
+        junk = [torch.full((128 * 128,), 7.0, dtype=BF16, device=dev) for _ in range(4)]  # memory a freed copy would give
+        graph.replay()
+        _same(out, want)
+        del junk
+
+
 def test_mlp_weight_packed_before_a_capture(dev):
     """A capture takes a copy that is complete, and packs for itself beside one that is not."""
     op, impl, (x, _, b) = _calls(dev)["mlp"]

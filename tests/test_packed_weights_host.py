@@ -20,9 +20,10 @@ def packs(monkeypatch):
     """pack_weight without a GPU: the packed copy is a copy; the list holds the weights' shapes as packed."""
     seen = []
 
-    def pack(w, swiglu_pairs=False, row_sums=True):
+    def pack(w, swiglu_pairs=False, row_sums=True, out=None):
         seen.append(tuple(w.shape))
-        return Fn.PackedWeight(w.clone().reshape(-1), *w.shape, swiglu_pairs)
+        data = torch.empty(w.numel(), dtype=BF16) if out is None else out
+        return Fn.PackedWeight(data.copy_(w.reshape(-1)), *w.shape, swiglu_pairs)
 
     monkeypatch.setattr(Fn, "pack_weight", pack)
     return seen
@@ -46,6 +47,19 @@ def test_storage_of_another_shape_is_packed_again(packs, change):
     after = ops._packed_weight(w, True)
     assert after is not before and (after.n, after.k) == tuple(w.shape)
     assert torch.equal(after.data.view(w.shape), w) and len(packs) == 2
+
+
+def test_update_in_place_is_packed_over_the_old_copy(packs):
+    """A captured graph holds the copy's address: it must stay the copy of this weight."""
+    w = _w(128, 128)
+    before = ops._packed_weight(w, True)
+    address = before.data.data_ptr()
+    w.mul_(0.5)
+    after = ops._packed_weight(w, True)
+    assert after.data.data_ptr() == address and len(packs) == 2
+    assert torch.equal(after.data.view(w.shape), w)
+    w.data = w.data.clone()  # other storage, to which nobody ordered the old copy's readers
+    assert ops._packed_weight(w, True).data.data_ptr() != address and len(packs) == 3
 
 
 def test_storage_grown_in_place_is_packed_again(packs):
