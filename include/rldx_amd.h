@@ -534,10 +534,12 @@ hipError_t rldx_copy_rows_many(const rldx_copy_rows_t* copies, int32_t count, in
 
 /*
  * dst[i][b] = src[i][idx[b]] for up to 16 stacked parameters of num_slabs slabs of
- * slab_bytes[i] bytes each (multiples of 16) and batch ids idx (device memory), one
- * launch: the per-embodiment weights W[e], b[e] of CategorySpecificLinear
+ * slab_bytes[i] bytes each (multiples of 2; pointers and sizes that are multiples of 16
+ * go in 16-byte pieces) and batch ids idx (device memory), one launch: the
+ * per-embodiment weights W[e], b[e] of CategorySpecificLinear
  * (rldx/model/modules/action_model/embodiment_conditioned_mlp.py:72-82).  An id
- * outside [0, num_slabs) copies nothing.
+ * outside [0, num_slabs) reads nothing and fills its slabs with bytes 0xff: NaN in every
+ * floating-point type, so that what is computed with them cannot pass for a result.
  */
 hipError_t rldx_gather_slabs(const void* const* src, void* const* dst, const int64_t* slab_bytes, int32_t count,
                              const int64_t* idx, int64_t batch, int64_t num_slabs, hipStream_t stream);

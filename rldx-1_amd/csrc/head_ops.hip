@@ -60,32 +60,46 @@ __global__ __launch_bounds__(256) void copy_rows_kernel(CopyArgs a) {
 struct SlabArgs {
   const char* src[kMaxSlabs];
   char* dst[kMaxSlabs];
-  int64_t units[kMaxSlabs];  // 16-byte units per slab
+  int64_t units[kMaxSlabs];  // units per slab
   int begin[kMaxSlabs + 1];
+  uint32_t narrow;           // bit i: units of 2 bytes (a bias of 7 actions: 14), else of 16
   const int64_t* idx;
   int64_t num;
   int count;
 };
 
+// piece `piece` of slab e of src -> slab b of dst; e < 0: bytes 0xff, NaN in every floating-point type
+template <class T>
+__device__ __forceinline__ void gather_piece(const char* src, char* dst, int64_t units, int64_t e, int64_t b, int piece,
+                                             T nan) {
+  const T* s = reinterpret_cast<const T*>(src) + e * units;
+  T* d = reinterpret_cast<T*>(dst) + b * units;
+  const int64_t base = static_cast<int64_t>(piece) * kPiece + threadIdx.x;
+  T v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int64_t u = base + 256 * j;
+    v[j] = nan;
+    if (e >= 0) v[j] = s[u < units ? u : units - 1];
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (base + 256 * j < units) d[base + 256 * j] = v[j];
+}
+
 __global__ __launch_bounds__(256) void gather_slabs_kernel(SlabArgs a) {
   int i = 0;
   for (int c = 1; c < a.count; ++c)
     if (static_cast<int>(blockIdx.x) >= a.begin[c]) i = c;
-  const int64_t b = blockIdx.y, e = a.idx[b];
-  if (e < 0 || e >= a.num) return;  // (the host checks the ids; never read outside the stack)
-  const int64_t units = a.units[i];
-  const u32x4* src = reinterpret_cast<const u32x4*>(a.src[i]) + e * units;
-  u32x4* dst = reinterpret_cast<u32x4*>(a.dst[i]) + b * units;
-  const int64_t base = static_cast<int64_t>(static_cast<int>(blockIdx.x) - a.begin[i]) * kPiece + threadIdx.x;
-  u32x4 v[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int64_t u = base + 256 * j;
-    v[j] = src[u < units ? u : units - 1];
-  }
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    if (base + 256 * j < units) dst[base + 256 * j] = v[j];
+  const int64_t b = blockIdx.y;
+  int64_t e = a.idx[b];
+  // (a bad id reads nothing, and the robot's weights become NaN: the previous robot's would pass for its own)
+  if (e < 0 || e >= a.num) e = -1;
+  const int piece = static_cast<int>(blockIdx.x) - a.begin[i];
+  if (a.narrow >> i & 1u)
+    gather_piece<uint16_t>(a.src[i], a.dst[i], a.units[i], e, b, piece, 0xffff);
+  else
+    gather_piece<u32x4>(a.src[i], a.dst[i], a.units[i], e, b, piece, u32x4{~0u, ~0u, ~0u, ~0u});
 }
 
 // One wave per row; lane j holds columns 8 (j + 64 c) .. +7.  LayerNorm without
@@ -206,12 +220,15 @@ extern "C" hipError_t rldx_gather_slabs(const void* const* src, void* const* dst
   int n = 0;
   int64_t blocks = 0;
   for (int i = 0; i < count; ++i) {
-    if (slab_bytes[i] < 0 || slab_bytes[i] % 16) return hipErrorInvalidValue;
+    if (slab_bytes[i] < 0 || slab_bytes[i] % 2) return hipErrorInvalidValue;
     if (slab_bytes[i] == 0) continue;
-    if (!src[i] || !dst[i] || !a16(src[i]) || !a16(dst[i])) return hipErrorInvalidValue;
+    if (!src[i] || !dst[i] || reinterpret_cast<uintptr_t>(src[i]) % 2 || reinterpret_cast<uintptr_t>(dst[i]) % 2)
+      return hipErrorInvalidValue;
+    const bool wide = slab_bytes[i] % 16 == 0 && a16(src[i]) && a16(dst[i]);
     a.src[n] = static_cast<const char*>(src[i]);
     a.dst[n] = static_cast<char*>(dst[i]);
-    a.units[n] = slab_bytes[i] / 16;
+    a.units[n] = slab_bytes[i] / (wide ? 16 : 2);
+    if (!wide) a.narrow |= 1u << n;
     a.begin[n] = static_cast<int>(blocks);
     blocks += (a.units[n] + kPiece - 1) / kPiece;
     if (blocks > (1 << 30)) return hipErrorInvalidValue;

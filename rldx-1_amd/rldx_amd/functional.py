@@ -878,7 +878,8 @@ def copy_rows_many(pairs: Sequence[tuple]) -> None:
 
 def gather_slabs(pairs: Sequence[tuple], idx: torch.Tensor) -> None:
     """out[b] = stack[idx[b]] of up to 16 (stack [E, ...], out [B, ...]) pairs in one
-    launch (rldx_gather_slabs); a pair the kernel does not take goes to torch.index_select."""
+    launch (rldx_gather_slabs; an id outside [0, E) makes out[b] NaN); a pair the kernel
+    does not take (strided, or slabs of an odd number of bytes) goes to torch.index_select."""
     _require(1 <= len(pairs) <= 16, "between 1 and 16 stacks")
     _require(idx.dtype == torch.int64 and idx.dim() == 1 and idx.is_contiguous(), "idx must be contiguous int64 [B]")
     _on_gpu(idx)
@@ -887,10 +888,10 @@ def gather_slabs(pairs: Sequence[tuple], idx: torch.Tensor) -> None:
         _require(stack.dtype == out.dtype and out.shape[0] == idx.numel() and out[0].numel() == stack[0].numel(),
                  "stacks [E, ...] and outs [B, ...] of one slab shape")
         if (stack.shape[0] == E and stack.device == out.device == idx.device and stack.is_contiguous() and
-                out.is_contiguous() and stack[0].numel() * stack.element_size() % 16 == 0 and
-                stack.data_ptr() % 16 == 0 and out.data_ptr() % 16 == 0):
+                out.is_contiguous() and stack[0].numel() * stack.element_size() % 2 == 0 and
+                stack.data_ptr() % 2 == 0 and out.data_ptr() % 2 == 0):
             take.append((stack, out))
-        else:  # (a bias of 7 actions: 14-byte slabs)
+        else:
             torch.index_select(stack, 0, idx, out=out.view(idx.numel(), *stack.shape[1:]))
     if not take:
         return

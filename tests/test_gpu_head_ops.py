@@ -38,18 +38,23 @@ def test_copy_rows_many(batch):
 
 @pytest.mark.parametrize("ids", [[2], [0, 4, 4]])
 def test_gather_slabs(ids):
-    """Slabs of one unit, of 1024 units and of one more, and one of 14 bytes (torch's
-    index_select); an id outside the stacks copies nothing."""
+    """Slabs of one unit, of 1024 units and of one more, and in 2-byte units: one of 14
+    bytes, one of 1025 units, one that is not 16-byte aligned; a strided stack takes
+    torch's index_select.  An id outside the stacks makes its slabs NaN and leaves the
+    other robots' right, whatever was there before."""
     idx = torch.tensor(ids, device="cuda")
-    stacks = [rnd(5, 8, seed=1), rnd(5, 64, 128, seed=2), rnd(5, 8200, seed=3), rnd(5, 7, seed=4)]
-    outs = [torch.zeros(len(ids), 1, *s.shape[1:], dtype=BF16, device="cuda") for s in stacks]
+    stacks = [rnd(5, 8, seed=1), rnd(5, 64, 128, seed=2), rnd(5, 8200, seed=3), rnd(5, 7, seed=4), rnd(5, 1025, seed=5),
+              rnd(1 + 5 * 16, seed=6)[1:].view(5, 16), rnd(5, 6, dtype=torch.float32, seed=7), rnd(10, 40, seed=8)[::2]]
+    outs = [torch.zeros(len(ids), 1, *s.shape[1:], dtype=s.dtype, device="cuda") for s in stacks]
     Fn.gather_slabs(list(zip(stacks, outs)), idx)
     for s, o in zip(stacks, outs):
         assert torch.equal(o[:, 0], s[idx])
-    kept = outs[1].clone()
-    Fn.gather_slabs([(stacks[1], outs[1])], idx * 0 + 5)
-    Fn.gather_slabs([(stacks[1], outs[1])], idx * 0 - 1)
-    assert torch.equal(outs[1], kept)
+    for bad in (5, -1, 2**40):
+        mixed = idx.clone()
+        mixed[0] = bad
+        Fn.gather_slabs(list(zip(stacks, outs))[:-1], mixed)
+        for s, o in zip(stacks[:-1], outs):
+            assert bool(torch.isnan(o[0]).all()) and torch.equal(o[1:, 0], s[idx[1:]])
 
 
 @pytest.mark.parametrize("batch,rows,d", [(1, 1, 16), (1, 17, 1536), (3, 31, 1040), (2, 33, 2064), (1, 3, 8192)])
