@@ -545,16 +545,15 @@ hipError_t rldx_gather_slabs(const void* const* src, void* const* dst, const int
                              const int64_t* idx, int64_t batch, int64_t num_slabs, hipStream_t stream);
 
 /*
- * packed [batch rows, d] (packed activation order) = LN(x) (1 + scale) + shift:
- * LayerNorm without affine parameters, then bf16(1 + scale), the product and the sum
- * each rounded to bf16 (MSAT._output_projection,
- * rldx/model/modules/action_model/msat.py:777-781).  x: rows of `batch` entries
- * (strides in elements, % 8), shift / scale [batch, d] with one batch stride (% 8);
- * d % 16 == 0, d <= 8192.
+ * packed [batch rows, d] (packed activation order) = x (1 + scale) + shift:
+ * bf16(1 + scale), the product and the sum each rounded to bf16 (the modulation of
+ * MSAT._output_projection, rldx/model/modules/action_model/msat.py:777-781, on the
+ * normalised rows).  x: rows of `batch` entries (strides in elements, % 8), shift / scale
+ * [batch, d] with one batch stride (% 8); d % 16 == 0.
  */
-hipError_t rldx_adaln_pack_bf16(const void* x, int64_t x_row_stride, int64_t x_batch_stride, int64_t rows,
-                                int64_t batch, const void* shift, const void* scale, int64_t mod_batch_stride,
-                                int64_t d, float eps, void* packed, hipStream_t stream);
+hipError_t rldx_modulate_pack_bf16(const void* x, int64_t x_row_stride, int64_t x_batch_stride, int64_t rows,
+                                   int64_t batch, const void* shift, const void* scale, int64_t mod_batch_stride,
+                                   int64_t d, void* packed, hipStream_t stream);
 
 /* One stream of a grouped GEMM. */
 typedef struct rldx_gemm_group {

@@ -1,17 +1,19 @@
 // The small data movements of the action head around the MSAT blocks, one launch
 // where the eager chain has several.  Each torch launch there runs 4-5 us of a
-// captured graph on a few hundred KB: latency, not bandwidth, so the win is the
-// number of launches:
-// an action of 4 steps at the release shape took 4.740 ms with the 14 index_selects,
-// 12 copies and 16 modulation launches they replace, 4.617 ms now (bits unchanged).
-// Row and slab pieces are 16 KB per workgroup (4 loads of 16 bytes in flight per
-// thread): below the size of every operand there, so each launch covers the chip.
+// captured graph on a few KB to a few hundred KB: latency, not bandwidth, so the win is
+// the number of launches: an action of 4 steps at the release shape took 4.740 ms with
+// the 14 index_selects, 12 copies and 12 modulation launches they replace, 4.64 ms now,
+// with the same bits: everything here copies, or rounds where the eager chain does.
+// A workgroup copies 16 KB of rows or slabs (4 loads of 16 bytes in flight per thread):
+// 37 workgroups for a step's inputs, about 1250 for an embodiment's weights.
 //   * copy_rows_many: up to 4 strided row blocks (time token, SA and VL inputs of a
 //     denoising step into the chain's buffers);
 //   * gather_slabs: slab idx[b] of up to 16 stacked parameters (the embodiment's
 //     encoder / decoder weights) into per-robot buffers;
-//   * adaln_pack: the output modulation LN(x) (1 + scale) + shift and the packing of
-//     its rows for the output projection.
+//   * modulate_pack: the output modulation LN(x) (1 + scale) + shift of normalised rows
+//     and their packing for the output projection.  (The LayerNorm stays torch's: one
+//     in this kernel adds in another order, and a value that rounds the other way in an
+//     early denoising step shows in the action.)
 #include "rldx_amd.h"
 #include "rldx_common.h"
 
@@ -102,74 +104,32 @@ __global__ __launch_bounds__(256) void gather_slabs_kernel(SlabArgs a) {
     gather_piece<u32x4>(a.src[i], a.dst[i], a.units[i], e, b, piece, u32x4{~0u, ~0u, ~0u, ~0u});
 }
 
-// One wave per row; lane j holds columns 8 (j + 64 c) .. +7.  LayerNorm without
-// affine parameters as rows_pack_kernel (two passes in registers, one rounding),
-// then bf16(1 + scale), the product and the sum, each rounded, as the eager chain.
-struct AdalnArgs {
+// One thread per 8 columns: bf16(1 + scale), the product and the sum, each rounded, as the eager chain.
+struct ModulateArgs {
   const uint16_t* x;
   const uint16_t *shift, *scale;
   uint16_t* out;
   int64_t x_row, x_batch, mod_batch;
-  int rows, batch, d;
-  float eps;
+  int rows, total, d;  // total: 8-column pieces
 };
 
-template <int CPL>
-__global__ __launch_bounds__(256) void adaln_pack_kernel(AdalnArgs a) {
+__global__ __launch_bounds__(256) void modulate_pack_kernel(ModulateArgs a) {
 #pragma clang fp contract(off)
-  const int lane = threadIdx.x & 63;
-  const int t = static_cast<int>(blockIdx.x) * 4 + (threadIdx.x >> 6);  // row of the packed output
-  if (t >= a.rows * a.batch) return;
-  const int b = t / a.rows, r = t - b * a.rows, d = a.d;
-  const uint16_t* xr = a.x + b * a.x_batch + r * a.x_row;
-  const uint16_t* sh = a.shift + b * a.mod_batch;
-  const uint16_t* sc = a.scale + b * a.mod_batch;
-  const u32x4 z = {0, 0, 0, 0};
-  u32x4 raw[CPL], shv[CPL], scv[CPL];
-  float sum = 0.f;
+  const int p = static_cast<int>(blockIdx.x) * 256 + static_cast<int>(threadIdx.x);
+  if (p >= a.total) return;
+  const int per = a.d / 8, t = p / per, col = (p - t * per) * 8;  // t: row of the packed output
+  const int b = t / a.rows, r = t - b * a.rows;
+  const u32x4 x = *reinterpret_cast<const u32x4*>(a.x + b * a.x_batch + r * a.x_row + col);
+  const u32x4 sh = *reinterpret_cast<const u32x4*>(a.shift + b * a.mod_batch + col);
+  const u32x4 sc = *reinterpret_cast<const u32x4*>(a.scale + b * a.mod_batch + col);
+  u32x4 o;
 #pragma unroll
-  for (int c = 0; c < CPL; ++c) {
-    const int col = 8 * (lane + 64 * c);
-    raw[c] = col < d ? *reinterpret_cast<const u32x4*>(xr + col) : z;
-    shv[c] = col < d ? *reinterpret_cast<const u32x4*>(sh + col) : z;
-    scv[c] = col < d ? *reinterpret_cast<const u32x4*>(sc + col) : z;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      sum += bf16x2_lo(raw[c][i]);
-      sum += bf16x2_hi(raw[c][i]);
-    }
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t s1 = pack_bf16x2(1.0f + bf16x2_lo(sc[i]), 1.0f + bf16x2_hi(sc[i]));
+    const uint32_t m = pack_bf16x2(bf16x2_lo(x[i]) * bf16x2_lo(s1), bf16x2_hi(x[i]) * bf16x2_hi(s1));
+    o[i] = pack_bf16x2(bf16x2_lo(m) + bf16x2_lo(sh[i]), bf16x2_hi(m) + bf16x2_hi(sh[i]));
   }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
-  const float mean = sum / static_cast<float>(d);
-  float sq = 0.f;
-#pragma unroll
-  for (int c = 0; c < CPL; ++c)
-    if (8 * (lane + 64 * c) < d) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float lo = bf16x2_lo(raw[c][i]) - mean, hi = bf16x2_hi(raw[c][i]) - mean;
-        sq += lo * lo;
-        sq += hi * hi;
-      }
-    }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) sq += __shfl_xor(sq, o, 64);
-  const float rstd = 1.0f / __builtin_sqrtf(sq / static_cast<float>(d) + a.eps);
-#pragma unroll
-  for (int c = 0; c < CPL; ++c) {
-    const int col = 8 * (lane + 64 * c);
-    if (col >= d) continue;
-    u32x4 o;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t y = pack_bf16x2((bf16x2_lo(raw[c][i]) - mean) * rstd, (bf16x2_hi(raw[c][i]) - mean) * rstd);
-      const uint32_t s1 = pack_bf16x2(1.0f + bf16x2_lo(scv[c][i]), 1.0f + bf16x2_hi(scv[c][i]));
-      const uint32_t p = pack_bf16x2(bf16x2_lo(y) * bf16x2_lo(s1), bf16x2_hi(y) * bf16x2_hi(s1));
-      o[i] = pack_bf16x2(bf16x2_lo(p) + bf16x2_lo(shv[c][i]), bf16x2_hi(p) + bf16x2_hi(shv[c][i]));
-    }
-    *reinterpret_cast<u32x4*>(a.out + packed_act_offset(t, col, d)) = o;
-  }
+  *reinterpret_cast<u32x4*>(a.out + packed_act_offset(t, col, a.d)) = o;
 }
 
 }  // namespace
@@ -244,29 +204,25 @@ extern "C" hipError_t rldx_gather_slabs(const void* const* src, void* const* dst
   return hipGetLastError();
 }
 
-extern "C" hipError_t rldx_adaln_pack_bf16(const void* x, int64_t x_row_stride, int64_t x_batch_stride, int64_t rows,
-                                           int64_t batch, const void* shift, const void* scale,
-                                           int64_t mod_batch_stride, int64_t d, float eps, void* packed,
-                                           hipStream_t stream) {
-  if (rows < 0 || batch < 0 || d < 0 || !(eps >= 0.f)) return hipErrorInvalidValue;
+extern "C" hipError_t rldx_modulate_pack_bf16(const void* x, int64_t x_row_stride, int64_t x_batch_stride, int64_t rows,
+                                              int64_t batch, const void* shift, const void* scale,
+                                              int64_t mod_batch_stride, int64_t d, void* packed, hipStream_t stream) {
+  if (rows < 0 || batch < 0 || d < 0) return hipErrorInvalidValue;
   if (rows == 0 || batch == 0 || d == 0) return hipSuccess;
   if (!x || !shift || !scale || !packed || !a16(x) || !a16(shift) || !a16(scale) || !a16(packed) || x_row_stride % 8 ||
-      x_batch_stride % 8 || mod_batch_stride % 8 || d % 16 || d > 8192 || rows * batch > (1 << 28))
+      x_batch_stride % 8 || mod_batch_stride % 8 || d % 16 || d > (1 << 24) || rows > (1 << 24) || batch > (1 << 24) ||
+      rows * batch > (1 << 28) || rows * batch * (d / 8) > (1 << 30))
     return hipErrorInvalidValue;
-  const AdalnArgs a{static_cast<const uint16_t*>(x),     static_cast<const uint16_t*>(shift),
-                    static_cast<const uint16_t*>(scale), static_cast<uint16_t*>(packed),
-                    x_row_stride,                        x_batch_stride,
-                    mod_batch_stride,                    static_cast<int>(rows),
-                    static_cast<int>(batch),             static_cast<int>(d),
-                    eps};
-  const dim3 grid(static_cast<unsigned>((rows * batch + 3) / 4)), block(256);
-  if (d <= 1024)
-    hipLaunchKernelGGL(adaln_pack_kernel<2>, grid, block, 0, stream, a);
-  else if (d <= 2048)
-    hipLaunchKernelGGL(adaln_pack_kernel<4>, grid, block, 0, stream, a);
-  else if (d <= 4096)
-    hipLaunchKernelGGL(adaln_pack_kernel<8>, grid, block, 0, stream, a);
-  else
-    hipLaunchKernelGGL(adaln_pack_kernel<16>, grid, block, 0, stream, a);
+  const ModulateArgs a{static_cast<const uint16_t*>(x),
+                       static_cast<const uint16_t*>(shift),
+                       static_cast<const uint16_t*>(scale),
+                       static_cast<uint16_t*>(packed),
+                       x_row_stride,
+                       x_batch_stride,
+                       mod_batch_stride,
+                       static_cast<int>(rows),
+                       static_cast<int>(rows * batch * (d / 8)),
+                       static_cast<int>(d)};
+  hipLaunchKernelGGL(modulate_pack_kernel, dim3(static_cast<unsigned>((a.total + 255) / 256)), dim3(256), 0, stream, a);
   return hipGetLastError();
 }

@@ -160,7 +160,7 @@ SIGNATURES = {
     "rldx_action_decode_euler_bf16": (c_i32, [c_vp, c_i64, c_i64, c_f32, c_vp, c_vp, c_i64, c_f32, c_vp, c_vp]),
     "rldx_copy_rows_many": (c_i32, [ctypes.POINTER(CopyRows), c_i32, c_i64, c_vp]),
     "rldx_gather_slabs": (c_i32, [ctypes.POINTER(c_vp), ctypes.POINTER(c_vp), c_i64p, c_i32, c_vp, c_i64, c_i64, c_vp]),
-    "rldx_adaln_pack_bf16": (c_i32, [c_vp, c_i64, c_i64, c_i64, c_i64, c_vp, c_vp, c_i64, c_i64, c_f32, c_vp, c_vp]),
+    "rldx_modulate_pack_bf16": (c_i32, [c_vp, c_i64, c_i64, c_i64, c_i64, c_vp, c_vp, c_i64, c_i64, c_vp, c_vp]),
     "rldx_grouped_gemm_mixed_bf16": (c_i32, [ctypes.POINTER(GemmGroup), c_i64p, c_i64p, ctypes.POINTER(c_i32),
                                              ctypes.POINTER(c_vp), c_i32, c_i32, c_i32, c_vp, c_i64, c_vp]),
     "rldx_grouped_gemm_mixed_workspace_bytes": (c_i64, [ctypes.POINTER(GemmGroup), c_i64p, c_i64p,

@@ -903,23 +903,24 @@ def gather_slabs(pairs: Sequence[tuple], idx: torch.Tensor) -> None:
 
 def adaln_pack(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor, out: PackedAct, eps: float = 1e-6) -> None:
     """out (PackedAct [B rows, d]) = LN(x) (1 + scale[:, None]) + shift[:, None] for x [B, rows, d] and shift, scale
-    [B, d], bf16, each step rounded (rldx_adaln_pack_bf16)."""
+    [B, d], bf16, each step rounded: torch's LayerNorm, then the modulation and the packing in one launch
+    (rldx_modulate_pack_bf16)."""
     B, rows, d = x.shape
+    y = torch.nn.functional.layer_norm(x, (d,), eps=eps)
     ok = all(t.dtype == BF16 and t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and t.device == x.device
-             for t in (x, shift, scale)) and tuple(shift.shape) == tuple(scale.shape) == (B, d)
-    if not (ok and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0 and
+             for t in (y, shift, scale)) and tuple(shift.shape) == tuple(scale.shape) == (B, d)
+    if not (ok and y.stride(0) % 8 == 0 and y.stride(1) % 8 == 0 and
             (B == 1 or (shift.stride(0) == scale.stride(0) and shift.stride(0) % 8 == 0))):
         # a modulation of the caller's own in another type, shape or layout
-        y = torch.nn.functional.layer_norm(x, (d,), eps=eps)
         mod = torch.empty_like(y, memory_format=torch.contiguous_format)
         torch.add(y * (1 + scale[:, None]), shift[:, None], out=mod)
         pack_act(mod.view(B * rows, d), out=out)
         return
-    _on_gpu(x, shift, scale)
+    _on_gpu(y, shift, scale)
     _check_pack_target(out, B * rows, d)
-    _lib.check(_lib.load().rldx_adaln_pack_bf16(x.data_ptr(), x.stride(1), x.stride(0), rows, B, shift.data_ptr(),
-                                                scale.data_ptr(), shift.stride(0) if B > 1 else 0, d, float(eps),
-                                                out.data.data_ptr(), _stream_ptr(x)), "rldx_adaln_pack_bf16")
+    _lib.check(_lib.load().rldx_modulate_pack_bf16(y.data_ptr(), y.stride(1), y.stride(0), rows, B, shift.data_ptr(),
+                                                   scale.data_ptr(), shift.stride(0) if B > 1 else 0, d,
+                                                   out.data.data_ptr(), _stream_ptr(y)), "rldx_modulate_pack_bf16")
 
 
 class GemmWorkspace:
