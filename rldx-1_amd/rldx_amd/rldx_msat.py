@@ -28,7 +28,7 @@ widths, so each linear is one launch of groups with their own n and k):
     w12 + SwiGLU -> packed             rldx_grouped_gemm_mixed_bf16 (swiglu)
     w3 + residual (in place)           rldx_grouped_gemm_mixed_bf16 (residual)
 Per SingleStreamBlock (5 launches for one robot without a P stream, heads of
-64; 7 otherwise):
+64, SA width below 4096; 7 otherwise):
     LayerNorm -> packed h; linear1: QKV columns (+ bias, QK-RMSNorm, RoPE, K/V)
     and MLP columns (SwiGLU -> packed) in one launch (else three: the two GEMMs
     and rldx_msat_qkv_norm_rope_bf16); attention -> columns [0, inner) of the
@@ -468,8 +468,7 @@ class RldxMsat:
         self._ninf = torch.full((), float("-inf"), dtype=torch.float32, device=self.dev)
         self._zero = torch.zeros((), dtype=torch.float32, device=self.dev)
         self.graph = None
-        # one robot without a P stream: the rows of x are the joint sequence, so linear1 is one launch
-        self.fused_linear1 = B == 1 and not self.phys and D == 64 and H % 2 == 0
+        self.fused_linear1 = self.fuse_linear1(cfg, B, self.phys)
         # the pre-norms of a block's streams, one launch each time
         self.ds_norms = [(self.x_sa, self.h_sa), (self.x_vl, self.h_vl)] + ([(self.x_p, self.h_p)] if self.phys else [])
         self.ss_norms = [(self.x, self.h)] + ([(self.x_p, self.h_p)] if self.phys else [])
@@ -509,6 +508,17 @@ class RldxMsat:
         while split < 8 and split * 2 <= k // 1024 and tiles * split * 2 <= 256:
             split *= 2
         return split
+
+    @staticmethod
+    def fuse_linear1(cfg: RldxMsatCfg, batch: int, physics: bool) -> bool:
+        """Whether a single-stream block's linear1 is one launch (rldx_gemm_qkv_swiglu_bf16):
+        for one robot without a P stream, where the rows of x are the joint sequence,
+        and below the K from which split_for divides the QKV columns (the one launch
+        never splits).  Measured, three launches / one (us, weights from HBM): K 512, 82
+        rows 15.7 / 9.0; 1536, 82 x (4608 + 12288) 32.7 / 23.2; 3072, 82 x (9216 + 24576)
+        78.9 / 63.2, 400 rows 138 / 134; but 4096, 82 x (1536 + 16384) 58.1 / 63.2, 400 x
+        (12288 + 32768) 194 / 214."""
+        return batch == 1 and not physics and cfg.head_dim == 64 and cfg.heads % 2 == 0 and cfg.sa_dim < 4096
 
     @staticmethod
     def wide_for(n: int, epi: str, split: int) -> bool:

@@ -355,3 +355,19 @@ def test_action_head_dispatcher_detects_weight_changes():
     assert d.weights_changed()
     d.refresh()
     assert d._stamp is None and d.rebuilds == 0  # nothing built yet, nothing counted
+
+
+def test_one_launch_linear1_splits_nothing():
+    """linear1 as one launch never splits K: it is chosen only where neither of its two
+    GEMMs would be split on its own, and not for batches, a P stream or odd heads."""
+    for sa_dim in (512, 1536, 3072, 4096, 6144):
+        for heads in (8, 24, 64):
+            cfg = RM.RldxMsatCfg(heads=heads, sa_dim=sa_dim)
+            splits = [RM.RldxMsat.split_for([m], n, sa_dim) for m in (18, 82, 200)
+                      for n in (3 * cfg.inner, 2 * cfg.ss_expanded)]
+            fused = RM.RldxMsat.fuse_linear1(cfg, 1, False)
+            assert not (fused and max(splits) > 1)
+            assert fused == (sa_dim < 4096)
+            assert not RM.RldxMsat.fuse_linear1(cfg, 2, False) and not RM.RldxMsat.fuse_linear1(cfg, 1, True)
+    assert not RM.RldxMsat.fuse_linear1(RM.RldxMsatCfg(heads=23), 1, False)
+    assert not RM.RldxMsat.fuse_linear1(RM.RldxMsatCfg(heads=12, head_dim=128), 1, False)
