@@ -27,6 +27,7 @@ fixed 4096-wide output), and `kv_mask` on the 3-way ops (1 = visible key,
 from __future__ import annotations
 
 import math
+import warnings
 import weakref
 from typing import Optional
 
@@ -559,8 +560,19 @@ def _(hidden, residual, weight):
 # Native dispatch (csrc/torch_ops.cpp): C++ kernels for the CUDA and AutogradCUDA
 # keys of the operators above.  Calls in the common forms run without Python
 # (host time per call 15-22 us -> 7-10 us); every other call, and every call where
-# the library was not built, runs the implementations above, on the same kernels.
+# the library was not built or belongs to another torch, runs the implementations
+# above, on the same kernels.
 # ---------------------------------------------------------------------------
-_native = _lib.LIB_PATH.with_name("librldx_torch.so").exists()
-if _native:
-    torch.ops.load_library(str(_lib.LIB_PATH.with_name("librldx_torch.so")))
+def _load_native(path) -> bool:
+    if not path.exists():
+        return False
+    try:
+        torch.ops.load_library(str(path))
+    except OSError as e:
+        warnings.warn(f"rldx_amd: {path.name} does not load with torch {torch.__version__} ({e}); rebuild it with "
+                      "`make -C rldx-1_amd`. The operators run through Python.", RuntimeWarning, stacklevel=2)
+        return False
+    return True
+
+
+_native = _load_native(_lib.LIB_PATH.with_name("librldx_torch.so"))

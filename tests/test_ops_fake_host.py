@@ -80,3 +80,13 @@ def test_epilogue_fakes():
     assert tuple(nh.shape) == (1, 82, 1536) and tuple(ln.shape) == (1, 82, 1536)
     assert all(tuple(t.shape) == (169, 4096) for t in (*a2, *a3))
     assert all(tuple(t.shape) == (1, 64, 2048) for t in m2)
+
+
+def test_a_dispatch_library_of_another_torch_is_left_out(tmp_path):
+    """librldx_torch.so is bound to one torch; where it does not load the operators stay, through Python."""
+    ops = rldx_amd.ops
+    assert not ops._load_native(tmp_path / "librldx_torch.so")  # not built
+    bad = tmp_path / "librldx_torch.so"
+    bad.write_bytes(b"\x7fELF of another build")
+    with pytest.warns(RuntimeWarning, match="rebuild"):
+        assert not ops._load_native(bad)
