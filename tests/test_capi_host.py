@@ -580,14 +580,16 @@ def test_residual_packed_epilogue_and_layernorm_fold_rejections():
     assert pack(4096, 1536, 10, 1536, 8192, 16388, None) == inval  # stats alignment
 
 
-def test_no_garbage_collection_while_a_graph_is_recorded():
-    """hold_gc (around every stream capture of the package) keeps cyclic garbage
-    alive whatever is allocated inside, also nested, and resumes collection after."""
+def test_no_garbage_collection_while_a_graph_is_recorded(monkeypatch):
+    """hold_gc keeps cyclic garbage alive whatever is allocated inside, also nested, and
+    resumes collection after; every capture of the package records inside it."""
+    import contextlib
     import gc
-    import inspect
+    import types
     import weakref
 
-    from rldx_amd import msat_step, rldx_msat
+    from rldx_amd.msat_step import MsatActionStep
+    from rldx_amd.rldx_msat import RldxActionHead, RldxMsat
 
     class Node:
         pass
@@ -605,5 +607,23 @@ def test_no_garbage_collection_while_a_graph_is_recorded():
     del keep
     gc.collect()
     assert seen() is None
-    for mod in (msat_step, rldx_msat):
-        assert "torch.cuda.graph(" not in inspect.getsource(mod)
+
+    recording = []  # (inside a capture, collection enabled) at each call of the recorded function
+
+    @contextlib.contextmanager
+    def graph(g):
+        g.open = True
+        yield
+        g.open = False
+
+    stream = types.SimpleNamespace(wait_stream=lambda other: None)
+    for name, stub in (("Stream", lambda: stream), ("current_stream", lambda: stream), ("synchronize", lambda: None),
+                       ("stream", lambda st: contextlib.nullcontext()), ("graph", graph),
+                       ("CUDAGraph", lambda: types.SimpleNamespace(open=False))):
+        monkeypatch.setattr(torch.cuda, name, stub)
+    for cls, fn in ((MsatActionStep, "run"), (RldxMsat, "_forward_static"), (RldxActionHead, "run")):
+        obj = types.SimpleNamespace(graph=None)
+        setattr(obj, fn, lambda: recording.append((bool(obj.graph and obj.graph.open), gc.isenabled())))
+        recording.clear()
+        cls.capture(obj)
+        assert recording == [(False, True), (False, True), (True, False)] and gc.isenabled()

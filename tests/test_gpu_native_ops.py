@@ -118,6 +118,38 @@ def test_inputs_with_gradients(dev):
             _same(op(*args), impl._init_fn(*args))
 
 
+def test_forward_mode_tangents(dev):
+    """An input with a tangent goes to the Python implementation, as one that needs a
+    gradient: no formula, so the call raises or its result carries no tangent."""
+    from torch.autograd import forward_ad as fw
+
+    for name, (op, impl, args) in _calls(dev).items():
+        with fw.dual_level():
+            dual = [fw.make_dual(a, torch.ones_like(a)) if i == 0 else a for i, a in enumerate(args)]
+            try:
+                out = op(*dual)
+            except (RuntimeError, NotImplementedError):
+                continue
+            first = out[0] if isinstance(out, tuple) else out
+            assert fw.unpack_dual(first).tangent is None, name
+
+
+def test_vmap(dev):
+    """Mapped over the first argument: each slice's own result, or the refusal of an operator without a
+    batching rule."""
+    for name, (op, impl, args) in _calls(dev).items():
+        pair = torch.stack([args[0], args[0] * 0.5])
+        try:
+            out = torch.vmap(lambda a: op(a, *args[1:]))(pair)
+        except RuntimeError as e:
+            assert "batching rule" in str(e) or "vmap" in str(e), name
+            continue
+        for i in range(2):
+            one = impl._init_fn(pair[i].clone(), *args[1:])
+            for got, want in zip(out if isinstance(out, tuple) else (out,), one if isinstance(one, tuple) else (one,)):
+                assert torch.equal(got[i].view(torch.int16), want.view(torch.int16)), name
+
+
 def test_mlp_weight_updates_and_lifetime(dev):
     op, impl, (x, w, b) = _calls(dev)["mlp"]
     op(x, w, b)
