@@ -914,7 +914,8 @@ def test_gemm_qkv_swiglu_rejections(dev):
             Fn.gemm_qkv_swiglu(*args)
 
 
-@pytest.mark.parametrize("m,n,k", [(700, 21696, 128), (2039, 8128, 384), (2048, 8192, 256)])
+@pytest.mark.parametrize("m,n,k", [(700, 21696, 128), (2039, 8128, 384), (2048, 8192, 256),
+                                   (700, 21696, 768), (2039, 8128, 896), (2048, 8192, 768)])  # (K enough for 256 x 256)
 @pytest.mark.parametrize("epilogue", ["bias", "residual", "swiglu", "swiglu_packed", "bias_packed", "residual_packed"])
 def test_gemm_256_tiles_bit_identical(dev, m, n, k, epilogue):
     """One long stream (256 x 256 tiles; ragged rows, a partial last column tile, one
