@@ -1646,10 +1646,17 @@ hipError_t plan(const rldx_gemm_group_t* groups, int32_t num_groups, int64_t n, 
     // 128 (32 x 128) where 64 x 64 (32 x 64) needs more than one workgroup per CU and
     // it does not (82 x 12288 x 1536 14.6 / 12.7 / 15.9; 18 x 22016 x 4096 44.1 / 40.9; but 82 x
     // 8192 x 1536, 256 workgroups, 10.4 / 12.4 / 15.8).
+    // Just past one workgroup per CU 64 x 64 still wins now and then (167 x 5568 x 1664, 261
+    // workgroups, 15.7 / 16.9): 64 x 128 from 305.  Three row tiles of 64 are two of 128, one
+    // half empty: those take 128 x 128 from 176 tiles (133 x 10816 x 256, 170, 8.5 / - / 9.1)
+    // and 64 x 128 again past 256 (134 x 17216 x 128, 270, - / 9.0 / 10.5).  The choice does not
+    // look at wide_tiles, which changes no sums.
     const bool alone = swiglu && num_groups == 1 && split_k <= 1 && !group_splits && !w_row_sums;
-    const int64_t m64 = (s.m + 63) / 64;
-    const bool wide1 = alone && m64 * (n / 64) > 256 && m64 * ((n + 127) / 128) <= 256;
-    if (static_cast<int64_t>(mt) * nt >= (s.m >= 256 ? 128 : 160) && (s.m >= 256 || (alone && s.m > 64))) {
+    const int64_t m64 = (s.m + 63) / 64, t128 = static_cast<int64_t>(mt) * nt;
+    const bool tall1 = alone && s.m > 64 && (m64 == 3 ? t128 >= 176 && t128 <= 256 : t128 >= 160);
+    const bool wide1 = alone && ((m64 * (n / 64) > (s.m > 32 ? 304 : 256) && m64 * ((n + 127) / 128) <= 256) ||
+                                 (m64 == 3 && t128 > 256));
+    if (s.m >= 256 ? t128 >= 128 : tall1) {
       cfg = kTile128;
       kg = Cfg128::KG;
     } else if ((wide || wide1) && s.m > 32) {
