@@ -1774,22 +1774,24 @@ void launch_qkv(const GemmArgs& args, dim3 grid, hipStream_t stream, bool deep) 
 
 // Whether a launch takes the 256 x 256 tiles.  They run in whole rounds of 256
 // workgroups, one per CU, and nothing overlaps a round's first loads and its epilogue:
-// a round costs 1.25 x as long per column of K as 512 of the 128 x 128 tiles, whose two
-// workgroups per CU overlap each other, and that of 200 (bias), 300 (residual) or 400
-// (SwiGLU) columns more.  Measured (us, 128 x 128 / 256 x 256): SwiGLU 2048 x 8192 x 1536
-// 59.2 / 50.0, x 256 18.0 / 23.2, 2048 x 22016 x 4096 403 / 315, 1500 x 22016 x 4096 294 /
-// 281 (the line's other side), 2048 x 4096 x 8192 133 / 149; residual 2922 x 20736 x 384
-// 97.8 / 119; bias 719 x 10944 x 128 14.6 / 10.8 (the other side again).  Of 5000 random
-// launches of 400 and more 128 x 128 tiles, 16 are more than 3 % slower by this rule, the
-// two worst by 7 and 10 %, the others 0 to 40 % faster.
+// per column of K such a round costs 1.3 of one of 512 of the 128 x 128 tiles, whose two
+// workgroups per CU overlap each other, and it costs 300 (bias), 500 (residual) or 550
+// (SwiGLU) columns more, theirs 200.  Theirs are counted in halves, four fifths of them
+// whole (the 257th tile starts a second pass over the chip).  Measured (us, 128 x 128 / 256 x
+// 256): SwiGLU 2048 x 8192 x 1536 63.5 / 52.1, 512 x 22016 x 4096 117 / 101, 2048 x 22016 x 4096
+// 404 / 325; across the line 1664 x 12288 x 1536 78 / 90, 2036 x 12672 x 128 (residual) 32 / 38,
+// 2572 x 3776 x 256 16.6 / 24.2.  Of 6300 random launches of 300 and more 128 x 128 tiles, 1.4 %
+// are more than 3 % slower by this rule (two by 17 and 20 %).
 bool big_tiles(const GemmArgs& args, int epilogue, bool ln) {
   const Group& G = args.g[0];
   if (args.num_groups != 1 || ln || G.splits > 1 || G.stats_out || epilogue < kEpiBias || epilogue > kEpiResidualPacked)
     return false;
   if (G.cfg != kTile128 || reinterpret_cast<uintptr_t>(G.bias) % 8) return false;
   const int64_t big = static_cast<int64_t>((G.m + 255) / 256) * ((G.n + 255) / 256);
-  const int64_t k = G.k, fixed = epilogue == kEpiBias || epilogue == kEpiBiasPacked ? 200 : residual_epi(epilogue) ? 300 : 400;
-  return (big + 255) / 256 * (k + fixed) * 5 * 128 <= k * G.items;  // (items: the 128 x 128 tiles)
+  const int64_t k = G.k, fixed = epilogue == kEpiBias || epilogue == kEpiBiasPacked ? 300 : residual_epi(epilogue) ? 500 : 550;
+  const int64_t small = G.items;  // the 128 x 128 tiles
+  // 1.3 rounds (k + fixed) against ((4 whole halves 256 + tiles) / 5) / 512 (k + 200)
+  return (big + 255) / 256 * (k + fixed) * 3328 <= ((small + 255) / 256 * 1024 + small) * (k + 200);
 }
 
 hipError_t launch_big(GemmArgs args, int epilogue, hipStream_t stream) {
