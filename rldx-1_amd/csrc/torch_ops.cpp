@@ -315,6 +315,11 @@ struct Made {
   c10::Stream stream;
   std::atomic<bool> done{false};
   explicit Made(c10::Stream s) : stream(s) { event.record(s); }
+  void again(c10::Stream s) {
+    stream = s;
+    done = false;
+    event.record(s);
+  }
 };
 struct Packed {
   c10::weak_intrusive_ptr<c10::TensorImpl> w;
@@ -332,18 +337,42 @@ std::unordered_map<int64_t, Packed>& packed_weights() {
 c10::Stream current_stream(const Tensor& t) {
   return c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getStream(t.device());
 }
+// Events of forgotten copies, at most 16: a new one costs 15-20 us of a first call.  (Under the mutex.)
+std::vector<std::shared_ptr<Made>>& spare_events() {
+  static auto* v = new std::vector<std::shared_ptr<Made>>();
+  return *v;
+}
+std::shared_ptr<Made> made_on(c10::Stream s) {
+  std::shared_ptr<Made> m;
+  {
+    const std::lock_guard<std::mutex> lock(g_packed_mutex);
+    auto& v = spare_events();
+    for (size_t i = 0; i < v.size() && !m; ++i)
+      if (v[i]->stream.device_index() == s.device_index()) {
+        m = std::move(v[i]);
+        v.erase(v.begin() + static_cast<std::ptrdiff_t>(i));
+      }
+  }
+  if (!m) return std::make_shared<Made>(s);
+  m->again(s);
+  return m;
+}
+void spare(std::shared_ptr<Made>& m) {  // (nobody else reads it: it came out of the table, and no call holds it)
+  if (m && m.use_count() == 1 && spare_events().size() < 16) spare_events().push_back(std::move(m));
+}
 int64_t key_of(const Tensor& w) { return reinterpret_cast<int64_t>(w.unsafeGetTensorImpl()); }
 
 void remember_packed(const Tensor& w, const Tensor& packed) {
   if (w.is_inference()) return;  // no version counter
   Packed p{c10::weak_intrusive_ptr<c10::TensorImpl>(w.getIntrusivePtr()), static_cast<uint32_t>(w._version()),
            w.data_ptr(), w.sizes().vec(), w.strides().vec(), packed,
-           packed.is_cuda() ? std::make_shared<Made>(current_stream(packed)) : nullptr};
+           packed.is_cuda() ? made_on(current_stream(packed)) : nullptr};
   std::optional<Packed> old;  // freed outside the lock: the last reference to a tensor of Python's takes the GIL
   const std::lock_guard<std::mutex> lock(g_packed_mutex);
   auto [it, inserted] = packed_weights().try_emplace(key_of(w), std::move(p));
   if (inserted) return;
   old.emplace(std::move(it->second));
+  spare(old->made);
   it->second = std::move(p);
 }
 void forget_packed(int64_t key) {
@@ -352,6 +381,7 @@ void forget_packed(int64_t key) {
   auto it = packed_weights().find(key);
   if (it == packed_weights().end()) return;
   old.emplace(std::move(it->second));
+  spare(old->made);
   packed_weights().erase(it);
 }
 // Whether work on the current stream can read a copy; makes the stream wait for it where it has to.

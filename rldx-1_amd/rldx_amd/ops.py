@@ -354,57 +354,64 @@ _packed_weights: dict = {}  # id(weight) -> _PackedEntry
 
 
 class _PackedEntry:
-    """A packed copy of `ref()` as it was in `state`, written by a launch on `stream` that `event` follows."""
+    """A packed copy of `ref()` as it was in `state`, written by a launch on `stream` that `event` follows
+    (None where the native table keeps them)."""
 
     __slots__ = ("ref", "state", "pw", "stream", "event")
 
     def __init__(self, w: torch.Tensor, state: tuple, pw: Fn.PackedWeight):
         self.ref, self.state, self.pw, self.stream = weakref.ref(w), state, pw, None
-        if w.is_cuda:
+        if w.is_cuda and not (_native and pw.swiglu_pairs):
             self.stream = torch.cuda.current_stream(w.device)
             self.event = torch.cuda.Event()
             self.event.record(self.stream)
 
-    def readable(self, w: torch.Tensor, cur, capturing: bool) -> bool:
-        """Whether work on stream `cur` can read the copy; makes `cur` wait for it where it has to.  A graph
-        takes it only when it is known to be complete: a recorded wait would not outlive the capture."""
+    def readable(self, w: torch.Tensor, capturing: bool) -> bool:
+        """Whether work on the current stream can read the copy; makes it wait where it has to.  A graph takes
+        a copy only when it is known to be complete: a recorded wait would not outlive the capture."""
         if _native and self.pw.swiglu_pairs:
             return torch.ops.rldx_native.packed_of(w) is not None
-        if capturing:
-            return False
-        if cur != self.stream:
+        if not capturing and self.stream is not None:
+            self.follow()
+        return not capturing
+
+    def follow(self) -> None:
+        """The current stream waits for the copy and keeps its memory from being reused under it."""
+        cur = torch.cuda.current_stream(self.pw.data.device)
+        if self.stream is not None and cur != self.stream:
             cur.wait_event(self.event)
-            self.pw.data.record_stream(cur)
-        return True
+        self.pw.data.record_stream(cur)
 
 
 def _packed_weight(w: torch.Tensor, swiglu_pairs: bool) -> Fn.PackedWeight:
     state = (w._version, w.data_ptr(), tuple(w.shape), w.stride(), swiglu_pairs)
-    cur = torch.cuda.current_stream(w.device) if w.is_cuda else None
-    capturing = cur is not None and torch.cuda.is_current_stream_capturing()
+    capturing = w.is_cuda and torch.cuda.is_current_stream_capturing()
     hit = _packed_weights.get(id(w))
     hit = hit if hit is not None and hit.ref() is w else None
-    if hit is not None and hit.state == state and hit.readable(w, cur, capturing):
+    if hit is not None and hit.state == state and hit.readable(w, capturing):
         return hit.pw
     old = None
     if hit is not None and not capturing and hit.state[1:] == state[1:]:
         # updated in place: written over the old copy, whose address captured graphs hold.  The update came after
         # every earlier call in stream order, and this call after the update.
         old = hit.pw.data
-        if cur is not None and cur != hit.stream:
-            cur.wait_event(hit.event)
-            old.record_stream(cur)
+        if w.is_cuda:
+            hit.follow()
     pw = Fn.pack_weight(w if w.stride(1) == 1 else w.contiguous(), swiglu_pairs=swiglu_pairs, row_sums=False, out=old)
     if capturing:  # only recorded: the graph packs at each replay, and nobody else may read this copy
         return pw
     if hit is None:
-        weakref.finalize(w, _packed_weights.pop, id(w), None)
-        if _native:
-            weakref.finalize(w, torch.ops.rldx_native.forget_packed, int(w._cdata)).atexit = False
+        weakref.finalize(w, _forget, id(w), int(w._cdata)).atexit = False
     _packed_weights[id(w)] = _PackedEntry(w, state, pw)
     if _native and swiglu_pairs:
         torch.ops.rldx_native.remember_packed(w, pw.data)
     return pw
+
+
+def _forget(key: int, impl: int) -> None:
+    _packed_weights.pop(key, None)
+    if _native:
+        torch.ops.rldx_native.forget_packed(impl)
 
 
 @torch.library.custom_op("ss::fused_mlp_swiglu", mutates_args=())
