@@ -714,16 +714,16 @@ __global__ __launch_bounds__(256, 1) void attn_fwd_kernel(AttnArgs a) {
 // CU at 32/8 heads x 4096 causal, close to the ~48 B/clk a CU gets from L2.
 //   * NG = 1 (128 queries, no merge): a wave runs S, softmax and P V of one tile
 //     in sequence within 168 VGPRs, and three workgroups per CU overlap each
-//     other's matrix and vector phases.  The matrix cores are then busy 48 % and
-//     the vector ALU 46 % of the time: the two barely overlap, which bounds it.
+//     other's matrix and vector phases.  Both are then busy just under half of the
+//     time: the two barely overlap, which bounds it.
 //   * NG = 2 (64 queries): half the chain of tiles per wave and twice the
 //     workgroups, for launches whose longest blocks bound NG = 1; S of the next
 //     tile is issued between the exponentials (two waves per SIMD), and the two
 //     partial states of a query block are merged at the end.
 // Operator times on MI355X, attn_fwd_kernel / NG = 1 / NG = 2 (us): causal GQA
-// 32/8 x 4096 215 / 153 / 182, 28/4 x 1280 40.5 / 39.7 / 34.2, 32/8 x 512 19.4 /
-// 23.0 / 19.5; ViT 16 x 72, images of 1024, 1600, 484, 2304, 196 tokens 110 / 91 /
-// 96, 2 x 196 10.8 / 13.0 / 12.2.
+// 32/8 x 4096 227 / 162 / 180, 28/4 x 1280 40.3 / 42.2 / 37.2, 32/8 x 512 18.3 /
+// 23.7 / 19.2; ViT 16 x 72, images of 1024, 1600, 484, 2304, 196 tokens 116 / 97 /
+// 99, 2 x 196 10.7 / 13.8 / 11.9.
 // ---------------------------------------------------------------------------
 template <int D, int KS, int NG, bool kCausal, bool kBias, bool kQNorm, bool kVarlen>
 __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_kernel(AttnArgs a) {
@@ -1521,15 +1521,15 @@ constexpr int vit_padded_dim(int64_t hd) {
 // Measured on MI355X (operator us, attn_fwd_kernel / NG = 1 / NG = 2):
 //   causal: the longest block bounds a launch until the blocks of every length
 //   fill the chip, which heads x (blocks + 1) measures (twice the work over the
-//   longest chain).  NG = 2 wins from 430 (32/8 x 800: 29.5 / 28.3 / 25.2 at 432; 32/8 x
-//   512: 19.4 / 23.0 / 19.5 at 288), with chains past 20 steps from 528 (16/8 x 1536: 34.6 /
+//   longest chain).  NG = 2 wins from 430 (32/8 x 800: 28.9 / 30.0 / 25.2 at 432; 32/8 x
+//   512: 18.3 / 23.7 / 19.2 at 288), with chains past 20 steps from 528 (16/8 x 1536: 34.6 /
 //   43.5 / 36.0 at 400, x 2048: 44.7 / 53.9 / 44.5 at 528, x 2560: 63.7 / 67.8 / 53.8),
-//   NG = 1 over it from 540 (32/8 x 2048: 79.7 / 64.2 / 66.1 at 544; 16/8 x 4096:
+//   NG = 1 over it from 540 (32/8 x 2048: 78.9 / 64.8 / 65.8 at 544; 16/8 x 4096:
 //   122 / 111 / 102 at 528, x 6144: 228 / 190 / 202 at 784).
 //   not causal: blocks of one length run in whole rounds over the chip.  NG = 1 wins
-//   from 380 workgroups (3 images of 1024: 51.9 / 43.5 / 44.4 at 384; 2304 + 0: 63.3 /
-//   64.1 / 64.1 at 288), below that NG = 2 where it makes one round of two
-//   workgroups per CU (1600: 42.3 / 40.8 / 35.9 at 400; joint 16 x 2144: 61.5 / 62.4 /
+//   from 380 workgroups (3 images of 1024: 51.2 / 45.3 / 43.7 at 384; 2304: 62.2 /
+//   70.1 / 65.0 at 288), below that NG = 2 where it makes one round of two
+//   workgroups per CU (1600: 41.8 / 43.0 / 36.6 at 400; joint 16 x 2144: 61.5 / 62.4 /
 //   71.7 at 544, 16 x 1120: 25.4 / 28.3 / 25.8 at 288).
 // head_dim 64 (half the matrix work per exponential: the old kernel and NG = 2 are
 // closer, NG = 1 is last until launches are very large), attention only / ViT:
