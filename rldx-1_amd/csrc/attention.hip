@@ -898,22 +898,50 @@ __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_ke
     for (int ks = 0; ks < KS; ++ks) score_mma(ks, sa);
   }
 
+  // The bias of a flagged tile: lane l < 32 holds key l's, and one fp32 MFMA with the
+  // column kb adds it to every query's scores.  Loaded one step ahead and before that
+  // step's ring loads: loads return in order, so a later one would wait for the rings
+  // (a bias on every key, 192 heads x 160 x 1830 keys, head_dim 128: loaded when needed,
+  // sixteen values a lane, 83.4 us, so 64.3, attn_fwd_kernel 60.3; 24 heads x 2196 of
+  // head_dim 64, 77.4 before, 58.4 in attn_fwd_kernel).
+  bool btile = false, bnext = false;
+  float bcur = 0.f, bload = 0.f;
+  const float bcol = lane < 32 ? kb : 0.f;
+  auto fetch_bias = [&](int t) {
+    bnext = t >= kFlagTiles || ((__builtin_amdgcn_readlane(bflag, t >> 5) >> (t & 31)) & 1u);
+    if (bnext) bload = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(bsr, (t * BN + l32) * 4, 0, 0));
+  };
+  auto next_bias = [&](int t) {
+    if constexpr (kBias) {
+      btile = bnext;
+      if (btile) {
+        bcur = bload;
+        if (a.bias_is_mask) bcur = bcur == 0.f ? -__builtin_inff() : 0.f;
+        if (g) bcur = 0.f;
+      }
+      fetch_bias(t + NG);
+    }
+  };
+  if constexpr (kBias) fetch_bias(kg);
+
   // Step i of the wave's tile t.  PIPE: scores S(i) in s; softmax of S(i) with the
   // S(i + 1) MFMAs between the exponentials, then P(i) V(i).  Otherwise S(i), its
   // softmax and P(i) V(i) in sequence.
   int kslot = PIPE ? 1 : 0;  // ring slot of the K part that step i reads
   auto body = [&](int i, int vslot, floatx16& s, floatx16& snew) {
     const int kprev = kslot == 0 ? NKS - 1 : kslot - 1;
+    const int t = i * NG + kg;
     if constexpr (PIPE) {
       vm_wait_barrier<NDK>();  // K(i + 1) and V(i) are in LDS; the slots of K(i) and V(i - 1) are free
+      next_bias(t);
       dma_v(i + 1, vslot ^ 1);
       dma_k(i + 3, kprev);
     } else {
       vm_wait_barrier<NDK + NDV>();  // K(i) and V(i) are in LDS; the slots of step i - 1 are free
+      next_bias(t);
       dma_k(i + 2, kprev);
       dma_v(i + 2, kprev);
     }
-    const int t = i * NG + kg;
     const int kcur = kslot;
     kslot = kslot + 1 == NKS ? 0 : kslot + 1;
     if (t >= tile_end) return;
@@ -927,24 +955,16 @@ __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_ke
       read_v(kcur);
     }
     const int k0 = t * BN;
-    bool btile = false;
-    if constexpr (kBias)
-      btile = t >= kFlagTiles || ((__builtin_amdgcn_readlane(bflag, t >> 5) >> (t & 31)) & 1u);
-    if ((k0 + BN > sk) || (kCausal && k0 + BN - 1 > q_first) || btile) {
-      floatx4 bn[4] = {};
-      if constexpr (kBias) {
-        if (btile) load_bias(bn, bsr, k0 + 4 * g, a.bias_is_mask);
-      }
+    if constexpr (kBias) {
+      if (btile) s = __builtin_amdgcn_mfma_f32_32x32x2f32(bcur, bcol, s, 0, 0, 0);
+    }
+    if ((k0 + BN > sk) || (kCausal && k0 + BN - 1 > q_first)) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         const int key = k0 + 8 * (e >> 2) + 4 * g + (e & 3);
-        float sv = s[e];
-        if constexpr (kBias) {
-          if (btile) sv += bn[e >> 2][e & 3] * kb;
-        }
         bool ok = key < sk;
         if constexpr (kCausal) ok = ok && (key <= q_idx);
-        s[e] = ok ? sv : -__builtin_inff();
+        s[e] = ok ? s[e] : -__builtin_inff();
       }
     }
     float mt = s[0];
@@ -1031,7 +1051,8 @@ __global__ __launch_bounds__(256, NG == 1 && !kBias ? 3 : 2) void attn_shared_ke
     const float m = fmaxf(m_ref, ml[0]);
     const float w0 = m_ref == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(m_ref - m);
     const float w1 = ml[0] == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(ml[0] - m);
-    l = kg == 0 ? l * w0 + ml[1] * w1 : ml[1] * w1 + l * w0;  // the same bits in both groups
+    // group 0's sum is the one inside the fma: the same bits in both groups
+    l = kg == 0 ? __builtin_fmaf(l, w0, ml[1] * w1) : __builtin_fmaf(ml[1], w1, l * w0);
     inv = l > 0.f ? 1.0f / l : 0.f;
 #pragma unroll
     for (int db = 0; db < DBLK; ++db)

@@ -65,6 +65,21 @@ def test_attention_shared_tiles(dev, B, Hq, Hkv, Sq, Sk, D, causal, bias):
     assert_bf16_close(o, r, "attention, shared tiles")
 
 
+@pytest.mark.parametrize("Hq,Hkv,Sq,D", [(400, 4, 33, 128), (3, 1, 17000, 128)])
+def test_shared_tiles_bias_past_the_flags(dev, Hq, Hkv, Sq, D):
+    """Tiles after the 2048 that have a flag: their bias decides the result (two key groups, one key group)."""
+    Sk = 2048 * 32 + 77
+    q, k, v, kb = _inputs(1, Hq, Hkv, Sq, Sk, D, True)
+    kb[0, 2048 * 32 - 5:] += 6.0
+    kb[0, -9:-3] = float("-inf")
+    o = Fn.attention(q.to(dev), k.to(dev), v.to(dev), key_bias=kb.to(dev))
+    for h in (0, Hq - 1):
+        kv = h // (Hq // Hkv)
+        rows = slice(max(0, Sq - 40), Sq)
+        r = ref.sdpa(q[:, h:h + 1, rows], k[:, kv:kv + 1], v[:, kv:kv + 1], key_bias=kb)
+        assert_bf16_close(o[:, h:h + 1, rows], r, "attention, bias past the flags")
+
+
 @pytest.mark.parametrize("Hq,Hkv,S,D,causal,part", [
     (400, 400, 128, 128, False, 80), (416, 416, 64, 64, False, 104), (64, 16, 600, 128, False, 4),  # part: heads per unshared launch
     (32, 8, 800, 128, True, 8), (300, 60, 128, 128, True, 40), (32, 8, 2100, 128, True, 4), (40, 8, 1100, 64, True, 10)])
