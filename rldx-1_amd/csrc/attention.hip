@@ -1572,8 +1572,9 @@ constexpr int vit_padded_dim(int64_t hd) {
 // 17.8), 33-64 rows from 640 heads (560 x 64 x 700 40.0 / 44.0 / 41.3, 640 42.6 / 45.7 / 41.8).
 // Partly filled blocks count by their rows where the launch has few blocks (156 heads x 78
 // causal, 7.3 / - / 7.8; head_dim 64 224 heads x 79 x 542 10.0 / - / 11.5, 208 x 214 x 1247, 695
-// by rows, 26.3 / - / 27.9) and in a batch of
-// images: many small images leave most blocks nearly empty and a long one bounds the
+// by rows, 26.3 / - / 27.9; head_dim 128 with masked keys 192 x 144 x 1400, 384 blocks of
+// 128 queries, 42.1 / 48.1 / 49.0, but 208 x 144 x 1400 48.5 / 47.9 / 48.8) and in a batch
+// of images: many small images leave most blocks nearly empty and a long one bounds the
 // launch (16 images of 2078 rows, the longest 661, 12 heads, 384 by blocks, 195 by rows:
 // 28.8 / 33.5; head_dim 64 3 images of 1574, the longest 1208, 16 heads: 23.5 / - / 26.0;
 // images of one size, 30 x 64 at 16 heads, 23.2 / 20.3, cannot be told from these).
@@ -1597,7 +1598,7 @@ int shared_groups(const AttnShape& s) {
     return s.rows > 32 && s.heads >= 380 && (s.heads <= 512 || s.heads >= 640) ? 2 : 0;
   const int64_t blocks = s.heads * s.b64, filled = s.heads * s.rows / 64;
   if (!narrow) {
-    if ((s.images ? filled / 2 : s.heads * s.b128) >= 380) return 1;
+    if (s.images ? filled / 2 >= 380 : s.heads * s.b128 >= (filled < 490 ? 400 : 380)) return 1;
     return blocks >= 400 && blocks <= 512 && (!s.images || filled >= 380) ? 2 : 0;
   }
   if (!s.images && s.rows <= 32) return 0;
